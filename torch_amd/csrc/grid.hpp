@@ -22,13 +22,9 @@
 #include "kernels.hpp"
 
 // Mixed-precision column kernel: 64-source LDS tiles whose FP32 partial sums are added to FP64
-// accumulators every TG_GRID_FOLD_TILES tiles; TG_GRID_RCP = 1 forms m / r^3 as (m y) rcp(r^2)
-// (a transcendental op in place of a multiply).
+// accumulators every TG_GRID_FOLD_TILES tiles.
 #ifndef TG_GRID_FOLD_TILES
 #define TG_GRID_FOLD_TILES 1
-#endif
-#ifndef TG_GRID_RCP
-#define TG_GRID_RCP 0
 #endif
 
 namespace tg {
@@ -136,7 +132,9 @@ __device__ __forceinline__ void grid_tile_f32(const float4* __restrict__ s4, con
                                               const float4 (*__restrict__ sdz)[2], float tx, float ty,
                                               const float (&tz)[8], float (&ax)[8], float (&ay)[8],
                                               float (&az)[8], float (&ap)[8]) {
-#pragma unroll 2
+  // One run of 8 v_rsq_f32 per source (rsq_run).  Unrolled by 4 sources: 7.02 ms on 16 uneven
+  // problems (3.7e10 pairs) against 7.21 by 2 and 7.02 by 8; two sources per run of 16: 7.05.
+#pragma unroll 4
   for (int j = 0; j < 64; ++j) {
     const float4 s = s4[j];
     const float dx = s.x - tx, dy = s.y - ty;
@@ -147,24 +145,22 @@ __device__ __forceinline__ void grid_tile_f32(const float4* __restrict__ s4, con
       zr[0] = d0.x; zr[1] = d0.y; zr[2] = d0.z; zr[3] = d0.w;
       zr[4] = d1.x; zr[5] = d1.y; zr[6] = d1.z; zr[7] = d1.w;
     }
+    float r2[8], y[8];
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
-      const float dz = (FL & F_ZROW) ? zr[k] : s.z - tz[k];
-      const float r2 = fmaf(dz, dz, base);
-      float y = __builtin_amdgcn_rsqf(r2);
-      if (FL & F_GUARD) y = r2 > 0.0f ? y : 0.0f;
-      const float mr = s.w * y;
-      if (!(FL & F_NOPOT)) ap[k] += mr;
-#if TG_GRID_RCP
-      float ri = __builtin_amdgcn_rcpf(r2);
-      if (FL & F_GUARD) ri = r2 > 0.0f ? ri : 0.0f;
-      const float w = mr * ri;
-#else
-      const float w = (mr * y) * y;
-#endif
+      if (!(FL & F_ZROW)) zr[k] = s.z - tz[k];
+      y[k] = r2[k] = fmaf(zr[k], zr[k], base);
+    }
+    rsq_run(y);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      if (FL & F_GUARD) y[k] = r2[k] > 0.0f ? y[k] : 0.0f;
+      const float mr = s.w * y[k];
+      if (!(FL & F_NOPOT)) ap[k] = fmaf(s.w, y[k], ap[k]);
+      const float w = (mr * y[k]) * y[k];
       ax[k] = fmaf(w, dx, ax[k]);
       ay[k] = fmaf(w, dy, ay[k]);
-      az[k] = fmaf(w, dz, az[k]);
+      az[k] = fmaf(w, zr[k], az[k]);
     }
   }
 }
@@ -400,9 +396,10 @@ __device__ __forceinline__ void grid_block(LdsCol<MIXED, W>& L, const Tgt& T, in
 }
 
 // blockIdx.x = leaf block, blockIdx.y = source chunk.  Requires T.blocks && T.nb == 8 and a
-// workgroup of 64 W lanes.
+// workgroup of 64 W lanes.  Mixed: held to 168 VGPRs (3 waves per SIMD, as the persistent kernel): the
+// loop of 4 sources takes 2.23 ms per call on c2's forward with them, 2.34 without the bound.
 template <bool MIXED, int W>
-__global__ __launch_bounds__(64 * W) void k_eval_grid(Tgt T, const double4* __restrict__ src4,
+__global__ __launch_bounds__(64 * W, MIXED ? 3 : 1) void k_eval_grid(Tgt T, const double4* __restrict__ src4,
                                                       const double* __restrict__ srce2, int64_t ns,
                                                       int64_t chunk, const double* sst, Out O) {
   __shared__ LdsCol<MIXED, W> L;
@@ -475,7 +472,7 @@ __device__ __forceinline__ void cols_group(LdsCol<MIXED, W>& L, const Tgt& T, in
 // blockIdx.x = group of 512 targets, blockIdx.y = source chunk.  Gated (Out::gate) against
 // the generic kernel on the check's flag.
 template <bool MIXED, int W>
-__global__ __launch_bounds__(64 * W) void k_eval_cols(Tgt T, const double4* __restrict__ src4,
+__global__ __launch_bounds__(64 * W, MIXED ? 3 : 1) void k_eval_cols(Tgt T, const double4* __restrict__ src4,
                                                       const double* __restrict__ srce2, int64_t ns,
                                                       int64_t chunk, const double* sst, Out O) {
   __shared__ LdsCol<MIXED, W> L;
@@ -525,31 +522,49 @@ __device__ __forceinline__ void gs_block(const LdsGS<MIXED>& L,
     T sw[K];
 #pragma unroll
     for (int k = 0; k < K; ++k) sw[k] = (T)0;
+    if constexpr (MIXED) {
+      // one run of 8 K v_rsq_f32 per column (K <= 2; rsq_run): c2 reverse 2.10 ms per call against
+      // 2.17 in runs of 8 and 2.22 of 4 (K = 2), 2.44 with the v_rsq_f32 spread over the column
+      float dz[8 * K], r2[8 * K], y[8 * K];
 #pragma unroll
-    for (int kk = 0; kk < 8; ++kk) {
-      const T zs = L.cz[kk];
-      const T m = L.m[col * 8 + kk];
+      for (int c = 0; c < 8; ++c)
 #pragma unroll
-      for (int k = 0; k < K; ++k) {
-        const T dz = zs - tz[k];
-        const T r2 = fma(dz, dz, base[k]);
-        T y;
-        if constexpr (MIXED) {
-          y = __builtin_amdgcn_rsqf(r2);
-          if (FL & F_GUARD) y = r2 > 0.0f ? y : 0.0f;
-        } else {
-          y = rsqrt_f64<FL>(r2);
+        for (int k = 0; k < K; ++k) {
+          const int q = c * K + k;
+          dz[q] = L.cz[c] - tz[k];
+          y[q] = r2[q] = fmaf(dz[q], dz[q], base[k]);
         }
-        const T mr = m * y;
-        if (!(FL & F_NOPOT)) ap[k] += mr;
-        const T w = (mr * y) * y;
-        if constexpr (MIXED) {
-          ax[k] = fma(w, dx[k], ax[k]);
-          ay[k] = fma(w, dy[k], ay[k]);
-        } else {
+      rsq_run(y);
+#pragma unroll
+      for (int c = 0; c < 8; ++c) {
+        const float m = L.m[col * 8 + c];
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+          const int q = c * K + k;
+          if (FL & F_GUARD) y[q] = r2[q] > 0.0f ? y[q] : 0.0f;
+          const float mr = m * y[q];
+          if (!(FL & F_NOPOT)) ap[k] = fmaf(m, y[q], ap[k]);
+          const float w = (mr * y[q]) * y[q];
+          ax[k] = fmaf(w, dx[k], ax[k]);
+          ay[k] = fmaf(w, dy[k], ay[k]);
+          az[k] = fmaf(w, dz[q], az[k]);
+        }
+      }
+    } else {
+#pragma unroll
+      for (int kk = 0; kk < 8; ++kk) {
+        const double zs = L.cz[kk];
+        const double m = L.m[col * 8 + kk];
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+          const double dz = zs - tz[k];
+          const double y = rsqrt_f64<FL>(fma(dz, dz, base[k]));
+          const double mr = m * y;
+          if (!(FL & F_NOPOT)) ap[k] += mr;
+          const double w = (mr * y) * y;
           sw[k] += w;
+          az[k] = fma(w, dz, az[k]);
         }
-        az[k] = fma(w, dz, az[k]);
       }
     }
     if constexpr (!MIXED) {
