@@ -334,7 +334,7 @@ __global__ void k_batch_reduce(int nred, const int* __restrict__ ids,
     s0 += pc[t];
     s1 += pc[n + t];
     s2 += pc[2 * n + t];
-    s3 += pc[3 * n + t];
+    if (!P.O.nopot) s3 += pc[3 * n + t];
   }
   Out o = P.O;
   o.part = nullptr;

@@ -35,23 +35,7 @@ struct Flash {
   int type;                       // 1 spline, 2 linear
   int quirks;                     // potential as the reference writes it
   int nrep;                       // periodic: images n in [-nrep, nrep]^3
-  int s32;                        // rsoft^2 > 1e-30: a tile may seed 1/sqrt in FP32 (r2_bound decides)
-  double reach;                   // periodic: (nrep + 1) max(L), the farthest image offset; else 0
 };
-
-// Largest |coordinate| of the workgroup's targets (NT lanes, K each; t >= n excluded), through
-// `red` (2 NT / 64 doubles of LDS).
-template <int K, int NT>
-__device__ __forceinline__ double tile_rmax(const double (&tx)[K], const double (&ty)[K],
-                                            const double (&tz)[K], int64_t tile0, int64_t n,
-                                            double* red) {
-  double mn[1] = {0.0}, mx[1] = {0.0};
-#pragma unroll
-  for (int k = 0; k < K; ++k)
-    if (tile0 + (int64_t)k * NT + threadIdx.x < n) mx[0] = fmax(mx[0], max_abs3(tx[k], ty[k], tz[k]));
-  block_minmax<NT, 1>(mn, mx, red);
-  return mx[0];
-}
 
 // Kernel values for r < rsoft.  Force: the reference's spline pieces and linear slope;
 // q <= 1e-5, where the reference leaves the force kernel unassigned, takes the r -> 0 limit
@@ -79,9 +63,8 @@ __device__ __forceinline__ void flash_soft(const Flash& P, double r, double& kv,
 }
 
 // Force kernel kv (the pair adds -m kv d, d = x_t - x_s) and potential kernel pk of one pair.
-template <bool S32>
 __device__ __forceinline__ void flash_pair(const Flash& P, double r2, double& kv, double& pk) {
-  const double y = rsqrt_f64<S32 ? F_SEED32 : 0>(r2);
+  const double y = rsqrt_f64<0>(r2);
   kv = (y * y) * y;
   pk = y;
   if (r2 <= P.soft_thr) flash_soft(P, sqrt(r2), kv, pk);   // inside rsoft (divergent, rare)
@@ -119,7 +102,7 @@ __device__ __forceinline__ void image_range(double d, double iL, double rem, int
 // inside the cutoff, as the reference assigns pgpot per image (Gravity_getPotentialAtPoint.F90:
 // 262-274).
 // Image indices run as doubles (exact for |n| <= 64), so n * L is formed without a conversion.
-template <bool S32, bool QUIRKS>
+template <bool QUIRKS>
 __device__ __forceinline__ void flash_images(const Flash& P, double dxi, double dyi, double dzi,
                                              double& px, double& py, double& pz, double& pp) {
   px = py = pz = pp = 0.0;
@@ -163,7 +146,7 @@ __device__ __forceinline__ void flash_images(const Flash& P, double dxi, double 
             r2 = xy + dz * dz;
           }
           if (r2 <= P.cut_thr) {
-            const double y = rsqrt_f64<S32 ? F_SEED32 : 0>(r2);
+            const double y = rsqrt_f64<0>(r2);
             const double kv = (y * y) * y;
             skv += kv;
             pz = fma(kv, dz, pz);
@@ -173,7 +156,7 @@ __device__ __forceinline__ void flash_images(const Flash& P, double dxi, double 
         }
         for (double fz = (double)z0 + 1.0; fz < fz1; fz += 1.0) {
           const double dz = fma(fz, P.lz, dzi);
-          const double y = rsqrt_f64<S32 ? F_SEED32 : 0>(fma(dz, dz, xy));
+          const double y = rsqrt_f64<0>(fma(dz, dz, xy));
           const double kv = (y * y) * y;
           skv += kv;
           pz = fma(kv, dz, pz);
@@ -188,7 +171,7 @@ __device__ __forceinline__ void flash_images(const Flash& P, double dxi, double 
             r2 = xy + dz * dz;
           }
           if (r2 <= P.cut_thr) {
-            const double y = rsqrt_f64<S32 ? F_SEED32 : 0>(r2);
+            const double y = rsqrt_f64<0>(r2);
             const double kv = (y * y) * y;
             skv += kv;
             pz = fma(kv, dz, pz);
@@ -209,7 +192,7 @@ __device__ __forceinline__ void flash_images(const Flash& P, double dxi, double 
         }
         if (r2 <= P.cut_thr) {
           double kv, pk;
-          flash_pair<S32>(P, r2, kv, pk);
+          flash_pair(P, r2, kv, pk);
           px = fma(kv, dx, px);
           py = fma(kv, dy, py);
           pz = fma(kv, dz, pz);
@@ -225,7 +208,7 @@ __device__ __forceinline__ void flash_images(const Flash& P, double dxi, double 
 // near2): remove the clamped Newtonian term that loop added and add the exact pair term.
 // Any pair the reference puts inside rsoft is flagged: its r2 is at most soft_thr, and the
 // FMA-formed r2 differs from the reference's by a few ulps.
-template <int K, bool S32>
+template <int K>
 __device__ __forceinline__ void flash_fix(const Flash& P, const double4 s, const double (&tx)[K],
                                           const double (&ty)[K], const double (&tz)[K],
                                           double (&ax)[K], double (&ay)[K], double (&az)[K],
@@ -235,7 +218,7 @@ __device__ __forceinline__ void flash_fix(const Flash& P, const double4 s, const
     const double fx = tx[k] - s.x, fy = ty[k] - s.y, fz = tz[k] - s.z;
     const double r2f = fma(fx, fx, fma(fy, fy, fz * fz));
     if (r2f < P.near2) {
-      const double y0 = rsqrt_f64<S32 ? F_SEED32 : 0>(P.near2);
+      const double y0 = rsqrt_f64<0>(P.near2);
       const double mr0 = s.w * y0;
       const double w0 = mr0 * (y0 * y0);
       double dx, dy, dz, r2;
@@ -247,7 +230,7 @@ __device__ __forceinline__ void flash_fix(const Flash& P, const double4 s, const
         r2 = (dx * dx + dy * dy) + dz * dz;
       }
       double kv, pk;
-      flash_pair<S32>(P, r2, kv, pk);
+      flash_pair(P, r2, kv, pk);
       const double w = s.w * kv;
       ax[k] += w0 * fx - w * dx;
       ay[k] += w0 * fy - w * dy;
@@ -258,7 +241,7 @@ __device__ __forceinline__ void flash_fix(const Flash& P, const double4 s, const
 }
 
 // The source loop of k_eval_flash over [sb, se) for one target tile (tx, ty, tz held by the lanes).
-template <int K, int NT, bool PER, bool S32, bool QUIRKS>
+template <int K, int NT, bool PER, bool QUIRKS>
 __device__ __forceinline__ void flash_sources(const Flash& P, double4* ls, const double4* __restrict__ src4,
                                               int64_t sb, int64_t se, const double (&tx)[K],
                                               const double (&ty)[K], const double (&tz)[K],
@@ -276,7 +259,7 @@ __device__ __forceinline__ void flash_sources(const Flash& P, double4* ls, const
 #pragma unroll
         for (int k = 0; k < K; ++k) {
           double px, py, pz, pp;
-          flash_images<S32, QUIRKS>(P, tx[k] - s.x, ty[k] - s.y, tz[k] - s.z, px, py, pz, pp);
+          flash_images<QUIRKS>(P, tx[k] - s.x, ty[k] - s.y, tz[k] - s.z, px, py, pz, pp);
           ax[k] = fma(-s.w, px, ax[k]);
           ay[k] = fma(-s.w, py, ay[k]);
           az[k] = fma(-s.w, pz, az[k]);
@@ -297,7 +280,7 @@ __device__ __forceinline__ void flash_sources(const Flash& P, double4* ls, const
             const double dx = tx[k] - s.x, dy = ty[k] - s.y, dz = tz[k] - s.z;
             const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
             nj = nj || r2 < P.near2;
-            const double y = rsqrt_f64<S32 ? F_SEED32 : 0>(fmax(r2, P.near2));
+            const double y = rsqrt_f64<0>(fmax(r2, P.near2));
             const double mr = s.w * y;
             ap[k] += mr;
             const double w = mr * (y * y);
@@ -310,7 +293,7 @@ __device__ __forceinline__ void flash_sources(const Flash& P, double4* ls, const
         while (fm) {
           const int j = j0 + __builtin_ctzll(fm);
           fm &= fm - 1ULL;
-          flash_fix<K, S32>(P, ls[j], tx, ty, tz, ax, ay, az, ap);
+          flash_fix<K>(P, ls[j], tx, ty, tz, ax, ay, az, ap);
         }
       }
     }
@@ -318,15 +301,11 @@ __device__ __forceinline__ void flash_sources(const Flash& P, double4* ls, const
 }
 
 // blockIdx.x = target tile of K*NT targets, blockIdx.y = source chunk.  Accumulators follow
-// store_result's convention (a = G s, phi = -G s_p): s -= m kv d, s_p += m pk.  The FP32 seed of
-// 1/sqrt is taken per tile where the tile's r^2 bound (source statistics sst, images included)
-// keeps r^2 inside the FP32 range.
+// store_result's convention (a = G s, phi = -G s_p): s -= m kv d, s_p += m pk.
 template <int K, int NT, bool PER, bool QUIRKS = false>
 __global__ __launch_bounds__(NT) void k_eval_flash(Tgt T, const double4* __restrict__ src4,
-                                                   int64_t ns, int64_t chunk, Flash P,
-                                                   const double* sst, Out O) {
+                                                   int64_t ns, int64_t chunk, Flash P, Out O) {
   __shared__ double4 ls[NT];
-  __shared__ double red[2 * (NT / 64)];
   if (gated_off(O)) return;
   const int tid = threadIdx.x;
   const int64_t tile0 = (int64_t)blockIdx.x * (K * NT);
@@ -342,11 +321,7 @@ __global__ __launch_bounds__(NT) void k_eval_flash(Tgt T, const double4* __restr
     load_target(T, t < T.n ? t : T.n - 1, tx[k], ty[k], tz[k], e2);
     ax[k] = ay[k] = az[k] = ap[k] = 0.0;
   }
-  const double rt = tile_rmax<K, NT>(tx, ty, tz, tile0, T.n, red);
-  if (P.s32 && r2_bound(sst, rt, 0.0, P.reach) < TG_F32_HUGE_R2)   // uniform over the workgroup
-    flash_sources<K, NT, PER, true, QUIRKS>(P, ls, src4, sb, se, tx, ty, tz, ax, ay, az, ap);
-  else
-    flash_sources<K, NT, PER, false, QUIRKS>(P, ls, src4, sb, se, tx, ty, tz, ax, ay, az, ap);
+  flash_sources<K, NT, PER, QUIRKS>(P, ls, src4, sb, se, tx, ty, tz, ax, ay, az, ap);
 #pragma unroll
   for (int k = 0; k < K; ++k) {
     const int64_t t = tile0 + (int64_t)k * NT + tid;
@@ -624,7 +599,7 @@ __global__ __launch_bounds__(64) void k_eval_flash_pairs(Tgt T, int64_t t0, cons
         }
         if (r2 <= cut) {
           double kv, pk;
-          flash_pair<false>(P, r2, kv, pk);
+          flash_pair(P, r2, kv, pk);
           skv += kv;
           pz = fma(kv, dz, pz);
           if (QUIRKS) pp = pk;
@@ -673,7 +648,7 @@ __global__ __launch_bounds__(64) void k_pair_reduce(const double4* __restrict__ 
 // exactly (reference-rounded r2, exact threshold) as flash_fix does.  FAR: no target of the wave
 // comes within the clamp of the block (block_far), so no pair is clamped or flagged -- the same
 // arithmetic without the clamp, the flags and their ballots.
-template <int K, bool S32, bool FAR>
+template <int K, bool FAR>
 __device__ __forceinline__ void flash_gs_block(const Flash& P, const LdsGS<false>& L,
                                                const double (&tx)[K], const double (&ty)[K],
                                                const double (&tz)[K], double (&ax)[K],
@@ -700,7 +675,7 @@ __device__ __forceinline__ void flash_gs_block(const Flash& P, const LdsGS<false
         const double dz = tz[k] - zs;
         const double r2 = fma(dz, dz, base[k]);
         if (!FAR) nj = nj || r2 < P.near2;
-        const double y = rsqrt_f64<S32 ? F_SEED32 : 0>(FAR ? r2 : fmax(r2, P.near2));
+        const double y = rsqrt_f64<0>(FAR ? r2 : fmax(r2, P.near2));
         const double mr = m * y;
         ap[k] += mr;
         const double w = mr * (y * y);
@@ -723,7 +698,7 @@ __device__ __forceinline__ void flash_gs_block(const Flash& P, const LdsGS<false
         const double dz = tz[k] - zs;
         const double r2f = fma(dz, dz, base[k]);
         if (r2f < P.near2) {
-          const double y0 = rsqrt_f64<S32 ? F_SEED32 : 0>(P.near2);
+          const double y0 = rsqrt_f64<0>(P.near2);
           const double mr0 = m * y0;
           const double w0 = mr0 * (y0 * y0);
           double ex, ey, ez, r2;
@@ -735,7 +710,7 @@ __device__ __forceinline__ void flash_gs_block(const Flash& P, const LdsGS<false
             r2 = (ex * ex + ey * ey) + ez * ez;
           }
           double kv, pk;
-          flash_pair<S32>(P, r2, kv, pk);
+          flash_pair(P, r2, kv, pk);
           const double wv = m * kv;
           ax[k] += w0 * dx[k] - wv * ex;
           ay[k] += w0 * dy[k] - wv * ey;
@@ -774,7 +749,7 @@ __global__ __launch_bounds__(NT) void k_eval_flash_gridsrc(Tgt T, const double* 
                                                            const double* __restrict__ be2,
                                                            const double* __restrict__ bm,
                                                            int64_t nblk, int64_t chunk, Flash P,
-                                                           const double* sst, Out O) {
+                                                           Out O) {
   __shared__ LdsGS<false> L;
   if (gated_off(O)) return;   // explicit sources that turned out not to be 8^3 blocks
   const int tid = threadIdx.x;
@@ -789,20 +764,13 @@ __global__ __launch_bounds__(NT) void k_eval_flash_gridsrc(Tgt T, const double* 
     load_target(T, t < T.n ? t : T.n - 1, tx[k], ty[k], tz[k], e2);
     ax[k] = ay[k] = az[k] = ap[k] = 0.0;
   }
-  const double rt = tile_rmax<K, NT>(tx, ty, tz, tile0, T.n, L.red);
-  const bool s32 = P.s32 && r2_bound(sst, rt, 0.0) < TG_F32_HUGE_R2;   // uniform over the workgroup
   for (int64_t blk = b0; blk < b1; ++blk) {
     __syncthreads();
     gs_stage<false>(L, sax, be2, bm, blk, 0.0, 0.0, 0.0, 0.0);
     __syncthreads();
     const bool far = block_far<K>(P, L, tx, ty, tz);   // uniform over the wave
-    if (s32) {
-      if (far) flash_gs_block<K, true, true>(P, L, tx, ty, tz, ax, ay, az, ap);
-      else flash_gs_block<K, true, false>(P, L, tx, ty, tz, ax, ay, az, ap);
-    } else {
-      if (far) flash_gs_block<K, false, true>(P, L, tx, ty, tz, ax, ay, az, ap);
-      else flash_gs_block<K, false, false>(P, L, tx, ty, tz, ax, ay, az, ap);
-    }
+    if (far) flash_gs_block<K, true>(P, L, tx, ty, tz, ax, ay, az, ap);
+    else flash_gs_block<K, false>(P, L, tx, ty, tz, ax, ay, az, ap);
   }
   Out o = O;
   if (o.part) o.part += (int64_t)blockIdx.y * 4 * o.pstride;

@@ -60,11 +60,15 @@ __device__ __forceinline__ void stage_sync() {
 // the same 8 target z, and the staged sources carry their 8 dz.
 enum { F_ZROW = 16 };
 
+// FP64: one 112-byte record per source, so a wave reads a source at immediate offsets of one address.
+struct __align__(16) GridSrc {
+  double4 s;
+  double dz[8];       // F_ZROW: z_s - z_k of the 8 target cells
+  double e2, pad;
+};
 template <int NT>
 struct LdsGrid {
-  double4 s4[NT];
-  double se2[NT];
-  double dz[NT][8];   // F_ZROW: z_s - z_k of the 8 target cells
+  GridSrc src[NT];
 };
 template <int NT>
 struct LdsGridF {
@@ -86,8 +90,7 @@ struct LdsCol {
 };
 
 template <int FL>
-__device__ __forceinline__ void grid_tile_f64(const double4* __restrict__ s4, const double* __restrict__ se2,
-                                              const double (*__restrict__ sdz)[8], double tx, double ty,
+__device__ __forceinline__ void grid_tile_f64(const GridSrc* __restrict__ src, double tx, double ty,
                                               const double (&tz)[8], double (&ax)[8], double (&ay)[8],
                                               double (&az)[8], double (&ap)[8]) {
   // The 8 cells' dependency chains are written step by step across the cells (each step for all 8
@@ -96,19 +99,18 @@ __device__ __forceinline__ void grid_tile_f64(const double4* __restrict__ s4, co
   // slower).
 #pragma unroll 1
   for (int j = 0; j < 64; ++j) {
-    const double4 s = s4[j];
+    const double4 s = src[j].s;
     const double dx = s.x - tx, dy = s.y - ty;
-    const double base = fma(dx, dx, fma(dy, dy, se2[j]));
+    const double base = fma(dx, dx, fma(dy, dy, src[j].e2));
     double dz[8], r2[8], y[8], e[8];
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
-      dz[k] = (FL & F_ZROW) ? sdz[j][k] : s.z - tz[k];
+      dz[k] = (FL & F_ZROW) ? src[j].dz[k] : s.z - tz[k];
       r2[k] = fma(dz[k], dz[k], base);
     }
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
-      if (FL & F_SEED32) y[k] = (double)__builtin_amdgcn_rsqf((float)r2[k]);
-      else y[k] = __builtin_amdgcn_rsq(r2[k]);
+      y[k] = __builtin_amdgcn_rsq(r2[k]);
       if (FL & F_GUARD) y[k] = r2[k] > 0.0 ? y[k] : 0.0;
     }
 #pragma unroll
@@ -119,10 +121,12 @@ __device__ __forceinline__ void grid_tile_f64(const double4* __restrict__ s4, co
     for (int k = 0; k < 8; ++k) {
       const double mr = s.w * y[k];
       if (!(FL & F_NOPOT)) ap[k] += mr;
-      const double w = mr * (y[k] * y[k]);
-      ax[k] = fma(w, dx, ax[k]);
-      ay[k] = fma(w, dy, ay[k]);
-      az[k] = fma(w, dz[k], az[k]);
+      if constexpr (!(FL & F_NOACC)) {
+        const double w = mr * (y[k] * y[k]);
+        ax[k] = fma(w, dx, ax[k]);
+        ay[k] = fma(w, dy, ay[k]);
+        az[k] = fma(w, dz[k], az[k]);
+      }
     }
   }
 }
@@ -155,6 +159,10 @@ __device__ __forceinline__ void grid_tile_f32(const float4* __restrict__ s4, con
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
       if (FL & F_GUARD) y[k] = r2[k] > 0.0f ? y[k] : 0.0f;
+      if constexpr (FL & F_NOACC) {
+        ap[k] = fmaf(s.w, y[k], ap[k]);
+        continue;
+      }
       const float mr = s.w * y[k];
       if (!(FL & F_NOPOT)) ap[k] = fmaf(s.w, y[k], ap[k]);
       const float w = (mr * y[k]) * y[k];
@@ -179,15 +187,16 @@ __device__ __forceinline__ void grid_sources_f64(LdsGrid<64 * W>& L, const doubl
     stage_sync<W>();
     const int64_t j = base + tid;
     const double4 s = j < se ? src4[j] : make_double4(0.0, 0.0, 0.0, 0.0);
-    L.s4[tid] = s;
-    L.se2[tid] = j < se ? srce2[j] + e2t : 1.0;
+    GridSrc& G = L.src[tid];
+    G.s = s;
+    G.e2 = j < se ? srce2[j] + e2t : 1.0;
     if (FL & F_ZROW) {   // this lane's tz are every lane's
 #pragma unroll
-      for (int k = 0; k < 8; ++k) L.dz[tid][k] = s.z - tz[k];
+      for (int k = 0; k < 8; ++k) G.dz[k] = s.z - tz[k];
     }
     stage_sync<W>();
     if (W == 1 || base + 64 * v < se)   // uniform over the wave
-      grid_tile_f64<FL>(L.s4 + 64 * v, L.se2 + 64 * v, L.dz + 64 * v, tx, ty, tz, ax, ay, az, ap);
+      grid_tile_f64<FL>(L.src + 64 * v, tx, ty, tz, ax, ay, az, ap);
   }
 }
 
@@ -224,9 +233,11 @@ __device__ __forceinline__ void grid_sources_f32(LdsGridF<64 * W>& L, const doub
       tiles = 0;
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
-        hx[k] += (double)ax[k];
-        hy[k] += (double)ay[k];
-        hz[k] += (double)az[k];
+        if (!(FL & F_NOACC)) {
+          hx[k] += (double)ax[k];
+          hy[k] += (double)ay[k];
+          hz[k] += (double)az[k];
+        }
         if (!(FL & F_NOPOT)) hp[k] += (double)ap[k];
         ax[k] = ay[k] = az[k] = ap[k] = 0.f;
       }
@@ -234,9 +245,11 @@ __device__ __forceinline__ void grid_sources_f32(LdsGridF<64 * W>& L, const doub
   }
 #pragma unroll
   for (int k = 0; k < 8; ++k) {
-    hx[k] += (double)ax[k];
-    hy[k] += (double)ay[k];
-    hz[k] += (double)az[k];
+    if (!(FL & F_NOACC)) {
+      hx[k] += (double)ax[k];
+      hy[k] += (double)ay[k];
+      hz[k] += (double)az[k];
+    }
     if (!(FL & F_NOPOT)) hp[k] += (double)ap[k];
   }
 }
@@ -266,13 +279,13 @@ struct GridF32Run {
 };
 
 #define TG_DISPATCH_GRID_(FN, Z, fl, ...)                                     \
-  switch (fl & (F_GUARD | F_NOPOT | F_SEED32)) {                              \
+  switch (fl & (F_GUARD | F_NOPOT | F_NOACC)) {                               \
     case 0: FN<Z>(__VA_ARGS__); break;                                        \
     case F_GUARD: FN<Z | F_GUARD>(__VA_ARGS__); break;                        \
     case F_NOPOT: FN<Z | F_NOPOT>(__VA_ARGS__); break;                        \
     case F_NOPOT | F_GUARD: FN<Z | F_NOPOT | F_GUARD>(__VA_ARGS__); break;    \
-    case F_SEED32: FN<Z | F_SEED32>(__VA_ARGS__); break;                      \
-    default: FN<Z | F_SEED32 | F_NOPOT>(__VA_ARGS__); break;                  \
+    case F_NOACC: FN<Z | F_NOACC>(__VA_ARGS__); break;                        \
+    default: FN<Z | F_NOACC | F_GUARD>(__VA_ARGS__); break;                   \
   }
 #define TG_DISPATCH_GRID(FN, fl, ...)                                         \
   if (fl & F_ZROW) {                                                          \
@@ -323,16 +336,15 @@ __device__ __forceinline__ bool wave_sum(double* red, double (&a)[N], double (&b
 // t0 + k that share x, y and eps^2 (e2t, uniform over the wave) and differ in z[k]; (cx, cy, cz) is
 // the FP64 anchor of the mixed form (the centre of the group's bounding box); targets t0 + k with
 // k >= nk are not stored.  `o` already points at this source chunk's partials if the sources are
-// split over workgroups.  sst: the source statistics; rt: the largest |coordinate| of the targets
-// (FP64 seed choice); zrow: every lane of the workgroup holds the same z[8] (F_ZROW).
+// split over workgroups.  sst: the source statistics; zrow: every lane of the workgroup holds the same
+// z[8] (F_ZROW).
 template <bool MIXED, int W>
 __device__ __forceinline__ void grid_columns(
     LdsCol<MIXED, W>& L, double x, double y,
     const double (&z)[8], double e2t, double cx, double cy, double cz, int64_t t0, int nk,
     const double4* __restrict__ src4, const double* __restrict__ srce2, int64_t sb, int64_t se,
-    const double* sst, double rt, const Out& o, bool zrow) {
-  const int fl = tile_flags(sst[ST_E2MIN], e2t, e2t, o, MIXED, r2_bound(sst, rt, e2t)) |
-                 (zrow ? F_ZROW : 0);
+    const double* sst, const Out& o, bool zrow) {
+  const int fl = tile_flags(sst[ST_E2MIN], e2t, e2t, o, MIXED) | (zrow ? F_ZROW : 0);
   if constexpr (MIXED) {
     const float tx = (float)(x - cx), ty = (float)(y - cy);
     float tz[8];
@@ -341,7 +353,7 @@ __device__ __forceinline__ void grid_columns(
     double hx[8], hy[8], hz[8], hp[8];
 #pragma unroll
     for (int k = 0; k < 8; ++k) hx[k] = hy[k] = hz[k] = hp[k] = 0.0;
-    TG_DISPATCH_GRID(GridF32Run<W>::template run, fl & ~F_SEED32, L.t, src4, srce2, sb, se, e2t, cx,
+    TG_DISPATCH_GRID(GridF32Run<W>::template run, fl, L.t, src4, srce2, sb, se, e2t, cx,
                      cy, cz, tx, ty, tz, hx, hy, hz, hp)
     if (wave_sum<W, 8>(L.red, hx, hy, hz, hp)) {
 #pragma unroll
@@ -388,11 +400,8 @@ __device__ __forceinline__ void grid_block(LdsCol<MIXED, W>& L, const Tgt& T, in
     cy = 0.5 * ((oy + 0.5 * d) + (oy + 7.5 * d));
     cz = 0.5 * ((oz + 0.5 * d) + (oz + 7.5 * d));
   }
-  // every cell centre lies within [o, o + 8 d] on each axis
-  const double rt = fmax(max_abs3(T.ox[b], T.oy[b], T.oz[b]),
-                         max_abs3(T.ox[b] + 8.0 * d, T.oy[b] + 8.0 * d, T.oz[b] + 8.0 * d));
   grid_columns<MIXED, W>(L, x, y, z, e * e, cx, cy, cz, b * 512 + (int64_t)lane * 8, 8, src4, srce2,
-                         sb, se, sst, rt, o, true);
+                         sb, se, sst, o, true);
 }
 
 // blockIdx.x = leaf block, blockIdx.y = source chunk.  Requires T.blocks && T.nb == 8 and a
@@ -450,14 +459,6 @@ __device__ __forceinline__ void cols_group(LdsCol<MIXED, W>& L, const Tgt& T, in
     cy = 0.5 * (mn[1] + mx[1]);
     cz = 0.5 * (mn[2] + mx[2]);
   }
-  double rt = 0.0;   // the group's largest |coordinate| (the FP64 seed choice)
-  if constexpr (!MIXED) {
-    rt = fmax(fabs(x), fabs(y));
-#pragma unroll
-    for (int k = 0; k < 8; ++k) rt = fmax(rt, fabs(z[k]));
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) rt = fmax(rt, __shfl_xor(rt, off));
-  }
   // the same 8 z in every lane (every wave of the workgroup holds these targets): the C order of
   // 8^3 leaf blocks has it; a ragged group's clamped lanes and other layouts take the per-lane dz
   bool same = true;
@@ -466,7 +467,7 @@ __device__ __forceinline__ void cols_group(LdsCol<MIXED, W>& L, const Tgt& T, in
   const bool zrow = __all(same) != 0;
   const int64_t left = T.n - t0;
   grid_columns<MIXED, W>(L, x, y, z, e * e, cx, cy, cz, t0, left < 8 ? (int)left : 8, src4, srce2,
-                         sb, se, sst, rt, o, zrow);
+                         sb, se, sst, o, zrow);
 }
 
 // blockIdx.x = group of 512 targets, blockIdx.y = source chunk.  Gated (Out::gate) against
@@ -491,7 +492,6 @@ struct LdsGS {
   T m[512];                    // cell masses of the staged block, C order
   T cx[8], cy[8], cz[8];       // cell-centre coordinates (mixed: relative to the anchor)
   T e2;                        // block eps^2 (+ the tile's uniform target eps^2)
-  double red[2 * 4 * 4];
 };
 
 template <int K, bool MIXED, int FL>
@@ -542,6 +542,10 @@ __device__ __forceinline__ void gs_block(const LdsGS<MIXED>& L,
         for (int k = 0; k < K; ++k) {
           const int q = c * K + k;
           if (FL & F_GUARD) y[q] = r2[q] > 0.0f ? y[q] : 0.0f;
+          if constexpr (FL & F_NOACC) {
+            ap[k] = fmaf(m, y[q], ap[k]);
+            continue;
+          }
           const float mr = m * y[q];
           if (!(FL & F_NOPOT)) ap[k] = fmaf(m, y[q], ap[k]);
           const float w = (mr * y[q]) * y[q];
@@ -559,6 +563,10 @@ __device__ __forceinline__ void gs_block(const LdsGS<MIXED>& L,
         for (int k = 0; k < K; ++k) {
           const double dz = zs - tz[k];
           const double y = rsqrt_f64<FL>(fma(dz, dz, base[k]));
+          if constexpr (FL & F_NOACC) {
+            ap[k] = fma(m, y, ap[k]);
+            continue;
+          }
           const double mr = m * y;
           if (!(FL & F_NOPOT)) ap[k] += mr;
           const double w = (mr * y) * y;
@@ -567,7 +575,7 @@ __device__ __forceinline__ void gs_block(const LdsGS<MIXED>& L,
         }
       }
     }
-    if constexpr (!MIXED) {
+    if constexpr (!MIXED && !(FL & F_NOACC)) {
 #pragma unroll
       for (int k = 0; k < K; ++k) {
         ax[k] = fma(sw[k], dx[k], ax[k]);
@@ -734,8 +742,7 @@ __device__ __forceinline__ void gridsrc_tile(LdsGSW<MIXED, W>& L, const Tgt& T, 
     ay_ = 0.5 * (mn[1] + mx[1]);
     az_ = 0.5 * (mn[2] + mx[2]);
   }
-  const double rt = fmax(fmax(max_abs3(mn[0], mn[1], mn[2]), max_abs3(mx[0], mx[1], mx[2])), 0.0);
-  const int fl = tile_flags(sst[ST_E2MIN], mn[3], mx[3], o, MIXED, r2_bound(sst, rt, mx[3]));
+  const int fl = tile_flags(sst[ST_E2MIN], mn[3], mx[3], o, MIXED);
   TT tx[K], ty[K], tz[K], te2[K];
 #pragma unroll
   for (int k = 0; k < K; ++k) {
@@ -748,13 +755,8 @@ __device__ __forceinline__ void gridsrc_tile(LdsGSW<MIXED, W>& L, const Tgt& T, 
 #pragma unroll
   for (int k = 0; k < K; ++k) hx[k] = hy[k] = hz[k] = hp[k] = 0.0;
   typedef GsRun<K, W, MIXED> R;
-  if constexpr (MIXED) {
-    TG_DISPATCH8(R::template run, fl, L, sax, be2, bm, b0, b1, mn[3], ax_, ay_, az_, tx, ty, tz, te2,
-                 hx, hy, hz, hp)
-  } else {
-    TG_DISPATCH(R::template run, fl, L, sax, be2, bm, b0, b1, mn[3], ax_, ay_, az_, tx, ty, tz, te2,
-                hx, hy, hz, hp)
-  }
+  TG_DISPATCH(R::template run, fl, L, sax, be2, bm, b0, b1, mn[3], ax_, ay_, az_, tx, ty, tz, te2,
+              hx, hy, hz, hp)
   if (!wave_sum<W, K>(L.red, hx, hy, hz, hp)) return;
 #pragma unroll
   for (int k = 0; k < K; ++k) {

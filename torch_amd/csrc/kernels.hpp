@@ -34,6 +34,7 @@ struct Out {
   int64_t pstride;
   double G;
   int nopot = 0;                // 1: the potential is not wanted (its accumulator is skipped)
+  int noacc = 0;                // 1: only the potential is wanted (no acceleration, no kick)
   const int* gate = nullptr;    // non-null: the kernel runs only if *gate == gate_on, else it
   int gate_on = 0;              //   returns at once (one of several launches picked on the device)
 };
@@ -113,10 +114,8 @@ __device__ __forceinline__ void block_minmax(double (&mn)[NV], double (&mx)[NV],
 //   F_GUARD  the tile's smallest possible eps^2 is 0: zero r2 -> the pair contributes 0
 //   F_UNIF   all targets of the tile share eps_t^2: folded into the staged source eps^2
 //   F_NOPOT  the caller did not ask for the potential
-//   F_SEED32 (FP64 only, built with TG_FP64_SEED32 = 1) r2 >= 1e-30 is guaranteed: seed 1/sqrt
-//            from v_rsq_f32 instead of the quarter-rate v_rsq_f64 (both seeds are ~2^-24 accurate;
-//            the refinement is the same)
-enum { F_GUARD = 1, F_UNIF = 2, F_NOPOT = 4, F_SEED32 = 8 };
+//   F_NOACC  the caller asked for the potential only (never together with F_NOPOT)
+enum { F_GUARD = 1, F_UNIF = 2, F_NOPOT = 4, F_NOACC = 8 };
 
 // --------------------------------------------------------------- FP64 tile loop ----
 // 1/sqrt(r2) in FP64: a hardware estimate refined by one third-order Newton/Householder
@@ -124,9 +123,7 @@ enum { F_GUARD = 1, F_UNIF = 2, F_NOPOT = 4, F_SEED32 = 8 };
 // an estimate with relative error d leaves ~2.5 d^3, below FP64 rounding for d ~ 2^-24).
 template <int FL>
 __device__ __forceinline__ double rsqrt_f64(double r2) {
-  double y;
-  if (FL & F_SEED32) y = (double)__builtin_amdgcn_rsqf((float)r2);
-  else y = __builtin_amdgcn_rsq(r2);
+  double y = __builtin_amdgcn_rsq(r2);
   if (FL & F_GUARD) y = r2 > 0.0 ? y : 0.0;   // |d|^2 + eps^2 == 0: the pair contributes 0
   const double t = r2 * y;
   const double e = fma(-t, y, 1.0);
@@ -151,6 +148,10 @@ __device__ __forceinline__ void fp64_tile(const double4* __restrict__ s4,
       const double dx = s.x - tx[k], dy = s.y - ty[k], dz = s.z - tz[k];
       const double r2 = fma(dx, dx, fma(dy, dy, fma(dz, dz, (FL & F_UNIF) ? e2 : e2 + te2[k])));
       const double y = rsqrt_f64<FL>(r2);
+      if constexpr (FL & F_NOACC) {
+        ap[k] = fma(s.w, y, ap[k]);
+        continue;
+      }
       const double mr = s.w * y;
       if (!(FL & F_NOPOT)) ap[k] += mr;
       const double w = mr * (y * y);
@@ -226,6 +227,10 @@ __device__ __forceinline__ void f32_tile(const float4* __restrict__ s4,
       for (int k = 0; k < K; ++k) {
         const int q = i * K + k;
         if (FL & F_GUARD) y[q] = r2[q] > 0.0f ? y[q] : 0.0f;
+        if constexpr (FL & F_NOACC) {
+          ap[k] = fmaf(s[i].w, y[q], ap[k]);
+          continue;
+        }
         const float mr = s[i].w * y[q];
         if (!(FL & F_NOPOT)) ap[k] = fmaf(s[i].w, y[q], ap[k]);
         const float w = (mr * y[q]) * y[q];
@@ -260,21 +265,8 @@ struct LdsF32 {
 };
 
 // Threshold on the smallest possible eps^2 of a tile below which the FP32 loop guards
-// r2 == 0 (and keeps rsq far from overflow) and the FP64 loop keeps the v_rsq_f64 seed.
+// r2 == 0 (and keeps rsq far from overflow).
 #define TG_F32_TINY_E2 1e-30
-// Bound on a tile's largest r^2 above which the FP64 loop keeps the v_rsq_f64 seed: the FP32
-// seed converts r^2 to float, and FLT_MAX is 3.4e38 (a separation of 1.8e19 in the caller's
-// units; cgs coordinates of a few kpc reach it).
-#define TG_F32_HUGE_R2 1e36
-// 1: the FP64 kernels seed 1/sqrt from v_rsq_f32 of the converted r2 where the tile's range allows
-// (F_SEED32, P.s32); 0: from v_rsq_f64 everywhere.  Measured on MI355X with the block kernels'
-// instruction mixes, the v_rsq_f64 seed (one quarter-rate transcendental, which the FP64 arithmetic
-// around it hides) is as fast or faster than the two conversions plus v_rsq_f32: c4 FP64 column
-// kernel 25.25 against 27.13 ms on one box and 26.55 against 26.69 on another, c5 forward 200.0
-// against 202.2 ms, c2 5.20 / 5.03 against 5.29 / 5.08 ms; the FLASH kernels within 1% either way.
-#ifndef TG_FP64_SEED32
-#define TG_FP64_SEED32 0
-#endif
 
 // Statistics of a packed source set, device words written by the pack kernels: doubles stored as
 // their bits (non-negative, so integer atomicMin / atomicMax order them like the values).
@@ -286,15 +278,6 @@ enum {
   ST_MMAX = 4,    // largest |m|
   ST_WORDS = 5
 };
-
-// Upper bound on r^2 = |x_s - x_t|^2 + eps_s^2 + eps_t^2 over the tile's pairs, from the source
-// statistics `sst` and the tile's largest |coordinate| `rt` and eps_t^2; `reach` widens the
-// displacement (periodic images).
-__device__ __forceinline__ double r2_bound(const double* sst, double rt, double e2t_max,
-                                           double reach = 0.0) {
-  const double d = sst[ST_RMAX] + rt + reach;
-  return 3.0 * d * d + sst[ST_E2MAX] + e2t_max;
-}
 
 __device__ __forceinline__ double max_abs3(double x, double y, double z) {
   return fmax(fabs(x), fmax(fabs(y), fabs(z)));
@@ -311,11 +294,13 @@ __device__ __forceinline__ void kick_one(const Out& O, int64_t t, double gx, dou
 
 __device__ __forceinline__ void store_result(const Out& O, int64_t t, double sx, double sy,
                                              double sz, double sp) {
-  if (O.part) {
-    O.part[t] = sx;
-    O.part[O.pstride + t] = sy;
-    O.part[2 * O.pstride + t] = sz;
-    O.part[3 * O.pstride + t] = sp;
+  if (O.part) {                 // components that nobody wants are neither written nor read back
+    if (!O.noacc) {
+      O.part[t] = sx;
+      O.part[O.pstride + t] = sy;
+      O.part[2 * O.pstride + t] = sz;
+    }
+    if (!O.nopot) O.part[3 * O.pstride + t] = sp;
     return;
   }
   const double gx = O.G * sx, gy = O.G * sy, gz = O.G * sz;
@@ -326,20 +311,15 @@ __device__ __forceinline__ void store_result(const Out& O, int64_t t, double sx,
   if (O.vx) kick_one(O, t, gx, gy, gz);
 }
 
-// Code path of a tile from its smallest/largest target eps^2, the sources' smallest and (FP64)
-// a bound on the tile's largest r^2: the FP32 seed needs r^2 inside [1e-30, 1e36].
+// Code path of a tile from its smallest/largest target eps^2 and the sources' smallest.
 __device__ __forceinline__ int tile_flags(double e2s_min, double e2t_min, double e2t_max,
-                                          const Out& O, bool f32, double r2max = 0.0) {
+                                          const Out& O, bool f32) {
   int fl = 0;
   if (e2t_min == e2t_max) fl |= F_UNIF;
   const double lo = e2s_min + e2t_min;
-  if (f32) {
-    if (!(lo > TG_F32_TINY_E2)) fl |= F_GUARD;
-  } else {
-    if (!(lo > 0.0)) fl |= F_GUARD;
-    else if (TG_FP64_SEED32 && lo > TG_F32_TINY_E2 && r2max < TG_F32_HUGE_R2) fl |= F_SEED32;
-  }
+  if (!(lo > (f32 ? TG_F32_TINY_E2 : 0.0))) fl |= F_GUARD;
   if (O.nopot) fl |= F_NOPOT;
+  else if (O.noacc) fl |= F_NOACC;
   return fl;
 }
 
@@ -367,18 +347,6 @@ __device__ __forceinline__ void fp64_sources(LdsF64<NT>& L, const double4* __res
   }
 }
 
-#define TG_DISPATCH8(FN, fl, ...)                                             \
-  switch (fl & ~F_SEED32) {                                                   \
-    case 0: FN<0>(__VA_ARGS__); break;                                        \
-    case F_GUARD: FN<F_GUARD>(__VA_ARGS__); break;                            \
-    case F_UNIF: FN<F_UNIF>(__VA_ARGS__); break;                              \
-    case F_UNIF | F_GUARD: FN<F_UNIF | F_GUARD>(__VA_ARGS__); break;          \
-    case F_NOPOT: FN<F_NOPOT>(__VA_ARGS__); break;                            \
-    case F_NOPOT | F_GUARD: FN<F_NOPOT | F_GUARD>(__VA_ARGS__); break;        \
-    case F_NOPOT | F_UNIF: FN<F_NOPOT | F_UNIF>(__VA_ARGS__); break;          \
-    default: FN<F_NOPOT | F_UNIF | F_GUARD>(__VA_ARGS__); break;              \
-  }
-
 #define TG_DISPATCH(FN, fl, ...)                                              \
   switch (fl) {                                                               \
     case 0: FN<0>(__VA_ARGS__); break;                                        \
@@ -389,10 +357,10 @@ __device__ __forceinline__ void fp64_sources(LdsF64<NT>& L, const double4* __res
     case F_NOPOT | F_GUARD: FN<F_NOPOT | F_GUARD>(__VA_ARGS__); break;        \
     case F_NOPOT | F_UNIF: FN<F_NOPOT | F_UNIF>(__VA_ARGS__); break;          \
     case F_NOPOT | F_UNIF | F_GUARD: FN<F_NOPOT | F_UNIF | F_GUARD>(__VA_ARGS__); break; \
-    case F_SEED32: FN<F_SEED32>(__VA_ARGS__); break;                          \
-    case F_SEED32 | F_UNIF: FN<F_SEED32 | F_UNIF>(__VA_ARGS__); break;        \
-    case F_SEED32 | F_NOPOT: FN<F_SEED32 | F_NOPOT>(__VA_ARGS__); break;      \
-    default: FN<F_SEED32 | F_NOPOT | F_UNIF>(__VA_ARGS__); break;             \
+    case F_NOACC: FN<F_NOACC>(__VA_ARGS__); break;                            \
+    case F_NOACC | F_GUARD: FN<F_NOACC | F_GUARD>(__VA_ARGS__); break;        \
+    case F_NOACC | F_UNIF: FN<F_NOACC | F_UNIF>(__VA_ARGS__); break;          \
+    default: FN<F_NOACC | F_UNIF | F_GUARD>(__VA_ARGS__); break;              \
   }
 
 template <int K, int NT>
@@ -416,7 +384,7 @@ __device__ void process_fp64(LdsF64<NT>& L, const Tgt& T, int64_t tile0,
                              int64_t s_begin, int64_t s_end, const double* sst, const Out& O) {
   const int tid = threadIdx.x;
   double tx[K], ty[K], tz[K], te2[K];
-  double mn[2] = {INFINITY, INFINITY}, mx[2] = {-INFINITY, 0.0};   // eps^2; |coordinate| (max only)
+  double mn[1] = {INFINITY}, mx[1] = {-INFINITY};   // eps^2
 #pragma unroll
   for (int k = 0; k < K; ++k) {
     const int64_t t = tile0 + (int64_t)k * NT + tid;
@@ -424,11 +392,10 @@ __device__ void process_fp64(LdsF64<NT>& L, const Tgt& T, int64_t tile0,
     if (t < T.n) {
       mn[0] = fmin(mn[0], te2[k]);
       mx[0] = fmax(mx[0], te2[k]);
-      mx[1] = fmax(mx[1], max_abs3(tx[k], ty[k], tz[k]));
     }
   }
-  block_minmax<NT, 2>(mn, mx, L.red);
-  const int fl = tile_flags(sst[ST_E2MIN], mn[0], mx[0], O, false, r2_bound(sst, mx[1], mx[0]));
+  block_minmax<NT, 1>(mn, mx, L.red);
+  const int fl = tile_flags(sst[ST_E2MIN], mn[0], mx[0], O, false);
   double ax[K], ay[K], az[K], ap[K];
 #pragma unroll
   for (int k = 0; k < K; ++k) ax[k] = ay[k] = az[k] = ap[k] = 0.0;
@@ -533,7 +500,7 @@ __device__ void process_mixed(LdsF32<NT>& L, const Tgt& T, int64_t tile0,
 #pragma unroll
   for (int k = 0; k < K; ++k) hx[k] = hy[k] = hz[k] = hp[k] = lx[k] = ly[k] = lz[k] = lp[k] = 0.f;
   typedef MixRun<K, NT> R;
-  TG_DISPATCH8(R::template run, fl, L, src4, srce2, s_begin, s_end, mn[3], cx, cy, cz, tx,
+  TG_DISPATCH(R::template run, fl, L, src4, srce2, s_begin, s_end, mn[3], cx, cy, cz, tx,
               ty, tz, te2, hx, hy, hz, hp, lx, ly, lz, lp)
 #pragma unroll
   for (int k = 0; k < K; ++k) {
@@ -584,10 +551,12 @@ __global__ void k_reduce_chunks(const double* __restrict__ part, int64_t pstride
   double s0 = 0, s1 = 0, s2 = 0, s3 = 0;
   for (int c = 0; c < nsplit; ++c) {
     const double* p = part + (int64_t)c * 4 * pstride;
-    s0 += p[t];
-    s1 += p[pstride + t];
-    s2 += p[2 * pstride + t];
-    s3 += p[3 * pstride + t];
+    if (!O.noacc) {
+      s0 += p[t];
+      s1 += p[pstride + t];
+      s2 += p[2 * pstride + t];
+    }
+    if (!O.nopot) s3 += p[3 * pstride + t];
   }
   Out o = O;
   o.part = nullptr;
@@ -611,10 +580,12 @@ __global__ __launch_bounds__(1024) void k_reduce_chunks_wide(const double* __res
   if (t < n) {
     for (int c = c0; c < c1; ++c) {
       const double* p = part + (int64_t)c * 4 * pstride;
-      s0 += p[t];
-      s1 += p[pstride + t];
-      s2 += p[2 * pstride + t];
-      s3 += p[3 * pstride + t];
+      if (!O.noacc) {
+        s0 += p[t];
+        s1 += p[pstride + t];
+        s2 += p[2 * pstride + t];
+      }
+      if (!O.nopot) s3 += p[3 * pstride + t];
     }
   }
   red[w][0][lane] = s0;

@@ -637,6 +637,9 @@ static int column_kernel(tgrav_ctx* c, int mode, bool blocks, int64_t ngrp, int 
   return 0;
 }
 
+// Only the potential is asked for: the Plummer kernels then skip the acceleration.
+static int potential_only(const tg::Out& O) { return O.phi && !O.ax && !O.ay && !O.az && !O.vx; }
+
 static int launch_grid(tgrav_ctx* c, int mode, const tg::Tgt& T, const tg::Out& O) {
   const int64_t nt = T.n, ns = c->ns, nblk = nt / 512;
   if (nblk > 0x7fffffffLL) return fail(TGRAV_ELIMIT, "too many blocks");
@@ -791,8 +794,7 @@ static int flash_gridsrc_kernel(tgrav_ctx* c, const tg::Tgt& T, const tg::Out& o
   const int K = TG_FLASH_GS_K, NT = 256;
   const dim3 g((unsigned)ntiles, (unsigned)nsplit);
   tg::k_eval_flash_gridsrc<K, NT><<<g, NT, 0, c->stream>>>(
-      T, c->sax.as<double>(), c->sbe2.as<double>(), c->sms.as<double>(), nblk, chunk, P,
-      c->stat.as<const double>(), o);
+      T, c->sax.as<double>(), c->sbe2.as<double>(), c->sms.as<double>(), nblk, chunk, P, o);
   LAUNCHCHECK("k_eval_flash_gridsrc");
   return 0;
 }
@@ -874,10 +876,6 @@ static int launch_flash(tgrav_ctx* c, int mode, const tg::Tgt& T, const tg::Out&
   P.type = c->soft;
   P.quirks = c->soft_quirks;
   P.nrep = per ? c->nrep : 0;
-  // Pairs reaching the refined 1/sqrt have r2 >= rsoft^2 (the rest take the softened
-  // branch); the FP32 seed is valid from 1e-30 up, and up to the tile's r^2 bound (in the kernels).
-  P.s32 = TG_FP64_SEED32 && c->rsoft * c->rsoft > TG_F32_TINY_E2;
-  P.reach = per ? (double)(c->nrep + 1) * std::max(P.lx, std::max(P.ly, P.lz)) : 0.0;
   // Periodic sums with the pairs grouped by separation, where the row table fits in LDS (nrep <= 7
   // static, nrep <= 10 sized at launch), in batches of targets of at most 2^25 pairs (1.3 GB of pair
   // arrays); tgrav_set_periodic(on = 2) keeps the per-target walk.
@@ -934,14 +932,13 @@ static int launch_flash(tgrav_ctx* c, int mode, const tg::Tgt& T, const tg::Out&
     if (srcb) return 0;
     const dim3 g((unsigned)ntiles, (unsigned)nsplit);
     const double4* s4 = c->s4.as<double4>();
-    const double* sst = c->stat.as<const double>();
     if (per) {
       if (P.quirks)
-        tg::k_eval_flash<1, 256, true, true><<<g, NT, 0, c->stream>>>(T, s4, ns, chunk, P, sst, o);
+        tg::k_eval_flash<1, 256, true, true><<<g, NT, 0, c->stream>>>(T, s4, ns, chunk, P, o);
       else
-        tg::k_eval_flash<1, 256, true, false><<<g, NT, 0, c->stream>>>(T, s4, ns, chunk, P, sst, o);
+        tg::k_eval_flash<1, 256, true, false><<<g, NT, 0, c->stream>>>(T, s4, ns, chunk, P, o);
     } else {
-      tg::k_eval_flash<2, 256, false><<<g, NT, 0, c->stream>>>(T, s4, ns, chunk, P, sst, o);
+      tg::k_eval_flash<2, 256, false><<<g, NT, 0, c->stream>>>(T, s4, ns, chunk, P, o);
     }
     LAUNCHCHECK("k_eval_flash");
     return 0;
@@ -1432,6 +1429,7 @@ static int eval_common(tgrav_ctx* c, tg::Tgt T, const double* tin[5], int ntin, 
       }
     tg::Out O{dout[0], dout[1], dout[2], dout[3], dvel[0], dvel[1], dvel[2], dt, nullptr, 0, c->G,
               outs[3] == nullptr};
+    O.noacc = potential_only(O);
     if ((rc = launch_eval(c, mode, T, O))) return rc;
     for (int q = 0; q < 4; ++q)
       if (outs[q])
@@ -1451,6 +1449,7 @@ static int eval_common(tgrav_ctx* c, tg::Tgt T, const double* tin[5], int ntin, 
   if (mode == TGRAV_MIXED && c->validate && (rc = eval_range_check(c, T, nin))) return rc;
   tg::Out O{outs[0], outs[1], outs[2], outs[3], vel[0], vel[1], vel[2], dt, nullptr, 0, c->G,
             outs[3] == nullptr};
+  O.noacc = potential_only(O);
   return launch_eval(c, mode, T, O);
 }
 
@@ -1568,6 +1567,7 @@ int tgrav_eval_static(tgrav_ctx* c, int64_t ns, const double* sx, const double* 
   tg::Tgt T{};
   T.x = x; T.y = y; T.z = z; T.eps = eps_t; T.n = nt;
   tg::Out O{ax, ay, az, phi, nullptr, nullptr, nullptr, 0.0, nullptr, 0, c->G, phi == nullptr};
+  O.noacc = potential_only(O);
   tg::Out o = O;
   o.part = nsplit > 1 ? part : nullptr;
   o.pstride = nt;
