@@ -1,0 +1,125 @@
+"""GPU tests of the one-pass input checks: statistics, NaN/Inf and structure found in a single launch
+over one or many workgroups, and block sources expanded only where a kernel reads them cell by cell
+(needs an MI355X)."""
+import numpy as np
+import pytest
+
+from torch_amd import GasGravityField, StellarGravityField, TgravError, _lib
+from torch_amd import workloads as W
+
+pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
+
+
+def dev(*arrs):
+    return [torch.as_tensor(np.ascontiguousarray(a), device="cuda") for a in arrs]
+
+
+# one lane, one workgroup, its edges, two workgroups, many, and past the most workgroups of a launch
+@pytest.mark.parametrize("n", [1, 255, 256, 257, 512, 4097, 131072, 131073, 400000])
+def test_bad_values_are_found_anywhere(n):
+    """The first, the last and a middle element of every input array: refused as source and as target,
+    and the next call on good inputs is accepted and equals the one before."""
+    rng = W.rng_for(n)
+    x, y, z, m, e = dev(*rng.uniform(-1, 1, (3, n)), rng.uniform(0.1, 1, n), np.full(n, 0.01))
+    few = [a[:7].clone() for a in (e, x, y, z)]
+    with StellarGravityField("fp64") as f:
+        f.set_stars(x[:3].clone(), y[:3].clone(), z[:3].clone(), m[:3].clone(), e[:3].clone())
+        ref = f.evaluate(e, x, y, z)
+        for q in range(4):
+            a = [e, x, y, z]
+            for at in {0, n // 2, n - 1}:
+                for v in (float("nan"), float("inf")):
+                    a[q] = a[q].clone()
+                    keep = float(a[q][at])
+                    a[q][at] = v
+                    with pytest.raises(TgravError) as err:
+                        f.evaluate(*a)
+                    assert err.value.code == _lib.ENONFINITE
+                    a[q][at] = keep
+        for r, g in zip(ref, f.evaluate(e, x, y, z)):
+            assert torch.equal(r, g)
+        src = [x, y, z, m, e]
+        for q in range(5):
+            for at in {0, n // 2, n - 1}:
+                bad = list(src)
+                bad[q] = src[q].clone()
+                bad[q][at] = float("nan")
+                with pytest.raises(TgravError) as err:
+                    f.set_stars(*bad)
+                assert err.value.code == _lib.ENONFINITE
+                with pytest.raises(TgravError) as err:     # no source set is left behind
+                    f.evaluate(*few)
+                assert err.value.code == _lib.ENOSOURCES
+        f.set_stars(*src)
+        assert torch.isfinite(f.evaluate(*few)[3]).all()
+
+
+@pytest.mark.parametrize("nblk", [1, 3, 300, 1025])
+def test_structure_is_decided_by_every_element(nblk):
+    """Explicit cells in block order take the column and block-source kernels, whose sums differ in
+    rounding from the generic kernel's; one moved cell, anywhere, sends the call to the generic one.
+    With and without validation (decided on the host, gated on the device) the bits are the same."""
+    rng = W.rng_for(nblk)
+    from torch_amd.blocks import block_centres
+    o = rng.uniform(-1, 1, (nblk, 3))
+    x, y, z, dx = block_centres(o, rng.uniform(0.01, 0.05, nblk))
+    m = rng.uniform(0.5, 1, x.size)
+    st = dev(*rng.uniform(-1, 1, (3, 700)), rng.uniform(0.1, 1, 700), np.full(700, 0.01))
+    for move in (None, 0, x.size // 2, x.size - 1):
+        cx = x.copy()
+        if move is not None:
+            cx[move] += 1e-3
+        c = dev(cx, y, z, m, dx)
+        got = []
+        for validate in (True, False):
+            with StellarGravityField("fp64", validate=validate) as f, GasGravityField("fp64", validate=validate) as g:
+                f.set_stars(*st)
+                a = f.evaluate(None, c[0], c[1], c[2])
+                g.set_sources(*c)
+                b = g.evaluate(None, st[0], st[1], st[2])
+                f.set_block_kernel(False)
+                g.set_block_kernel(False)
+                got.append(a + b)
+                if validate:
+                    plain = f.evaluate(None, c[0], c[1], c[2]) + g.evaluate(None, st[0], st[1], st[2])
+        for p, q in zip(*got):
+            assert torch.equal(p, q)
+        for p, q in zip(got[0], plain):
+            assert torch.allclose(p, q, rtol=1e-11, atol=1e-11 * float(q.abs().max()))
+        if move is not None:
+            assert all(torch.equal(p, q) for p, q in zip(got[0], plain))
+
+
+@pytest.mark.parametrize("nblk", [1, 5])
+def test_block_sources_expand_where_needed(nblk):
+    """Block sources under every kernel that reads them cell by cell equal the same cells given as
+    points, also after the set is replaced (and through a graph captured before that)."""
+    rng = W.rng_for(77 + nblk)
+    from torch_amd.blocks import block_centres
+    o, d = rng.uniform(-1, 1, (nblk, 3)), rng.uniform(0.02, 0.1, nblk)
+    x, y, z, dx = block_centres(o, d)
+    to, td = dev(rng.uniform(-1, 1, (2, 3)), np.full(2, 0.03))
+    t = dev(*rng.uniform(-1, 1, (3, 300)))
+    masses = [rng.uniform(0.5, 1, x.size) for _ in range(2)]
+    with GasGravityField("fp64", validate=False) as g, GasGravityField("fp64") as p:
+        g.set_block_kernel(False)
+        p.set_block_kernel(False)
+        outs = None
+        graph = torch.cuda.CUDAGraph()
+        for step, m in enumerate(masses):
+            g.set_blocks(*dev(o, d, m))
+            p.set_sources(*dev(x, y, z, m, dx))
+            a = g.evaluate(None, *t) + g.evaluate_blocks(to, td)
+            b = p.evaluate(None, *t) + p.evaluate_blocks(to, td)
+            for q, r in zip(a, b):
+                assert torch.equal(q, r)
+            if step == 0:
+                torch.cuda.synchronize()
+                with torch.cuda.graph(graph):
+                    outs = g.evaluate(None, *t)
+            for _ in range(3):
+                graph.replay()
+                torch.cuda.synchronize()
+                for q, r in zip(outs, b):
+                    assert torch.equal(q, r)

@@ -166,7 +166,8 @@ __global__ void k_batch_check_cols(int ncand, const int* __restrict__ ids,
   if (i >= prefix[ncand]) return;
   const int q = find_segment(prefix, ncand, i);
   const int p = ids[q];
-  if (!column_ok(probs[p].T, i - prefix[q])) {
+  const Tgt& T = probs[p].T;
+  if (!column_ok(T.x, T.y, T.eps, i - prefix[q])) {
     colflag[p] = 0;
     counter[3] = 0u;
   }

@@ -120,7 +120,7 @@ __device__ __forceinline__ void grid_tile_f64(const GridSrc* __restrict__ src, d
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
       const double mr = s.w * y[k];
-      if (!(FL & F_NOPOT)) ap[k] += mr;
+      if (!(FL & F_NOPOT)) ap[k] = fma(s.w, y[k], ap[k]);
       if constexpr (!(FL & F_NOACC)) {
         const double w = mr * (y[k] * y[k]);
         ax[k] = fma(w, dx, ax[k]);
@@ -419,6 +419,32 @@ __global__ __launch_bounds__(64 * W, MIXED ? 3 : 1) void k_eval_grid(Tgt T, cons
   grid_block<MIXED, W>(L, T, blockIdx.x, src4, srce2, sb, se, sst, o);
 }
 
+// Mixed anchor of a group of 512 explicit targets: the centre of their bounding box.  Lane l of a wave
+// (each wave of the workgroup alike) takes column l.
+__device__ __forceinline__ void column_anchor(const Tgt& T, int64_t g, int lane, double& cx, double& cy, double& cz) {
+  const int64_t t0 = g * 512 + (int64_t)lane * 8, last = T.n - 1;
+  const int64_t tc = t0 < last ? t0 : last;
+  double mn[3] = {T.x[tc], T.y[tc], T.z[tc]};
+  double mx[3] = {mn[0], mn[1], mn[2]};
+#pragma unroll
+  for (int k = 1; k < 8; ++k) {
+    const double z = T.z[t0 + k < last ? t0 + k : last];
+    mn[2] = fmin(mn[2], z);
+    mx[2] = fmax(mx[2], z);
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+#pragma unroll
+    for (int v = 0; v < 3; ++v) {
+      mn[v] = fmin(mn[v], __shfl_xor(mn[v], off));
+      mx[v] = fmax(mx[v], __shfl_xor(mx[v], off));
+    }
+  }
+  cx = 0.5 * (mn[0] + mx[0]);
+  cy = 0.5 * (mn[1] + mx[1]);
+  cz = 0.5 * (mn[2] + mx[2]);
+}
+
 // Explicit targets with column structure (every aligned group of 8 consecutive targets shares
 // x and y, every aligned group of 512 shares eps: the C order of 8^3 leaf-block meshgrids, as
 // checked by k_check_cols): the column code of k_eval_grid on explicit coordinates.  Group g =
@@ -440,25 +466,7 @@ __device__ __forceinline__ void cols_group(LdsCol<MIXED, W>& L, const Tgt& T, in
   const int64_t te = g * 512 < last ? g * 512 : last;
   const double e = T.eps ? T.eps[te] : 0.0;
   double cx = 0.0, cy = 0.0, cz = 0.0;
-  if constexpr (MIXED) {   // centre of the bounding box of the group's targets
-    double mn[3] = {x, y, z[0]}, mx[3] = {x, y, z[0]};
-#pragma unroll
-    for (int k = 1; k < 8; ++k) {
-      mn[2] = fmin(mn[2], z[k]);
-      mx[2] = fmax(mx[2], z[k]);
-    }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-#pragma unroll
-      for (int v = 0; v < 3; ++v) {
-        mn[v] = fmin(mn[v], __shfl_xor(mn[v], off));
-        mx[v] = fmax(mx[v], __shfl_xor(mx[v], off));
-      }
-    }
-    cx = 0.5 * (mn[0] + mx[0]);
-    cy = 0.5 * (mn[1] + mx[1]);
-    cz = 0.5 * (mn[2] + mx[2]);
-  }
+  if constexpr (MIXED) column_anchor(T, g, lane, cx, cy, cz);
   // the same 8 z in every lane (every wave of the workgroup holds these targets): the C order of
   // 8^3 leaf blocks has it; a ragged group's clamped lanes and other layouts take the per-lane dz
   bool same = true;
@@ -793,70 +801,56 @@ __global__ __launch_bounds__(64 * W) void k_eval_gridsrc(Tgt T, const double* __
   gridsrc_tile<K, W, MIXED>(L, T, tile * (K * 64), sax, be2, bm, b0, b1, sst, o);
 }
 
-// Expands 8^3 source blocks into the packed per-cell form (so every kernel can use them),
-// writes each block's eps^2 (be2), cell-centre axes (sax) and the cell masses as one contiguous
-// array (sm; the three staged by the block-source kernels, which then read 8 B per cell instead
-// of a 32 B record) and folds the source statistics (ST_*) into stat; one lane per cell,
-// workgroups of 256 lanes.
+// Source set given as 8^3 blocks, in the form the block-source kernels read: each block's eps^2 (be2),
+// its cell-centre axes (sax) and the cell masses as one contiguous array (sm), 8 B per cell, with the
+// set's statistics; with `check`, a NaN/Inf input sets ST_BAD.  One lane per cell.
 __global__ __launch_bounds__(256) void k_pack_source_blocks(int64_t nblk, const double* __restrict__ ox,
                                      const double* __restrict__ oy, const double* __restrict__ oz,
                                      const double* __restrict__ dx, const double* __restrict__ m,
-                                     const double* __restrict__ eps, double4* __restrict__ s4,
-                                     double* __restrict__ se2, double* __restrict__ be2,
-                                     double* __restrict__ sax, double* __restrict__ sm,
-                                     unsigned long long* stat) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+                                     const double* __restrict__ eps, double* __restrict__ be2,
+                                     double* __restrict__ sax, double* __restrict__ sm, int check, Publish P) {
   unsigned long long e2min = 0x7ff0000000000000ULL, rmax = 0ULL, e2max = 0ULL, mmax = 0ULL;
-  if (i < nblk * 512) {
+  int bad = 0;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < nblk * 512; i += (int64_t)gridDim.x * 256) {
     const int64_t b = i >> 9;
     const int c = (int)(i & 511);
-    const double d = dx[b];
-    double x, y, z;
-    {
-#pragma clang fp contract(off)
-      x = ox[b] + ((double)(c >> 6) + 0.5) * d;
-      y = oy[b] + ((double)((c >> 3) & 7) + 0.5) * d;
-      z = oz[b] + ((double)(c & 7) + 0.5) * d;
-    }
-    const double e = eps ? eps[b] : 0.0;
     const double mi = m[i];
-    s4[i] = make_double4(x, y, z, mi);
-    se2[i] = e * e;
     sm[i] = mi;
-    const int ci = c >> 6, cj = (c >> 3) & 7, ck = c & 7;
-    if (cj == 0 && ck == 0) sax[b * 24 + ci] = x;
-    if (ci == 0 && ck == 0) sax[b * 24 + 8 + cj] = y;
-    if (ci == 0 && cj == 0) sax[b * 24 + 16 + ck] = z;
-    if (c == 0) be2[b] = e * e;
-    e2min = e2max = dbits(e * e);
-    rmax = dbits(max_abs3(x, y, z));
-    mmax = dbits(fabs(mi));
+    mmax = max(mmax, dbits(fabs(mi)));
+    if (check && !isfinite(mi)) bad = 1;
+    if (c < 24) {                 // the block's 24 axis values
+      const int axis = c >> 3, idx = c & 7;
+      const double d = dx[b], o = axis == 0 ? ox[b] : axis == 1 ? oy[b] : oz[b];
+      double v;
+      {
+#pragma clang fp contract(off)
+        v = o + ((double)idx + 0.5) * d;
+      }
+      sax[b * 24 + c] = v;
+      rmax = max(rmax, dbits(fabs(v)));
+      const double e = eps ? eps[b] : 0.0;
+      if (c == 0) be2[b] = e * e;
+      e2min = min(e2min, dbits(e * e));
+      e2max = max(e2max, dbits(e * e));
+      if (check && !finite5(o, d, e, 0.0, 0.0)) bad = 1;
+    }
   }
-  fold_source_stats(e2min, 0, rmax, e2max, mmax, stat);
+  publish_stats(e2min, rmax, e2max, mmax, bad, 0, P);
 }
 
-// Explicit sources that are 8^3 leaf blocks in C order (cell c = 64 i + 8 j + k of block b at
-// b * 512 + c): x depends on i only, y on j only, z on k only, and eps^2 is the block's.  Reads
-// the packed sources; writes the axis arrays sax, the block eps^2 and the contiguous cell masses
-// sm (as k_pack_source_blocks does), and clears flag[0] (set to 1 before) on any violation.  One
-// thread per source.
-__global__ void k_detect_source_blocks(int64_t nblk, const double4* __restrict__ s4,
-                                       const double* __restrict__ se2, double* __restrict__ sax,
-                                       double* __restrict__ be2, double* __restrict__ sm, int* flag) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+// The packed per-cell form of such a set ({x, y, z, m} and eps^2, 40 B per cell), for the kernels that
+// read sources one by one (block targets, the generic and periodic kernels).  One lane per cell.
+__global__ __launch_bounds__(256) void k_expand_source_blocks(int64_t nblk, const double* __restrict__ be2,
+                                                              const double* __restrict__ sax,
+                                                              const double* __restrict__ sm,
+                                                              double4* __restrict__ s4, double* __restrict__ se2) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= nblk * 512) return;
-  const int64_t b = i >> 9, base = b * 512;
+  const int64_t b = i >> 9;
   const int c = (int)(i & 511);
-  const int ci = c >> 6, cj = (c >> 3) & 7, ck = c & 7;
-  const double4 s = s4[i];
-  const bool ok = s.x == s4[base + ci * 64].x && s.y == s4[base + cj * 8].y &&
-                  s.z == s4[base + ck].z && se2[i] == se2[base];
-  if (!ok) flag[0] = 0;
-  sm[i] = s.w;
-  if (cj == 0 && ck == 0) sax[b * 24 + ci] = s.x;
-  if (ci == 0 && ck == 0) sax[b * 24 + 8 + cj] = s.y;
-  if (ci == 0 && cj == 0) sax[b * 24 + 16 + ck] = s.z;
-  if (c == 0) be2[b] = se2[i];
+  const double* a = sax + b * 24;
+  s4[i] = make_double4(a[c >> 6], a[8 + ((c >> 3) & 7)], a[16 + (c & 7)], sm[i]);
+  se2[i] = be2[b];
 }
 
 }  // namespace tg

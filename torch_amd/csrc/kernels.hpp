@@ -670,80 +670,189 @@ __device__ __forceinline__ void fold_source_stats(unsigned long long e2min, int 
   }
 }
 
-// Pack SoA FP64 sources into {x,y,z,m} + eps^2 and fold their statistics into stat (ST_*:
-// smallest and largest eps^2, largest |coordinate| and |m|).  With `check`, stat[ST_BAD]
-// becomes non-zero if any input is NaN/Inf.  stat must be reset first (k_reset_stats).
-// Workgroups of 256 lanes.
+// ---- one-pass reductions of an input set, read by the host ----
+// The pack and check kernels reduce their set's statistics (ST_*) and one violation bit over the whole
+// grid in the same launch: each workgroup writes its six words to its slot, takes a ticket, and the
+// last one reduces the slots, writes the results (device words for later kernels, pinned host words for
+// a caller that waits) and returns the ticket to 0.  No reset launch before it, no copy after it, and
+// no queue of atomics on five shared words, which took 75 of 85 us on a million cells.
+#define TG_PUB_WG 512            // most workgroups of such a launch (slots)
+struct Publish {
+  unsigned long long* slots;     // TG_PUB_WG x 8 words
+  unsigned int* ticket;          // 0 between launches
+  unsigned long long* stat;      // device result: ST_WORDS words (may be null)
+  int* flag;                     // device result: 1 if nothing was violated, else 0 (may be null)
+  unsigned long long* host;      // pinned result: ST_WORDS words, then the violation bit (may be null)
+  const unsigned long long* src_stat;   // non-null: host[8 ...] = these ST_WORDS words of the source set,
+  const int* src_flag;                  //   host[13] = *src_flag (null: 0)
+};
+
+// One lane's (e2min, rmax, e2max, mmax, bad | viol << 1) -> the workgroup's, in every lane.  256 lanes.
+__device__ __forceinline__ void wg_stats(unsigned long long (&v)[4], int& bits, unsigned long long (*sm)[5]) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    v[0] = min(v[0], shfl_xor_u64(v[0], off));
+#pragma unroll
+    for (int q = 1; q < 4; ++q) v[q] = max(v[q], shfl_xor_u64(v[q], off));
+    bits |= __shfl_xor(bits, off);
+  }
+  __syncthreads();               // an earlier use of sm is over
+  if ((threadIdx.x & 63) == 0) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) sm[threadIdx.x >> 6][q] = v[q];
+    sm[threadIdx.x >> 6][4] = (unsigned long long)bits;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    v[0] = min(v[0], sm[w][0]);
+#pragma unroll
+    for (int q = 1; q < 4; ++q) v[q] = max(v[q], sm[w][q]);
+    bits |= (int)sm[w][4];
+  }
+}
+
+// Every lane of every workgroup (256 lanes, at most TG_PUB_WG workgroups) calls it once, last.
+__device__ __forceinline__ void publish_stats(unsigned long long e2min, unsigned long long rmax,
+                                              unsigned long long e2max, unsigned long long mmax, int bad,
+                                              int viol, const Publish& P) {
+  __shared__ unsigned long long sm[4][5];
+  __shared__ int last;
+  unsigned long long v[4] = {e2min, rmax, e2max, mmax};
+  int bits = (bad ? 1 : 0) | (viol ? 2 : 0);
+  wg_stats(v, bits, sm);
+  if (gridDim.x > 1) {
+    if (threadIdx.x == 0) {
+      unsigned long long* s = P.slots + (size_t)blockIdx.x * 8;
+      // agent-scope stores go through to where every XCD sees them; the wait completes them before the
+      // ticket is taken, so whoever takes the last ticket reads every slot whole
+#pragma unroll
+      for (int q = 0; q < 4; ++q) __hip_atomic_store(s + q, v[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(s + 4, (unsigned long long)bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      last = __hip_atomic_fetch_add(P.ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+    }
+    __syncthreads();
+    if (!last) return;
+    asm volatile("" ::: "memory");
+    for (unsigned int b = threadIdx.x; b < gridDim.x; b += 256) {
+      unsigned long long* s = P.slots + (size_t)b * 8;
+      v[0] = min(v[0], __hip_atomic_load(s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+#pragma unroll
+      for (int q = 1; q < 4; ++q)
+        v[q] = max(v[q], __hip_atomic_load(s + q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+      bits |= (int)__hip_atomic_load(s + 4, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    wg_stats(v, bits, sm);
+    if (threadIdx.x == 0) __hip_atomic_store(P.ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  if (threadIdx.x != 0) return;
+  const unsigned long long st[ST_WORDS] = {v[0], (unsigned long long)(bits & 1), v[1], v[2], v[3]};
+  static_assert(ST_E2MIN == 0 && ST_BAD == 1 && ST_RMAX == 2 && ST_E2MAX == 3 && ST_MMAX == 4, "");
+#pragma unroll
+  for (int q = 0; q < ST_WORDS; ++q) {
+    if (P.stat) P.stat[q] = st[q];
+    if (P.host) P.host[q] = st[q];
+  }
+  if (P.flag) *P.flag = (bits & 2) ? 0 : 1;
+  if (P.host) {
+    P.host[ST_WORDS] = (unsigned long long)(bits >> 1);
+    if (P.src_stat) {
+#pragma unroll
+      for (int q = 0; q < ST_WORDS; ++q) P.host[8 + q] = P.src_stat[q];
+      P.host[8 + ST_WORDS] = P.src_flag ? (unsigned long long)*P.src_flag : 0ULL;
+    }
+    __threadfence_system();
+  }
+}
+
+__device__ __forceinline__ bool finite5(double a, double b, double c, double d, double e) {
+  return isfinite(a) && isfinite(b) && isfinite(c) && isfinite(d) && isfinite(e);
+}
+
+// Packs SoA FP64 sources into {x,y,z,m} + eps^2 with their statistics.  nb8 > 0 (n = 512 nb8): the
+// sources may be 8^3 leaf blocks in C order (cell c = 64 i + 8 j + k of block b at b * 512 + c): x
+// depends on i only, y on j only, z on k only, and eps^2 is the block's.  Each source is compared with
+// the first of its line (any difference is a violation: P.flag = 0), and the block-source form is
+// written too: the axes sax, the block eps^2 be2 and the contiguous cell masses sm.  With `check`, a
+// NaN/Inf input sets ST_BAD.
 __global__ __launch_bounds__(256) void k_pack_sources(int64_t n, const double* __restrict__ x,
                                                       const double* __restrict__ y,
                                                       const double* __restrict__ z,
                                                       const double* __restrict__ m,
                                                       const double* __restrict__ eps,
                                                       double4* __restrict__ s4,
-                                                      double* __restrict__ se2,
-                                                      unsigned long long* stat, int check) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+                                                      double* __restrict__ se2, int64_t nb8,
+                                                      double* __restrict__ sax, double* __restrict__ be2,
+                                                      double* __restrict__ sm, int check, Publish P) {
   unsigned long long e2min = 0x7ff0000000000000ULL, rmax = 0ULL, e2max = 0ULL, mmax = 0ULL;
-  int bad = 0;
-  if (i < n) {
+  int bad = 0, viol = 0;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
     const double4 v = make_double4(x[i], y[i], z[i], m[i]);
     const double e = eps ? eps[i] : 0.0;
     s4[i] = v;
     const double e2 = e * e;
     se2[i] = e2;
-    e2min = e2max = dbits(e2);
-    rmax = dbits(max_abs3(v.x, v.y, v.z));
-    mmax = dbits(fabs(v.w));
-    if (check)
-      bad = !(isfinite(v.x) && isfinite(v.y) && isfinite(v.z) && isfinite(v.w) && isfinite(e));
+    e2min = min(e2min, dbits(e2));
+    e2max = max(e2max, dbits(e2));
+    rmax = max(rmax, dbits(max_abs3(v.x, v.y, v.z)));
+    mmax = max(mmax, dbits(fabs(v.w)));
+    if (check && !finite5(v.x, v.y, v.z, v.w, e)) bad = 1;
+    if (nb8 > 0) {
+      const int64_t b = i >> 9, base = b * 512;
+      const int c = (int)(i & 511), ci = c >> 6, cj = (c >> 3) & 7, ck = c & 7;
+      const double eb = eps ? eps[base] : 0.0;
+      if (!(v.x == x[base + ci * 64] && v.y == y[base + cj * 8] && v.z == z[base + ck] && e2 == eb * eb)) viol = 1;
+      sm[i] = v.w;
+      if (cj == 0 && ck == 0) sax[b * 24 + ci] = v.x;
+      if (ci == 0 && ck == 0) sax[b * 24 + 8 + cj] = v.y;
+      if (ci == 0 && cj == 0) sax[b * 24 + 16 + ck] = v.z;
+      if (c == 0) be2[b] = e2;
+    }
   }
-  fold_source_stats(e2min, bad, rmax, e2max, mmax, stat);
+  publish_stats(e2min, rmax, e2max, mmax, bad, viol, P);
 }
 
-// Range statistics (ST_* words: largest |coordinate|, smallest / largest eps^2, largest |m|) of a
-// point set (x, y, z, eps per point; dx == null) or of a set of 8^3 blocks (x, y, z the lower
-// corners and dx the cell widths, so the centres lie within [x, x + 8 dx]; eps per block), with nm
-// masses m (may be null).  For the mixed mode's range check.  out is reset first (k_reset_stats);
-// workgroups of 256 lanes over max(n, nm).
-__global__ __launch_bounds__(256) void k_range(int64_t n, const double* __restrict__ x,
-                                               const double* __restrict__ y, const double* __restrict__ z,
-                                               const double* __restrict__ dx, const double* __restrict__ e,
-                                               int64_t nm, const double* __restrict__ m,
-                                               unsigned long long* out) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+// Column structure of explicit targets, the C order of 8^3 leaf blocks
+// (.deprecated/bridge_multiples.py:566-575 flattens each block's meshgrid this way): every
+// aligned group of 8 consecutive targets shares x and y, and every aligned group of 512 shares
+// eps.  One lane per target, compared with the first of its group (coalesced reads).
+__device__ __forceinline__ bool column_ok(const double* x, const double* y, const double* eps, int64_t t) {
+  const int64_t g = t & ~(int64_t)7;
+  bool ok = x[t] == x[g] && y[t] == y[g];
+  if (eps) ok = ok && eps[t] == eps[t & ~(int64_t)511];
+  return ok;
+}
+
+// Checks a point set (x, y, z, eps per point; dx == null) or a set of 8^3 blocks (x, y, z the lower
+// corners and dx the cell widths, so the centres lie within [x, x + 8 dx]; eps per block), with nm masses
+// m (may be null): NaN/Inf (ST_BAD), the range statistics (ST_*) and, with `cols`, the points' column
+// structure (a violation: not columns).
+__global__ __launch_bounds__(256) void k_check_set(int64_t n, const double* __restrict__ x,
+                                                   const double* __restrict__ y, const double* __restrict__ z,
+                                                   const double* __restrict__ dx, const double* __restrict__ e,
+                                                   int64_t nm, const double* __restrict__ m, int cols, Publish P) {
   unsigned long long e2min = 0x7ff0000000000000ULL, rmax = 0ULL, e2max = 0ULL, mmax = 0ULL;
-  if (i < n) {
-    double r = max_abs3(x[i], y[i], z[i]);
-    if (dx) r = fmax(r, max_abs3(x[i] + 8.0 * dx[i], y[i] + 8.0 * dx[i], z[i] + 8.0 * dx[i]));
-    const double ei = e ? e[i] : 0.0;
-    rmax = dbits(r);
-    e2min = e2max = dbits(ei * ei);
+  int bad = 0, viol = 0;
+  const int64_t most = m && nm > n ? nm : n;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < most; i += (int64_t)gridDim.x * 256) {
+    if (i < n) {
+      const double px = x[i], py = y[i], pz = z[i], ei = e ? e[i] : 0.0, d = dx ? dx[i] : 0.0;
+      double r = max_abs3(px, py, pz);
+      if (dx) r = fmax(r, max_abs3(px + 8.0 * d, py + 8.0 * d, pz + 8.0 * d));
+      rmax = max(rmax, dbits(r));
+      e2min = min(e2min, dbits(ei * ei));
+      e2max = max(e2max, dbits(ei * ei));
+      if (!finite5(px, py, pz, ei, d)) bad = 1;
+      if (cols && !column_ok(x, y, e, i)) viol = 1;
+    }
+    if (m && i < nm) {
+      const double mi = m[i];
+      mmax = max(mmax, dbits(fabs(mi)));
+      if (!isfinite(mi)) bad = 1;
+    }
   }
-  if (m && i < nm) mmax = dbits(fabs(m[i]));
-  fold_source_stats(e2min, 0, rmax, e2max, mmax, out);
-}
-
-__global__ void k_reset_stats(unsigned long long* stat) {
-  if (threadIdx.x == 0) {
-    stat[ST_E2MIN] = 0x7ff0000000000000ULL;
-    stat[ST_BAD] = 0ULL;
-    stat[ST_RMAX] = 0ULL;
-    stat[ST_E2MAX] = 0ULL;
-    stat[ST_MMAX] = 0ULL;
-  }
-}
-
-// NaN/Inf check of up to five target arrays (any may be null) into flag[0].
-__global__ void k_check_finite(int64_t n, const double* c0, const double* c1, const double* c2,
-                               const double* c3, const double* c4, unsigned long long* flag) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const double* cs[5] = {c0, c1, c2, c3, c4};
-  int bad = 0;
-#pragma unroll
-  for (int q = 0; q < 5; ++q)
-    if (cs[q] && !isfinite(cs[q][i])) bad = 1;
-  if (bad) atomicOr(flag, 1ULL);
+  publish_stats(e2min, rmax, e2max, mmax, bad, viol, P);
 }
 
 __global__ void k_kick(int64_t n, double dt, const double* __restrict__ ax,
@@ -764,30 +873,19 @@ __global__ void k_set_flag(int* flag, int v) {
   if (blockIdx.x == 0 && threadIdx.x == 0) flag[0] = v;
 }
 
-// Gate value of an explicit-target evaluation: 2 if the sources are explicit 8^3 blocks
-// (*sflag, set by k_detect_source_blocks; sflag null: they are not), else `tcand` (1: the targets
-// may have column structure, which k_check_cols then tests; 0: they do not).
+// Gate value of an explicit-target evaluation whose structure the host does not know: 2 if the sources
+// are explicit 8^3 blocks (*sflag, written when they were packed; sflag null: they are not), else
+// `tcand` (1: the targets may have column structure, which k_check_cols then tests; 0: they do not).
 __global__ void k_eval_gate(int* gate, const int* sflag, int tcand) {
   if (blockIdx.x == 0 && threadIdx.x == 0) gate[0] = (sflag && sflag[0] == 1) ? 2 : tcand;
 }
 
-// Column structure of explicit targets, the C order of 8^3 leaf blocks
-// (.deprecated/bridge_multiples.py:566-575 flattens each block's meshgrid this way): every
-// aligned group of 8 consecutive targets shares x and y, and every aligned group of 512 shares
-// eps.  One lane per target, compared with the first of its group (coalesced reads); any
-// violation clears flag[0] (1 before; 2, the block-source path, is left alone); all writers store
-// the same value.
-__device__ __forceinline__ bool column_ok(const Tgt& T, int64_t t) {
-  const int64_t g = t & ~(int64_t)7;
-  bool ok = T.x[t] == T.x[g] && T.y[t] == T.y[g];
-  if (T.eps) ok = ok && T.eps[t] == T.eps[t & ~(int64_t)511];
-  return ok;
-}
-
+// The column test for such an evaluation: any violation clears flag[0] (1 before; 2, the block-source
+// path, is left alone); all writers store the same value.
 __global__ void k_check_cols(Tgt T, int* flag) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= T.n || flag[0] != 1) return;   // 2: the block-source kernel runs; nothing to test
-  if (!column_ok(T, t)) flag[0] = 0;
+  if (!column_ok(T.x, T.y, T.eps, t)) flag[0] = 0;
 }
 
 __global__ void k_fill(int64_t n, double v, double* a, double* b, double* c, double* d) {

@@ -337,12 +337,15 @@ struct tgrav_ctx {
   DevBuf sbe2, sax, sms;     // source blocks: eps^2, cell-centre axes (24 per block), cell masses
   int64_t src_cols = 0;      // > 0: explicit sources that may be 8^3 blocks (scolflag says)
   DevBuf scolflag;
-  // staging for host pointers and scratch; flag[0] = NaN flag of the targets
-  DevBuf in[12], outb[8], vel[3], part, flag;
+  // Block sources: whether s4 / se2 hold the packed per-cell form of the current set, and whether any
+  // evaluation ever needed it (then every later set is expanded at once, so that a captured graph that
+  // reads it stays valid when the blocks are set again).
+  bool expanded = false, expand_used = false;
+  DevBuf pub;                // slots and ticket of the one-pass reductions (tg::Publish)
+  DevBuf in[12], outb[8], vel[3], part;      // staging for host pointers and scratch
   DevBuf colflag;            // explicit targets: 1 if they have 8^3 column structure
   DevBuf bp4, bpe2, bstat, bppart, bpgrp;   // fused passes: packed particles, partials
   DevBuf pm[16], pm_acc[3], pm_stat;  // particle-mesh pieces: staging, fixed-point sums, stat
-  DevBuf rstat;              // range statistics of the mixed mode's check (2 x tg::ST_WORDS)
   DevBuf pkey, pidx, ptmp, pbuf;   // periodic pairs: sort keys and indices (2 x each), sort scratch,
                                    //   per-pair image sums
   unsigned long long* host_flag = nullptr;   // pinned, kHostWords words
@@ -377,7 +380,9 @@ static int tuned_block_split(const tgrav_ctx* c, int mode, const char* dir, int6
 }
 
 static const int kTimingSlots = 256;
-static const int kHostWords = 16;   // pinned host words: flags and two sets of range statistics
+// Pinned host words: results of the one-pass reductions (tg::Publish::host), by use.
+static const int kHostWords = 32;
+enum { HW_EVAL = 0, HW_A = 16, HW_B = 24, HW_FLAG = 31 };
 
 template <class F>
 static int timed_launch_on(tgrav_ctx* c, hipStream_t s, int64_t nt, int64_t ns, F launch) {
@@ -461,14 +466,29 @@ static int reduce_chunks(tgrav_ctx* c, const double* part, int64_t pstride, int 
   return 0;
 }
 
-// Reads a device flag word written by k_pack_sources / k_check_finite (synchronous).
+// Reads a device flag word (synchronous).
 static int read_flag(tgrav_ctx* c, const void* dflag, bool* bad) {
-  HIPCHECK(hipMemcpyAsync(c->host_flag, dflag, sizeof(unsigned long long), hipMemcpyDeviceToHost,
+  HIPCHECK(hipMemcpyAsync(c->host_flag + HW_FLAG, dflag, sizeof(unsigned long long), hipMemcpyDeviceToHost,
                           c->stream));
   HIPCHECK(hipStreamSynchronize(c->stream));
-  *bad = *c->host_flag != 0ULL;
+  *bad = c->host_flag[HW_FLAG] != 0ULL;
   return 0;
 }
+
+// Where a one-pass reduction writes: device words (stat, flag; may be null) and, with hw >= 0, the
+// pinned host words from hw on.
+static tg::Publish publish_to(tgrav_ctx* c, unsigned long long* stat, int* flag, int hw) {
+  tg::Publish P{};
+  P.slots = c->pub.as<unsigned long long>();
+  P.ticket = (unsigned int*)(P.slots + (size_t)TG_PUB_WG * 8);
+  P.stat = stat;
+  P.flag = flag;
+  P.host = hw >= 0 ? c->host_flag + hw : nullptr;
+  return P;
+}
+static unsigned pub_grid(int64_t n) { return (unsigned)std::max<int64_t>(1, std::min<int64_t>(TG_PUB_WG, (n + 255) / 256)); }
+static bool host_bad(const tgrav_ctx* c, int hw) { return c->host_flag[hw + tg::ST_BAD] != 0ULL; }
+static const double* host_stats(const tgrav_ctx* c, int hw) { return reinterpret_cast<const double*>(c->host_flag + hw); }
 
 // ---- range of the mixed mode (only with validation on) ----
 // The mixed kernels hold displacements, r^2 and m / r^3 in FP32.  With S and T the statistics of
@@ -493,60 +513,49 @@ static int mixed_range_ok(const double* S, const double* T, const char* what) {
   return 0;
 }
 
-// Statistics (tg::ST_*) of a device point set (dx == null) or block set (x, y, z corners, dx cell
-// widths) with nm masses, into out[slot * ST_WORDS ...] of the pinned host words (synchronous).
-static int range_stats(tgrav_ctx* c, int slot, int64_t n, const double* x, const double* y,
-                       const double* z, const double* dx, const double* e, int64_t nm,
-                       const double* m) {
-  int rc = c->rstat.ensure(2 * tg::ST_WORDS * sizeof(unsigned long long));
-  if (rc) return rc;
-  unsigned long long* d = c->rstat.as<unsigned long long>() + slot * tg::ST_WORDS;
-  tg::k_reset_stats<<<1, 64, 0, c->stream>>>(d);
-  LAUNCHCHECK("k_reset_stats");
-  if (std::max(n, nm) > 0) {
-    tg::k_range<<<grid1(std::max(n, nm), 256), 256, 0, c->stream>>>(n, x, y, z, dx, e, nm, m, d);
-    LAUNCHCHECK("k_range");
-  }
-  HIPCHECK(hipMemcpyAsync(c->host_flag + slot * tg::ST_WORDS, d, tg::ST_WORDS * sizeof(unsigned long long),
-                          hipMemcpyDeviceToHost, c->stream));
+// What the host learned about an evaluation's inputs while it validated them: whether the explicit
+// targets are 8^3 columns and the explicit sources 8^3 blocks.  valid = false: not known (nothing was
+// waited for), the kernels are then gated on the device.
+struct Known {
+  bool valid = false, cols = false, srcb = false;
+};
+
+// One pass over the (device) targets of an evaluation and one wait: NaN/Inf, column structure and, mixed,
+// the range check against the source set.
+static int check_targets(tgrav_ctx* c, const tg::Tgt& T, int64_t nin, int mode, bool finite, Known* k) {
+  tg::Publish P = publish_to(c, nullptr, nullptr, HW_EVAL);
+  P.src_stat = c->ns > 0 ? c->stat.as<unsigned long long>() : nullptr;
+  P.src_flag = c->src_cols > 0 ? c->scolflag.as<int>() : nullptr;
+  if (T.blocks)
+    tg::k_check_set<<<pub_grid(nin), 256, 0, c->stream>>>(nin, T.ox, T.oy, T.oz, T.bdx, T.beps, 0, nullptr, 0, P);
+  else
+    tg::k_check_set<<<pub_grid(nin), 256, 0, c->stream>>>(nin, T.x, T.y, T.z, nullptr, T.eps, 0, nullptr, 1, P);
+  LAUNCHCHECK("k_check_set");
   HIPCHECK(hipStreamSynchronize(c->stream));
-  return 0;
-}
-
-static const double* host_stats(const tgrav_ctx* c, int slot) {
-  return reinterpret_cast<const double*>(c->host_flag + slot * tg::ST_WORDS);
-}
-
-// Mixed-mode range check of an evaluation: the current source set (its device statistics) against
-// targets given as points or blocks (device pointers).
-static int eval_range_check(tgrav_ctx* c, const tg::Tgt& T, int64_t nin) {
+  if (finite && host_bad(c, HW_EVAL)) return fail(TGRAV_ENONFINITE, "non-finite value in a target array");
   int rc;
-  if (T.blocks) rc = range_stats(c, 1, nin, T.ox, T.oy, T.oz, T.bdx, T.beps, 0, nullptr);
-  else rc = range_stats(c, 1, nin, T.x, T.y, T.z, nullptr, T.eps, 0, nullptr);
-  if (rc) return rc;
-  if (c->ns > 0) {
-    HIPCHECK(hipMemcpyAsync(c->host_flag, c->stat.p, tg::ST_WORDS * sizeof(unsigned long long),
-                            hipMemcpyDeviceToHost, c->stream));
-    HIPCHECK(hipStreamSynchronize(c->stream));
-    if ((rc = mixed_range_ok(host_stats(c, 0), host_stats(c, 1), "the sources and targets"))) return rc;
-  }
+  if (mode == TGRAV_MIXED && c->ns > 0 &&
+      (rc = mixed_range_ok(host_stats(c, HW_EVAL + 8), host_stats(c, HW_EVAL), "the sources and targets")))
+    return rc;
+  k->valid = true;
+  k->cols = !T.blocks && c->host_flag[HW_EVAL + tg::ST_WORDS] == 0ULL;
+  k->srcb = c->ns > 0 && c->host_flag[HW_EVAL + 8 + tg::ST_WORDS] == 1ULL;
   return 0;
 }
 
-// NaN/Inf check of device target arrays (synchronous; only with validation on).
-static int device_check_finite(tgrav_ctx* c, int64_t n, const double* const* chk, int nchk,
-                               bool* bad) {
-  *bad = false;
-  if (n <= 0) return 0;
-  int rc = c->flag.ensure(sizeof(unsigned long long));
-  if (rc) return rc;
-  const double* cs[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
-  for (int q = 0; q < nchk && q < 5; ++q) cs[q] = chk[q];
-  HIPCHECK(hipMemsetAsync(c->flag.p, 0, sizeof(unsigned long long), c->stream));
-  tg::k_check_finite<<<grid1(n, 256), 256, 0, c->stream>>>(n, cs[0], cs[1], cs[2], cs[3], cs[4],
-                                                          c->flag.as<unsigned long long>());
-  LAUNCHCHECK("k_check_finite");
-  return read_flag(c, c->flag.p, bad);
+// The packed per-cell form of block sources, for the kernels that read s4 / se2.
+static int expand_sources(tgrav_ctx* c) {
+  if (c->src_nblk == 0) return 0;
+  c->expand_used = true;
+  if (c->expanded) return 0;
+  tg::k_expand_source_blocks<<<grid1(c->src_nblk * 512, 256), 256, 0, c->stream>>>(
+      c->src_nblk, c->sbe2.as<double>(), c->sax.as<double>(), c->sms.as<double>(), c->s4.as<double4>(),
+      c->se2.as<double>());
+  LAUNCHCHECK("k_expand_source_blocks");
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  HIPCHECK(hipStreamIsCapturing(c->stream, &cap));
+  c->expanded = cap == hipStreamCaptureStatusNone;   // a captured launch has not run yet
+  return 0;
 }
 
 // Launch shape: the variant's target tile and a source split that gives about
@@ -853,7 +862,7 @@ static int launch_flash_pairs(tgrav_ctx* c, const tg::Tgt& T, const tg::Out& O, 
 // FLASH softening kernels (FP64 only).  Isolated: K = 2 targets per lane, sources split until
 // there are about 16 workgroups per CU (4 waves each, so the last round of workgroups is a
 // small share of the launch); periodic: K = 1 (hundreds of images per pair), about 8.
-static int launch_flash(tgrav_ctx* c, int mode, const tg::Tgt& T, const tg::Out& O) {
+static int launch_flash(tgrav_ctx* c, int mode, const tg::Tgt& T, const tg::Out& O, const Known& known) {
   if (mode != TGRAV_PLAIN_FP64)
     return fail(TGRAV_EINVAL, "the FLASH softening kernels run in TGRAV_PLAIN_FP64 only");
   const int64_t nt = T.n, ns = c->ns;
@@ -886,11 +895,11 @@ static int launch_flash(tgrav_ctx* c, int mode, const tg::Tgt& T, const tg::Out&
   // C-ordered 8^3 blocks (flagged on the device when they were set) launch it too, gated against
   // the generic kernel on that flag, as in the Plummer path.
   const bool isolated_blocks = !per && !T.blocks && c->block_kernel;
-  const bool srcb = isolated_blocks && c->src_nblk > 0;
-  const bool cand = isolated_blocks && !srcb && c->src_cols > 0;
+  const bool srcb = isolated_blocks && (c->src_nblk > 0 || (known.valid && known.srcb));
+  const bool cand = isolated_blocks && !srcb && c->src_cols > 0 && !known.valid;
   int64_t ntiles_s = 0, chunk_s = 0;
   int nsplit_s = 1;
-  const int64_t nblk_s = srcb ? c->src_nblk : c->src_cols;
+  const int64_t nblk_s = c->src_nblk > 0 ? c->src_nblk : c->src_cols;
   if (srcb || cand) flash_gridsrc_shape(c, nt, nblk_s, &ntiles_s, &nsplit_s, &chunk_s);
   if (ntiles_s > 0x7fffffffLL) return fail(TGRAV_ELIMIT, "too many targets (%lld)", (long long)nt);
   const int64_t ntiles = (nt + (int64_t)K * NT - 1) / ((int64_t)K * NT);
@@ -1002,7 +1011,7 @@ static const Variant* generic_variant(const tgrav_ctx* c, int mode, int64_t ns, 
   return v;
 }
 
-static int launch_eval(tgrav_ctx* c, int mode, const tg::Tgt& T, const tg::Out& O) {
+static int launch_eval(tgrav_ctx* c, int mode, const tg::Tgt& T, const tg::Out& O, const Known& known) {
   const int64_t nt = T.n, ns = c->ns;
   if (nt == 0) return 0;
   // Every pointer a kernel dereferences must be set before anything is launched.
@@ -1020,7 +1029,9 @@ static int launch_eval(tgrav_ctx* c, int mode, const tg::Tgt& T, const tg::Out& 
     LAUNCHCHECK("k_fill");
     return 0;
   }
-  if (c->soft != TGRAV_SOFT_PLUMMER) return launch_flash(c, mode, T, O);
+  int rcx;
+  if (!(c->block_kernel && !T.blocks && !c->periodic) && (rcx = expand_sources(c))) return rcx;
+  if (c->soft != TGRAV_SOFT_PLUMMER) return launch_flash(c, mode, T, O, known);
   if (T.blocks && T.nb == 8 && c->block_kernel) return launch_grid(c, mode, T, O);
   if (!T.blocks && c->src_nblk > 0 && c->block_kernel) return launch_gridsrc(c, mode, T, O);
   int force_split = -1;
@@ -1037,8 +1048,15 @@ static int launch_eval(tgrav_ctx* c, int mode, const tg::Tgt& T, const tg::Out& 
   // Likewise explicit sources that are C-ordered 8^3 blocks (k_detect_source_blocks flagged
   // them when they were set) run the block-source kernel: gate value 2 wins over the column
   // test (1) and the generic kernel (0).
-  const bool cols = c->block_kernel && !T.blocks && nt >= 512;
-  const bool srcb = c->block_kernel && !T.blocks && c->src_cols > 0;
+  // An evaluation that validated its inputs knows both answers already (Known) and launches the one
+  // kernel, ungated.
+  bool cols = c->block_kernel && !T.blocks && nt >= 512;
+  bool srcb = c->block_kernel && !T.blocks && c->src_cols > 0;
+  if (known.valid) {
+    srcb = srcb && known.srcb;
+    cols = cols && !srcb && known.cols;
+  }
+  const bool generic = !known.valid || !(srcb || cols);
   const int64_t ngrp = (nt + 511) / 512;
   int nsplit_c = 1, nsplit_s = 1;
   int64_t chunk_c = 0, chunk_s = 0, ntiles_s = 0;
@@ -1047,6 +1065,7 @@ static int launch_eval(tgrav_ctx* c, int mode, const tg::Tgt& T, const tg::Out& 
     grid_shape(c, mode, ns, ngrp, &nsplit_c, &chunk_c);
   }
   if (srcb) gridsrc_shape(c, mode, nt, c->src_cols, &ntiles_s, &nsplit_s, &chunk_s);
+  if (!generic) nsplit = 1;
   const int nsp = std::max(nsplit, std::max(cols ? nsplit_c : 1, srcb ? nsplit_s : 1));
   if (nsp > 1) {
     int rc0 = c->part.ensure((size_t)nsp * 4 * nt * sizeof(double));
@@ -1057,7 +1076,7 @@ static int launch_eval(tgrav_ctx* c, int mode, const tg::Tgt& T, const tg::Out& 
   oc.part = nsplit_c > 1 ? c->part.as<double>() : nullptr;
   os.part = nsplit_s > 1 ? c->part.as<double>() : nullptr;
   o.pstride = oc.pstride = os.pstride = nt;
-  if (cols || srcb) {
+  if (!known.valid && (cols || srcb)) {
     int rc0 = c->colflag.ensure(sizeof(int));
     if (rc0) return rc0;
     int* flag = c->colflag.as<int>();
@@ -1082,6 +1101,7 @@ static int launch_eval(tgrav_ctx* c, int mode, const tg::Tgt& T, const tg::Out& 
       int r = column_kernel(c, mode, false, ngrp, nsplit_c, T, ns, chunk_c, oc);
       if (r) return r;
     }
+    if (!generic) return 0;
     v->fn(dim3((unsigned)ntiles, (unsigned)nsplit), dim3(v->nt), c->stream, T, c->s4.as<double4>(),
           c->se2.as<double>(), ns, chunk, c->stat.as<const double>(), o);
     LAUNCHCHECK(mode == TGRAV_MIXED ? "k_eval_mixed" : "k_eval_fp64");
@@ -1160,8 +1180,11 @@ int tgrav_create(tgrav_ctx** out, int device, const char* tune_cache_path) {
     delete c;
     return fail(TGRAV_EHIP, "tgrav_create: %s", hipGetErrorString(e));
   }
-  const int rs = scratch_init(device);
+  int rs = scratch_init(device);
+  if (!rs) rs = c->pub.ensure((size_t)TG_PUB_WG * 64 + 64);
+  if (!rs && hipMemset(c->pub.p, 0, c->pub.cap) != hipSuccess) rs = fail(TGRAV_EHIP, "tgrav_create: hipMemset failed");
   if (rs) {
+    c->pub.release();
     (void)hipHostFree(c->host_flag);
     (void)hipStreamDestroy(c->own);
     delete c;
@@ -1184,8 +1207,7 @@ int tgrav_destroy(tgrav_ctx* c) {
   for (auto& b : c->vel) b.release();
   c->part.release();
   c->stat.release();
-  c->rstat.release();
-  c->flag.release();
+  c->pub.release();
   c->colflag.release();
   c->sbe2.release();
   c->sms.release();
@@ -1300,36 +1322,27 @@ int tgrav_set_sources(tgrav_ctx* c, int64_t n, const double* x, const double* y,
         if (!host_finite(n, a[q])) return fail(TGRAV_ENONFINITE, "non-finite value in source array %d", q);
     if ((rc = stage_in(c, 0, n, a, 5))) return rc;
   }
-  tg::k_reset_stats<<<1, 64, 0, c->stream>>>(c->stat.as<unsigned long long>());
-  LAUNCHCHECK("k_reset_stats");
-  tg::k_pack_sources<<<grid1(n, 256), 256, 0, c->stream>>>(
-      n, a[0], a[1], a[2], a[3], a[4], c->s4.as<double4>(), c->se2.as<double>(),
-      c->stat.as<unsigned long long>(), kind == TGRAV_DEVICE && c->validate);
+  const int64_t nb8 = n % 512 == 0 ? n / 512 : 0;   // > 0: perhaps C-ordered 8^3 blocks
+  if (nb8 > 0 && ((rc = c->sax.ensure((size_t)nb8 * 24 * sizeof(double))) ||
+                  (rc = c->sbe2.ensure((size_t)nb8 * sizeof(double))) || (rc = c->sms.ensure((size_t)n * 8)) ||
+                  (rc = c->scolflag.ensure(sizeof(int)))))
+    return rc;
+  const bool wait = kind == TGRAV_DEVICE && c->validate;
+  tg::k_pack_sources<<<pub_grid(n), 256, 0, c->stream>>>(
+      n, a[0], a[1], a[2], a[3], a[4], c->s4.as<double4>(), c->se2.as<double>(), nb8, c->sax.as<double>(),
+      c->sbe2.as<double>(), c->sms.as<double>(), wait,
+      publish_to(c, c->stat.as<unsigned long long>(), nb8 > 0 ? c->scolflag.as<int>() : nullptr, wait ? HW_A : -1));
   LAUNCHCHECK("k_pack_sources");
-  const int64_t nb8 = n / 512;
-  if (n % 512 == 0) {   // C-ordered 8^3 blocks? decided on the device (k_detect_source_blocks)
-    if ((rc = c->sax.ensure((size_t)nb8 * 24 * sizeof(double))) ||
-        (rc = c->sbe2.ensure((size_t)nb8 * sizeof(double))) || (rc = c->sms.ensure((size_t)n * 8)) ||
-        (rc = c->scolflag.ensure(sizeof(int))))
-      return rc;
-    tg::k_set_flag<<<1, 64, 0, c->stream>>>(c->scolflag.as<int>(), 1);
-    LAUNCHCHECK("k_set_flag");
-    tg::k_detect_source_blocks<<<grid1(n, 256), 256, 0, c->stream>>>(
-        nb8, c->s4.as<double4>(), c->se2.as<double>(), c->sax.as<double>(), c->sbe2.as<double>(),
-        c->sms.as<double>(), c->scolflag.as<int>());
-    LAUNCHCHECK("k_detect_source_blocks");
-  }
   if (kind == TGRAV_DEVICE) {
-    if (c->validate) {
-      bool bad = false;
-      if ((rc = read_flag(c, c->stat.as<unsigned long long>() + tg::ST_BAD, &bad))) return rc;
-      if (bad) return fail(TGRAV_ENONFINITE, "non-finite value in a source array");
+    if (wait) {
+      HIPCHECK(hipStreamSynchronize(c->stream));
+      if (host_bad(c, HW_A)) return fail(TGRAV_ENONFINITE, "non-finite value in a source array");
     }
   } else {
     HIPCHECK(hipStreamSynchronize(c->stream));   // host arrays may be freed on return
   }
   c->ns = n;
-  c->src_cols = n % 512 == 0 ? nb8 : 0;
+  c->src_cols = nb8;
   return 0;
 }
 
@@ -1376,27 +1389,23 @@ int tgrav_set_source_blocks(tgrav_ctx* c, int64_t nblk, int nb, const double* ox
       if (!host_finite(n, m)) return fail(TGRAV_ENONFINITE, "non-finite cell mass");
     }
     if ((rc = stage_in(c, 0, nblk, a, 5)) || (rc = stage_in(c, 5, n, a + 5, 1))) return rc;
-  } else if (c->validate) {
-    bool bad = false;
-    if ((rc = device_check_finite(c, nblk, a, 5, &bad))) return rc;
-    if (!bad && (rc = device_check_finite(c, n, a + 5, 1, &bad))) return rc;
-    if (bad) return fail(TGRAV_ENONFINITE, "non-finite value in a source block array");
   }
   if ((rc = c->s4.ensure((size_t)n * sizeof(double4))) || (rc = c->se2.ensure((size_t)n * 8)) ||
       (rc = c->stat.ensure(tg::ST_WORDS * sizeof(unsigned long long))) ||
       (rc = c->sbe2.ensure((size_t)nblk * 8)) || (rc = c->sms.ensure((size_t)n * 8)) ||
       (rc = c->sax.ensure((size_t)nblk * 24 * sizeof(double))))
     return rc;
-  tg::k_reset_stats<<<1, 64, 0, c->stream>>>(c->stat.as<unsigned long long>());
-  LAUNCHCHECK("k_reset_stats");
-  tg::k_pack_source_blocks<<<grid1(n, 256), 256, 0, c->stream>>>(
-      nblk, a[0], a[1], a[2], a[3], a[5], a[4], c->s4.as<double4>(), c->se2.as<double>(),
-      c->sbe2.as<double>(), c->sax.as<double>(), c->sms.as<double>(), c->stat.as<unsigned long long>());
+  const bool wait = kind == TGRAV_DEVICE && c->validate;
+  tg::k_pack_source_blocks<<<pub_grid(n), 256, 0, c->stream>>>(
+      nblk, a[0], a[1], a[2], a[3], a[5], a[4], c->sbe2.as<double>(), c->sax.as<double>(), c->sms.as<double>(), wait,
+      publish_to(c, c->stat.as<unsigned long long>(), nullptr, wait ? HW_A : -1));
   LAUNCHCHECK("k_pack_source_blocks");
-  if (kind == TGRAV_HOST) HIPCHECK(hipStreamSynchronize(c->stream));
+  if (kind == TGRAV_HOST || wait) HIPCHECK(hipStreamSynchronize(c->stream));
+  if (wait && host_bad(c, HW_A)) return fail(TGRAV_ENONFINITE, "non-finite value in a source block array");
   c->ns = n;
   c->src_nblk = nblk;
-  return 0;
+  c->expanded = false;
+  return c->expand_used ? expand_sources(c) : 0;
 }
 
 // Shared body of tgrav_eval / tgrav_eval_kick / tgrav_eval_blocks.
@@ -1413,7 +1422,8 @@ static int eval_common(tgrav_ctx* c, tg::Tgt T, const double* tin[5], int ntin, 
           return fail(TGRAV_ENONFINITE, "non-finite value in target array %d", q);
     if ((rc = stage_in(c, 0, nin, tin, ntin))) return rc;
     bind_targets(T, tin, ntin);
-    if (mode == TGRAV_MIXED && c->validate && (rc = eval_range_check(c, T, nin))) return rc;
+    Known known;
+    if (mode == TGRAV_MIXED && c->validate && (rc = check_targets(c, T, nin, mode, false, &known))) return rc;
     double* dout[4] = {nullptr, nullptr, nullptr, nullptr};
     for (int q = 0; q < 4; ++q)
       if (outs[q]) {
@@ -1430,7 +1440,7 @@ static int eval_common(tgrav_ctx* c, tg::Tgt T, const double* tin[5], int ntin, 
     tg::Out O{dout[0], dout[1], dout[2], dout[3], dvel[0], dvel[1], dvel[2], dt, nullptr, 0, c->G,
               outs[3] == nullptr};
     O.noacc = potential_only(O);
-    if ((rc = launch_eval(c, mode, T, O))) return rc;
+    if ((rc = launch_eval(c, mode, T, O, known))) return rc;
     for (int q = 0; q < 4; ++q)
       if (outs[q])
         HIPCHECK(hipMemcpyAsync(outs[q], dout[q], (size_t)n * 8, hipMemcpyDeviceToHost, c->stream));
@@ -1440,17 +1450,13 @@ static int eval_common(tgrav_ctx* c, tg::Tgt T, const double* tin[5], int ntin, 
     HIPCHECK(hipStreamSynchronize(c->stream));
     return 0;
   }
-  if (c->validate && ntin > 0) {
-    bool bad = false;
-    if ((rc = device_check_finite(c, nin, tin, ntin, &bad))) return rc;
-    if (bad) return fail(TGRAV_ENONFINITE, "non-finite value in a target array");
-  }
   bind_targets(T, tin, ntin);
-  if (mode == TGRAV_MIXED && c->validate && (rc = eval_range_check(c, T, nin))) return rc;
+  Known known;
+  if (c->validate && ntin > 0 && (rc = check_targets(c, T, nin, mode, true, &known))) return rc;
   tg::Out O{outs[0], outs[1], outs[2], outs[3], vel[0], vel[1], vel[2], dt, nullptr, 0, c->G,
             outs[3] == nullptr};
   O.noacc = potential_only(O);
-  return launch_eval(c, mode, T, O);
+  return launch_eval(c, mode, T, O, known);
 }
 
 static int eval_prologue(tgrav_ctx* c, int64_t n, int mode, int kind) {
@@ -1571,9 +1577,8 @@ int tgrav_eval_static(tgrav_ctx* c, int64_t ns, const double* sx, const double* 
   tg::Out o = O;
   o.part = nsplit > 1 ? part : nullptr;
   o.pstride = nt;
-  tg::k_reset_stats<<<1, 64, 0, c->stream>>>(stat);
-  LAUNCHCHECK("k_reset_stats");
-  tg::k_pack_sources<<<grid1(ns, 256), 256, 0, c->stream>>>(ns, sx, sy, sz, sm, se, s4, se2, stat, 0);
+  tg::k_pack_sources<<<pub_grid(ns), 256, 0, c->stream>>>(ns, sx, sy, sz, sm, se, s4, se2, 0, nullptr, nullptr,
+                                                          nullptr, 0, publish_to(c, stat, nullptr, -1));
   LAUNCHCHECK("k_pack_sources");
   v->fn(dim3((unsigned)ntiles, (unsigned)nsplit), dim3(v->nt), c->stream, T, s4, se2, ns, chunk,
         (const double*)stat, o);
@@ -1633,20 +1638,45 @@ int tgrav_bidir_variant_info(int mode, int variant, int* k, int* threads) {
   return 0;
 }
 
-// Fused passes: packs the particles (x, y, z, m, eps) into c->bp4 / c->bpe2 and their smallest
-// eps^2 into c->bstat.
-static int bidir_pack_particles(tgrav_ctx* c, int64_t np, const double* const* pa) {
+// Fused passes: packs the particles (x, y, z, m, eps) into c->bp4 / c->bpe2 with their statistics in
+// c->bstat (and, with hw >= 0, in the pinned host words, inputs checked for NaN/Inf).
+static int bidir_pack_particles(tgrav_ctx* c, int64_t np, const double* const* pa, int hw) {
   int rc;
   if ((rc = c->bp4.ensure((size_t)np * sizeof(double4))) ||
       (rc = c->bpe2.ensure((size_t)np * sizeof(double))) ||
       (rc = c->bstat.ensure(tg::ST_WORDS * sizeof(unsigned long long))))
     return rc;
-  tg::k_reset_stats<<<1, 64, 0, c->stream>>>(c->bstat.as<unsigned long long>());
-  LAUNCHCHECK("k_reset_stats");
-  tg::k_pack_sources<<<grid1(np, 256), 256, 0, c->stream>>>(
-      np, pa[0], pa[1], pa[2], pa[3], pa[4], c->bp4.as<double4>(), c->bpe2.as<double>(),
-      c->bstat.as<unsigned long long>(), 0);
+  tg::k_pack_sources<<<pub_grid(np), 256, 0, c->stream>>>(
+      np, pa[0], pa[1], pa[2], pa[3], pa[4], c->bp4.as<double4>(), c->bpe2.as<double>(), 0, nullptr, nullptr, nullptr,
+      hw >= 0, publish_to(c, c->bstat.as<unsigned long long>(), nullptr, hw));
   LAUNCHCHECK("k_pack_sources");
+  return 0;
+}
+
+// Packs the particles of a fused pass and, where its inputs are validated (device arrays; mixed: their
+// range too), checks the cells (dx == null: points; else blocks) in the same wait.  *cols: 1 / 0 whether
+// explicit cells are 8^3 columns, left alone (-1) when nothing was waited for.
+static int bidir_inputs(tgrav_ctx* c, int mode, int kind, int64_t n, const double* x, const double* y,
+                        const double* z, const double* dx, const double* e, int64_t nm, const double* m,
+                        int64_t np, const double* const* pa, int* cols) {
+  const bool finite = kind == TGRAV_DEVICE && c->validate;
+  const bool range = mode == TGRAV_MIXED && c->validate && n > 0 && np > 0;
+  const bool wait = finite || range;
+  int rc;
+  if (wait && n > 0) {
+    tg::k_check_set<<<pub_grid(std::max(n, nm)), 256, 0, c->stream>>>(n, x, y, z, dx, e, nm, m, dx ? 0 : 1,
+                                                                     publish_to(c, nullptr, nullptr, HW_A));
+    LAUNCHCHECK("k_check_set");
+  }
+  if (np > 0 && (rc = bidir_pack_particles(c, np, pa, wait ? HW_B : -1))) return rc;
+  if (!wait) return 0;
+  HIPCHECK(hipStreamSynchronize(c->stream));
+  if (finite && ((n > 0 && host_bad(c, HW_A)) || (np > 0 && host_bad(c, HW_B))))
+    return fail(TGRAV_ENONFINITE, "non-finite value in an input array");
+  if (range && ((rc = mixed_range_ok(host_stats(c, HW_A), host_stats(c, HW_B), "the cells and particles")) ||
+                (rc = mixed_range_ok(host_stats(c, HW_B), host_stats(c, HW_A), "the particles and cells"))))
+    return rc;
+  if (n > 0 && !dx) *cols = c->host_flag[HW_A + tg::ST_WORDS] == 0ULL ? 1 : 0;
   return 0;
 }
 
@@ -1686,10 +1716,9 @@ static void bidir_grid_kernel(tgrav_ctx* c, int mode, const tg::CellBlocks& C, i
 
 // The fused pass with the cells as 8^3 block descriptors (k_bidir_grid).
 static int bidir_grid_pass(tgrav_ctx* c, int mode, const tg::CellBlocks& C, int64_t np,
-                           const double* const* pa, const tg::Out& CO, const tg::Out& PO) {
+                           const tg::Out& CO, const tg::Out& PO) {
   int rc;
   const int64_t nblk = C.nblk, nc = nblk * 512;
-  if ((rc = bidir_pack_particles(c, np, pa))) return rc;
   int64_t chunk;
   int nsplit;
   if ((rc = bidir_grid_shape(c, mode, nblk, np, &chunk, &nsplit))) return rc;
@@ -1746,19 +1775,10 @@ int tgrav_bidirectional(tgrav_ctx* c, int64_t nc, const double* cx, const double
         if ((rc = c->outb[4 + q].ensure((size_t)std::max<int64_t>(np, 1) * 8))) return rc;
       }
     }
-  } else if (c->validate) {
-    bool bad = false;
-    if ((rc = device_check_finite(c, nc, ca, 5, &bad))) return rc;
-    if (!bad && (rc = device_check_finite(c, np, pa, 5, &bad))) return rc;
-    if (bad) return fail(TGRAV_ENONFINITE, "non-finite value in an input array");
   }
-  if (mode == TGRAV_MIXED && c->validate && nc > 0 && np > 0) {
-    if ((rc = range_stats(c, 0, nc, ca[0], ca[1], ca[2], nullptr, ca[4], nc, ca[3])) ||
-        (rc = range_stats(c, 1, np, pa[0], pa[1], pa[2], nullptr, pa[4], np, pa[3])) ||
-        (rc = mixed_range_ok(host_stats(c, 0), host_stats(c, 1), "the cells and particles")) ||
-        (rc = mixed_range_ok(host_stats(c, 1), host_stats(c, 0), "the particles and cells")))
-      return rc;
-  }
+  int known_cols = -1;
+  if ((rc = bidir_inputs(c, mode, kind, nc, ca[0], ca[1], ca[2], nullptr, ca[4], nc, ca[3], np, pa, &known_cols)))
+    return rc;
   double* dco[4];
   double* dpo[4];
   for (int q = 0; q < 4; ++q) {
@@ -1776,11 +1796,11 @@ int tgrav_bidirectional(tgrav_ctx* c, int64_t nc, const double* cx, const double
     LAUNCHCHECK("k_fill");
   }
   if (nc > 0 && np > 0) {
-    if ((rc = bidir_pack_particles(c, np, pa))) return rc;
     // Cells in the C order of 8^3 leaf-block meshgrids take the block-column kernel.  Whether
     // they are is tested on the device (k_check_cols writes a gate word: 1 columns, 0 not); both
-    // kernels and their reductions are launched, and the word lets one of them run.
-    bool cand = nc % 512 == 0 && c->block_kernel;
+    // kernels and their reductions are launched, and the word lets one of them run -- unless the
+    // inputs were validated, which answers it before the launch.
+    bool cand = nc % 512 == 0 && c->block_kernel && known_cols != 0;
     const BiVariant& v = kBiVariants[mode][c->bvariant[mode]];
     const int64_t tile = (int64_t)v.k * v.nt;
     const int64_t ntiles = (nc + tile - 1) / tile;
@@ -1815,13 +1835,14 @@ int tgrav_bidirectional(tgrav_ctx* c, int64_t nc, const double* cx, const double
     const int nsp = std::max(nsplit, cand ? nsplit_g : 1);
     if (nsp > 1 && (rc = c->part.ensure((size_t)nsp * 4 * nc * sizeof(double)))) return rc;
     tg::Out CG = CO, PG = PO, CX = CO, PX = PO;   // column pipeline (G), generic pipeline (X)
-    if (cand) {
+    const bool both = cand && known_cols < 0, generic = !cand || both;
+    if (both) {
       if ((rc = c->colflag.ensure(sizeof(int)))) return rc;
       int* fl = c->colflag.as<int>();
       tg::Tgt T{};
       T.x = ca[0]; T.y = ca[1]; T.z = ca[2]; T.eps = ca[4]; T.n = nc;
-      tg::k_set_flag<<<1, 64, 0, c->stream>>>(fl, 1);
-      LAUNCHCHECK("k_set_flag");
+      tg::k_eval_gate<<<1, 64, 0, c->stream>>>(fl, nullptr, 1);
+      LAUNCHCHECK("k_eval_gate");
       tg::k_check_cols<<<grid1(nc, 256), 256, 0, c->stream>>>(T, fl);
       LAUNCHCHECK("k_check_cols");
       CG.gate = PG.gate = CX.gate = PX.gate = fl;
@@ -1839,6 +1860,7 @@ int tgrav_bidirectional(tgrav_ctx* c, int64_t nc, const double* cx, const double
         bidir_grid_kernel(c, mode, CB, np, chunk_g, nsplit_g, og);
         LAUNCHCHECK("k_bidir_grid");
       }
+      if (!generic) return 0;
       v.fn(dim3((unsigned)ntiles, (unsigned)nsplit), dim3(v.nt), c->stream, C, c->bp4.as<double4>(),
            c->bpe2.as<double>(), np, chunk, c->bstat.as<const double>(), ox, c->bppart.as<double>());
       LAUNCHCHECK("k_bidir");
@@ -1849,8 +1871,10 @@ int tgrav_bidirectional(tgrav_ctx* c, int64_t nc, const double* cx, const double
       if (nsplit_g > 1 && (rc = reduce_chunks(c, c->part.as<double>(), nc, nsplit_g, nc, CG))) return rc;
       if ((rc = reduce_particle_partials(c, nblk, np, PG))) return rc;
     }
-    if (nsplit > 1 && (rc = reduce_chunks(c, c->part.as<double>(), nc, nsplit, nc, CX))) return rc;
-    if ((rc = reduce_particle_partials(c, ntiles, np, PX))) return rc;
+    if (generic) {
+      if (nsplit > 1 && (rc = reduce_chunks(c, c->part.as<double>(), nc, nsplit, nc, CX))) return rc;
+      if ((rc = reduce_particle_partials(c, ntiles, np, PX))) return rc;
+    }
   }
   if (kind == TGRAV_HOST) {
     for (int q = 0; q < 4; ++q) {
@@ -1905,21 +1929,10 @@ int tgrav_bidirectional_blocks(tgrav_ctx* c, int64_t nblk, int nb, const double*
       if (co[q] && (rc = c->outb[q].ensure((size_t)std::max<int64_t>(nc, 1) * 8))) return rc;
       if (po[q] && (rc = c->outb[4 + q].ensure((size_t)std::max<int64_t>(np, 1) * 8))) return rc;
     }
-  } else if (c->validate) {
-    bool bad = false;
-    if ((rc = device_check_finite(c, nblk, ba, 4, &bad))) return rc;
-    if (!bad && (rc = device_check_finite(c, nc, mc, 1, &bad))) return rc;
-    if (!bad && (rc = device_check_finite(c, nblk, be, 1, &bad))) return rc;
-    if (!bad && (rc = device_check_finite(c, np, pa, 5, &bad))) return rc;
-    if (bad) return fail(TGRAV_ENONFINITE, "non-finite value in an input array");
   }
-  if (mode == TGRAV_MIXED && c->validate && nc > 0 && np > 0) {
-    if ((rc = range_stats(c, 0, nblk, ba[0], ba[1], ba[2], ba[3], be[0], nc, mc[0])) ||
-        (rc = range_stats(c, 1, np, pa[0], pa[1], pa[2], nullptr, pa[4], np, pa[3])) ||
-        (rc = mixed_range_ok(host_stats(c, 0), host_stats(c, 1), "the cells and particles")) ||
-        (rc = mixed_range_ok(host_stats(c, 1), host_stats(c, 0), "the particles and cells")))
-      return rc;
-  }
+  int no_cols = -1;
+  if ((rc = bidir_inputs(c, mode, kind, nblk, ba[0], ba[1], ba[2], ba[3], be[0], nc, mc[0], np, pa, &no_cols)))
+    return rc;
   double* dco[4];
   double* dpo[4];
   for (int q = 0; q < 4; ++q) {
@@ -1938,7 +1951,7 @@ int tgrav_bidirectional_blocks(tgrav_ctx* c, int64_t nblk, int nb, const double*
   }
   if (nc > 0 && np > 0) {
     tg::CellBlocks C{ba[0], ba[1], ba[2], ba[3], mc[0], be[0], nblk, nullptr, nullptr, nullptr, nullptr};
-    if ((rc = bidir_grid_pass(c, mode, C, np, pa, CO, PO))) return rc;
+    if ((rc = bidir_grid_pass(c, mode, C, np, CO, PO))) return rc;
   }
   if (kind == TGRAV_HOST) {
     for (int q = 0; q < 4; ++q) {
