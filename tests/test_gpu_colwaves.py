@@ -207,3 +207,40 @@ def test_column_waves_argument_errors():
             with pytest.raises(TgravError):
                 f.set_column_waves(bad)
         assert f.column_waves() == 4           # the default
+
+
+@pytest.mark.parametrize("mode", ["fp64", "mixed"])
+@pytest.mark.parametrize("ns", [1, 63, 64, 65, 255, 256, 257, 1000])
+def test_thin_launches_give_the_column_kernels_bits(mode, ns):
+    """Launches too small to fill the chip take one target per lane (k_eval_thin): block targets, the
+    same targets as explicit centres and a plan (which keeps the column code) agree bit for bit, with
+    softened and unsoftened sources (coincident pairs among them), and so do the potential and the
+    acceleration asked for alone."""
+    import torch
+    from torch_amd.blocks import block_centres
+    d = lambda a: torch.as_tensor(np.ascontiguousarray(a), device="cuda")  # noqa: E731
+    rng = W.rng_for(1300 + ns)
+    nblk = 3
+    o, w = rng.uniform(-1, 1, (nblk, 3)), rng.uniform(0.01, 0.1, nblk)
+    cx, cy, cz, _ = block_centres(o, w)
+    pos = rng.uniform(-1, 1, (3, ns))
+    k = min(ns, 5)
+    pos[:, :k] = np.stack([cx[:k * 100:100], cy[:k * 100:100], cz[:k * 100:100]])
+    for eps in (None, np.full(ns, 0.01)):
+        s = [d(a) for a in pos] + [d(rng.uniform(0.1, 1, ns)), None if eps is None else d(eps)]
+        with StellarGravityField(mode) as f:
+            f.set_config(nsplit=1)
+            f.set_stars(*s)
+            a = f.evaluate_blocks(d(o), d(w))
+            b = f.evaluate(None, d(cx), d(cy), d(cz))
+            src = dict(x=s[0], y=s[1], z=s[2], m=s[3])
+            if eps is not None:
+                src["eps"] = s[4]
+            plan = BatchPlan(f, [dict(sources=src, targets=dict(block_origin=d(o), block_dx=d(w)))])
+            c = plan.run()[0]
+            phi = f.get_potential_at_point(None, d(cx), d(cy), d(cz))
+            acc = f.get_gravity_at_point(None, d(cx), d(cy), d(cz))
+            for q in range(4):
+                assert torch.equal(a[q], b[q]) and torch.equal(a[q], c[q])
+                assert torch.equal(a[q], phi if q == 3 else acc[q])
+            assert torch.isfinite(a[3]).all()

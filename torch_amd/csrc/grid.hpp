@@ -493,6 +493,137 @@ __global__ __launch_bounds__(64 * W, MIXED ? 3 : 1) void k_eval_cols(Tgt T, cons
   cols_group<MIXED, W>(L, T, blockIdx.x, src4, srce2, sb, se, sst, o);
 }
 
+// ---------------------------------------------------------------- thin columns ----
+// The column code for launches too small to fill the chip: one target per lane instead of 8, so a
+// group of 512 targets is 8 workgroups and a wave's pass over its 64 sources an eighth as long.  Same
+// partition of the sources, same operations per pair and same order of sums as k_eval_grid / k_eval_cols,
+// hence the same bits.
+template <bool MIXED, int W>
+struct LdsThin {
+  typedef typename std::conditional<MIXED, float, double>::type T;
+  union {
+    struct {
+      typename std::conditional<MIXED, float4, double4>::type s4[64 * W];
+      T se2[64 * W];
+    };
+    double red[W > 1 ? 4 * 64 : 1];
+  };
+};
+
+template <bool MIXED, int W>
+struct ThinRun {
+  typedef typename LdsThin<MIXED, W>::T T;
+  template <int FL>
+  static __device__ __forceinline__ void run(LdsThin<MIXED, W>& L, const double4* src4, const double* srce2,
+                                             int64_t sb, int64_t se, double e2t, double cx, double cy, double cz,
+                                             T tx, T ty, T tz, double (&h)[4]) {
+    const int tid = threadIdx.x, v = tid >> 6;
+    T ax = 0, ay = 0, az = 0, ap = 0;
+    for (int64_t base = sb; base < se; base += 64 * W) {
+      stage_sync<W>();
+      const int64_t j = base + tid;
+      if constexpr (MIXED) {
+        float4 q = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (j < se) {
+          const double4 s = src4[j];
+          q = make_float4((float)(s.x - cx), (float)(s.y - cy), (float)(s.z - cz), (float)s.w);
+        }
+        L.s4[tid] = q;
+        L.se2[tid] = j < se ? (float)(srce2[j] + e2t) : 1.0f;
+      } else {
+        L.s4[tid] = j < se ? src4[j] : make_double4(0.0, 0.0, 0.0, 0.0);
+        L.se2[tid] = j < se ? srce2[j] + e2t : 1.0;
+      }
+      stage_sync<W>();
+      if (W > 1 && base + 64 * v >= se) continue;   // uniform over the wave
+#pragma unroll 1
+      for (int i = 64 * v; i < 64 * v + 64; i += 4) {
+        T dx[4], dy[4], dz[4], m[4], r2[4], y[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const auto s = L.s4[i + u];
+          dx[u] = s.x - tx;
+          dy[u] = s.y - ty;
+          dz[u] = s.z - tz;
+          m[u] = s.w;
+          r2[u] = fma(dz[u], dz[u], fma(dx[u], dx[u], fma(dy[u], dy[u], L.se2[i + u])));
+          if constexpr (MIXED) y[u] = r2[u];
+          else y[u] = rsqrt_f64<FL>(r2[u]);
+        }
+        if constexpr (MIXED) rsq_run(y);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          if constexpr (MIXED && (FL & F_GUARD) != 0) y[u] = r2[u] > 0.0f ? y[u] : 0.0f;
+          if (!(FL & F_NOPOT)) ap = fma(m[u], y[u], ap);
+          if constexpr (!(FL & F_NOACC)) {
+            const T mr = m[u] * y[u];
+            const T w = MIXED ? (mr * y[u]) * y[u] : mr * (y[u] * y[u]);
+            ax = fma(w, dx[u], ax);
+            ay = fma(w, dy[u], ay);
+            az = fma(w, dz[u], az);
+          }
+        }
+      }
+      if constexpr (MIXED) {      // the 64 sources' FP32 sums, as the column code folds them
+        h[0] += (double)ax;
+        h[1] += (double)ay;
+        h[2] += (double)az;
+        h[3] += (double)ap;
+        ax = ay = az = ap = 0;
+      }
+    }
+    if constexpr (!MIXED) {
+      h[0] = ax;
+      h[1] = ay;
+      h[2] = az;
+      h[3] = ap;
+    }
+  }
+};
+
+// blockIdx.x = 8 g + q: targets 512 g + 64 q ... + 63, blockIdx.y = source chunk.  Block targets with
+// nb == 8, or explicit targets with column structure (gated like k_eval_cols).
+template <bool MIXED, int W>
+__global__ __launch_bounds__(64 * W) void k_eval_thin(Tgt T, const double4* __restrict__ src4,
+                                                      const double* __restrict__ srce2, int64_t ns,
+                                                      int64_t chunk, const double* sst, Out O) {
+  __shared__ LdsThin<MIXED, W> L;
+  if (gated_off(O)) return;
+  const int64_t g = blockIdx.x >> 3;
+  const int lane = threadIdx.x & 63;
+  const int64_t t = (int64_t)blockIdx.x * 64 + lane, last = T.n - 1;
+  const int64_t sb = (int64_t)blockIdx.y * chunk;
+  const int64_t se = sb + chunk < ns ? sb + chunk : ns;
+  Out o = O;
+  if (o.part) o.part += (int64_t)blockIdx.y * 4 * o.pstride;
+  double x, y, z, e2, cx = 0.0, cy = 0.0, cz = 0.0;
+  load_target(T, t < last ? t : last, x, y, z, e2);
+  if (!T.blocks) {                // the group's eps, as the column code reads it
+    const int64_t te = g * 512 < last ? g * 512 : last;
+    const double e = T.eps ? T.eps[te] : 0.0;
+    e2 = e * e;
+  }
+  if constexpr (MIXED) {          // the group's anchor (grid_block, cols_group)
+    if (T.blocks) {
+#pragma clang fp contract(off)
+      const double ox = T.ox[g], oy = T.oy[g], oz = T.oz[g], d = T.bdx[g];
+      cx = 0.5 * ((ox + 0.5 * d) + (ox + 7.5 * d));
+      cy = 0.5 * ((oy + 0.5 * d) + (oy + 7.5 * d));
+      cz = 0.5 * ((oz + 0.5 * d) + (oz + 7.5 * d));
+    } else {
+      column_anchor(T, g, lane, cx, cy, cz);
+    }
+  }
+  typedef typename LdsThin<MIXED, W>::T TT;
+  const int fl = tile_flags(sst[ST_E2MIN], e2, e2, o, MIXED);
+  double h[4] = {0.0, 0.0, 0.0, 0.0};
+  typedef ThinRun<MIXED, W> R;
+  TG_DISPATCH_GRID_(R::template run, 0, fl, L, src4, srce2, sb, se, e2, cx, cy, cz, (TT)(x - cx), (TT)(y - cy),
+                    (TT)(z - cz), h)
+  double a[1] = {h[0]}, b[1] = {h[1]}, c[1] = {h[2]}, d[1] = {h[3]};
+  if (wave_sum<W, 1>(L.red, a, b, c, d) && t < T.n) store_result(o, t, a[0], b[0], c[0], d[0]);
+}
+
 // ---------------------------------------------------------------- block sources ----
 template <bool MIXED>
 struct LdsGS {

@@ -612,12 +612,21 @@ static void grid_shape(const tgrav_ctx* c, int mode, int64_t ns, int64_t nblk, i
   *nsplit = (int)((ns + ch - 1) / ch);
 }
 
+// Launches of at most this many column waves per CU (2 per SIMD) take k_eval_thin, whose waves are 8
+// times as many and an eighth as long: a column wave's pass over 64 sources alone takes 15 us in FP64.
+// Per call, thin / column: 1 block x 1,024 stars 66 / 81 us (FP64), 66 / 73 (mixed); 7 x 4,000 75 / 106;
+// 28 x 3,000 94 / 107, mixed 82 / 89; 56 x 4,000 146 / 187, mixed 104 / 128; 200 x 1,000 156 / 167.  Past
+// the line the column's shared dx, dy, dz win: 700 x 300 with the line at 16 or 32 163 against 161.
+#define TG_THIN_WAVES 8
 // The column kernels for the context's waves per workgroup: k_eval_grid (block targets) or
 // k_eval_cols (explicit targets in the blocks' C order), grid (groups, source chunks).
 template <bool MIXED, int W>
 static void column_kernel_w(tgrav_ctx* c, bool blocks, dim3 g, const tg::Tgt& T, int64_t ns,
                             int64_t chunk, const tg::Out& o) {
-  if (blocks)
+  if ((int64_t)g.x * g.y * W <= TG_THIN_WAVES * (int64_t)c->num_cu)
+    tg::k_eval_thin<MIXED, W><<<dim3(8 * g.x, g.y), 64 * W, 0, c->stream>>>(
+        T, c->s4.as<double4>(), c->se2.as<double>(), ns, chunk, c->stat.as<const double>(), o);
+  else if (blocks)
     tg::k_eval_grid<MIXED, W><<<g, 64 * W, 0, c->stream>>>(T, c->s4.as<double4>(), c->se2.as<double>(), ns,
                                                             chunk, c->stat.as<const double>(), o);
   else
