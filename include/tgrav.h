@@ -287,6 +287,16 @@ int tgrav_pm_interpolate(tgrav_ctx* ctx, int64_t np, const double* x, const doub
                          const double* bsize, const double* gx, const double* gy,
                          const double* gz, double* ax, double* ay, double* az, int ptr_kind);
 
+/* The two steps of Particles_longRangeForce (Particles_longRangeForce.F90:70-97) in one: the
+ * accelerations of the particles from the block potential phi, by the row rule of tgrav_pm_gradient at
+ * the corners of each particle's cloud and the interpolation of tgrav_pm_interpolate.  Bit for bit the
+ * two calls' result; the acceleration is formed only where a particle needs it and not stored. */
+int tgrav_pm_long_range(tgrav_ctx* ctx, int64_t np, const double* x, const double* y,
+                        const double* z, const int64_t* blk, int64_t nblk, int nb, int ng,
+                        const double* ox, const double* oy, const double* oz,
+                        const double* bsize, const double* phi, double* ax, double* ay, double* az,
+                        int ptr_kind);
+
 /* ---- batched uneven evaluations --------------------------------------- */
 /* Many independent problems in one persistent launch (device pointers only).  The plan
  * packs the sources, builds cost-sorted work lists (target tile x source chunk) and

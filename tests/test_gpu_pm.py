@@ -142,3 +142,42 @@ def test_device_tensors_match_host(pm, c2pm):
     for q in range(3):
         np.testing.assert_array_equal(g_d[q].cpu().numpy(), g_h[q])
         np.testing.assert_array_equal(a_d[q].cpu().numpy(), a_h[q])
+
+
+# guarded blocks of one slice of the LDS deposit, just over one, several, and too large for it; particles
+# none, one, one per block and many in one block
+@pytest.mark.parametrize("nb,ng,nblk", [(2, 1, 5), (8, 2, 300), (8, 4, 7), (11, 1, 3), (16, 2, 3), (18, 2, 2)])
+@pytest.mark.parametrize("crowd", [0, 1, 700, 3000])
+def test_deposit_and_long_range_at_block_sizes(pm, nb, ng, nblk, crowd):
+    """The deposit against the oracle and under a permutation (bit for bit), clouds reaching into the
+    guard layers, with accumulation; the long-range force equal to the gradient followed by the
+    interpolation, bit for bit."""
+    rng = W.rng_for(1000 * nb + 10 * ng + nblk + crowd)
+    B = LeafBlocks(rng.uniform(-2, 2, (nblk, 3)), rng.uniform(0.1, 1.0, nblk), nb=nb, ng=ng)
+    blk = np.concatenate([np.arange(nblk), np.full(crowd, nblk // 2)])[: crowd + nblk if crowd else 0]
+    h = (B.size / nb)[blk]
+    pos = B.origin[blk] + h[:, None] * rng.uniform(0.6 - ng, nb + ng - 0.6, (blk.size, 3))
+    m = rng.uniform(0.1, 2.0, blk.size)
+    a = [pos[:, 0], pos[:, 1], pos[:, 2], m, blk]
+    got = pm.update_grid_var(*a, B)
+    ref = oracle.pm_deposit(*a, oblocks(B)) if blk.size else np.zeros(B.ncell)
+    np.testing.assert_allclose(got, ref, rtol=1e-13, atol=1e-300)
+    p = rng.permutation(blk.size)
+    np.testing.assert_array_equal(pm.update_grid_var(*[q[p] for q in a], B), got)
+    base = rng.uniform(-1, 1, B.ncell)
+    acc = pm.update_grid_var(*a, B, rho=base.copy(), accumulate=True)
+    np.testing.assert_array_equal(acc, base + got)
+    phi = rng.normal(size=B.ncell)
+    one = pm.long_range_force(pos[:, 0], pos[:, 1], pos[:, 2], blk, B, phi)
+    two = pm.map_mesh_to_particles(pos[:, 0], pos[:, 1], pos[:, 2], blk, B, *pm.accel_list_of_blocks(phi, B))
+    for u, v in zip(one, two):
+        np.testing.assert_array_equal(u, v)
+    if blk.size:
+        bad = blk.copy()
+        bad[-1] = nblk
+        with pytest.raises(TgravError):
+            pm.long_range_force(pos[:, 0], pos[:, 1], pos[:, 2], bad, B, phi)
+        keep = base.copy()
+        with pytest.raises(TgravError):
+            pm.update_grid_var(*a[:4], bad, B, rho=keep)
+        np.testing.assert_array_equal(keep, base)

@@ -75,6 +75,8 @@ SIGNATURES = [
     ("tgrav_pm_gradient", _I32, [_P, _I64, _I32, _I32, _P, _P, _P, _P, _P, _D, _P, _P, _P, _I32]),
     ("tgrav_pm_interpolate", _I32, [_P, _I64, _P, _P, _P, _P, _I64, _I32, _I32, _P, _P, _P, _P, _P,
                                     _P, _P, _P, _P, _P, _I32]),
+    ("tgrav_pm_long_range", _I32, [_P, _I64, _P, _P, _P, _P, _I64, _I32, _I32, _P, _P, _P, _P, _P,
+                                   _P, _P, _P, _I32]),
     ("tgrav_set_bidir_config", _I32, [_P, _I32, _I32, _I32]),
     ("tgrav_bidir_variant_info", _I32, [_I32, _I32, ctypes.POINTER(_I32), ctypes.POINTER(_I32)]),
     ("tgrav_batch_create", _I32, [_P, ctypes.c_int32, ctypes.POINTER(Problem), _I32, _D,

@@ -58,6 +58,17 @@ __device__ __forceinline__ int pm_scale(unsigned long long cmax, int64_t np) {
   return 94 - e;
 }
 
+// c 2^S = H 2^32 + L exactly, 0 <= L < 2^32, and back from the sums of H and L.
+__device__ __forceinline__ void pm_split(double c, int S, unsigned long long& H, unsigned long long& L) {
+  const double t = ldexp(c, S - 32);
+  const double h = floor(t);
+  H = (unsigned long long)(long long)h;
+  L = (unsigned long long)ldexp(t - h, 32);
+}
+__device__ __forceinline__ double pm_value(unsigned long long H, unsigned long long L, int S) {
+  return ldexp((double)(long long)H, 32 - S) + ldexp((double)L, -S);
+}
+
 // Particle p's block, densities and weights; false if the block index or the CIC stencil
 // is outside the guarded block.
 __device__ __forceinline__ bool pm_particle(const PmBlocks& B, const int64_t* blk, int64_t p,
@@ -122,13 +133,10 @@ __global__ void k_pm_deposit(int64_t np, const double* __restrict__ x, const dou
   const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= np) return;
   pm_corners(B, x, y, z, m, blk, p, [&](int64_t idx, double c) {
-    const int S = pm_scale(cmax[idx], np);
-    const double t = ldexp(c, S - 32);
-    const double h = floor(t);
-    const long long H = (long long)h;
-    const unsigned long long L = (unsigned long long)ldexp(t - h, 32);
-    atomicAdd(&accH[idx], (unsigned long long)H);
-    atomicAdd(&accL[idx], L);
+    unsigned long long h, l;
+    pm_split(c, pm_scale(cmax[idx], np), h, l);
+    atomicAdd(&accH[idx], h);
+    atomicAdd(&accL[idx], l);
   });
 }
 
@@ -139,9 +147,121 @@ __global__ void k_pm_finalize(int64_t n, const unsigned long long* __restrict__ 
                               double* __restrict__ rho, int accumulate) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  const int S = pm_scale(cmax[i], np);
-  const double v = ldexp((double)(long long)accH[i], 32 - S) + ldexp((double)accL[i], -S);
+  const double v = pm_value(accH[i], accL[i], pm_scale(cmax[i], np));
   rho[i] = accumulate ? rho[i] + v : v;
+}
+
+// ---- the deposit block by block, in LDS (guarded blocks of at most TG_PM_LDS_CELLS cells) ----
+// The passes above move 56 B per cell through memory (zero three words, read them back, write rho) for
+// particles that touch a few cells of some blocks.  Here the particles are binned by block, and one
+// workgroup per block keeps the three words of its cells in LDS, TG_PM_LDS_SLICE cells at a time, and
+// writes each cell's density once: 8 B per cell.  The sums are integers (and a maximum), so the order
+// of a block's particles does not matter and the densities are the ones above, bit for bit.
+// 8.2 million cells, 10,000 particles: 89 us for the passes above, 30 us here and 14 for the binning.
+#define TG_PM_LDS_CELLS 8192
+#define TG_PM_LDS_SLICE 2048     // 48 KB: three workgroups per CU
+
+// n zeroes (counts, then the offsets' total and the error word).
+__global__ void k_zero_u32(int64_t n, unsigned int* a) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) a[i] = 0u;
+}
+
+// rank[p] = particle p's place among its block's particles (any order); ~0u and *err for a bad particle.
+__global__ __launch_bounds__(256) void k_pm_bin(int64_t np, const double* __restrict__ x, const double* __restrict__ y,
+                                                const double* __restrict__ z, const int64_t* __restrict__ blk,
+                                                PmBlocks B, unsigned int* cnt, unsigned int* __restrict__ rank,
+                                                unsigned long long* err) {
+  const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (p >= np) return;
+  int64_t b;
+  double del, w[3][2];
+  int c0[3];
+  if (!pm_particle(B, blk, p, x[p], y[p], z[p], b, del, c0, w)) {
+    rank[p] = ~0u;
+    if (err) *err = 1ULL;        // every writer stores the same value
+    return;
+  }
+  rank[p] = atomicAdd(&cnt[b], 1u);
+}
+
+// off[b]: a stretch of perm for each block with particles, in whatever order the workgroups come.
+__global__ __launch_bounds__(256) void k_pm_offsets(int64_t nblk, const unsigned int* __restrict__ cnt,
+                                                    unsigned int* __restrict__ off, unsigned int* total) {
+  __shared__ unsigned int wsum[4], start;
+  const int64_t b = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const unsigned int n = b < nblk ? cnt[b] : 0u;
+  unsigned int s = n;            // inclusive sum over the wave
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const unsigned int t = __shfl_up(s, o);
+    if (lane >= o) s += t;
+  }
+  if (lane == 63) wsum[w] = s;
+  __syncthreads();
+  if (threadIdx.x == 0) start = atomicAdd(total, wsum[0] + wsum[1] + wsum[2] + wsum[3]);
+  __syncthreads();
+  unsigned int at = start + s - n;
+  for (int q = 0; q < w; ++q) at += wsum[q];
+  if (b < nblk) off[b] = at;
+}
+
+__global__ __launch_bounds__(256) void k_pm_scatter(int64_t np, const int64_t* __restrict__ blk,
+                                                    const unsigned int* __restrict__ rank,
+                                                    const unsigned int* __restrict__ off,
+                                                    unsigned int* __restrict__ perm) {
+  const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (p >= np) return;
+  const unsigned int r = rank[p];
+  if (r != ~0u) perm[off[blk[p]] + r] = (unsigned int)p;
+}
+
+// One workgroup of 512 lanes per block.
+__global__ __launch_bounds__(512) void k_pm_block(int64_t np, const double* __restrict__ x,
+                                                  const double* __restrict__ y, const double* __restrict__ z,
+                                                  const double* __restrict__ m, const int64_t* __restrict__ blk,
+                                                  PmBlocks B, const unsigned int* __restrict__ cnt,
+                                                  const unsigned int* __restrict__ off,
+                                                  const unsigned int* __restrict__ perm,
+                                                  double* __restrict__ rho, int accumulate) {
+  __shared__ unsigned long long M[TG_PM_LDS_SLICE], H[TG_PM_LDS_SLICE], L[TG_PM_LDS_SLICE];
+  const int64_t b = blockIdx.x, base = b * B.nc;
+  const int nc = (int)B.nc;
+  const unsigned int n = cnt[b];
+  if (n == 0u) {                 // uniform over the workgroup
+    for (int i = threadIdx.x; i < nc; i += 512) rho[base + i] = accumulate ? rho[base + i] + 0.0 : 0.0;
+    return;
+  }
+  const unsigned int o = off[b];
+  for (int lo = 0; lo < nc; lo += TG_PM_LDS_SLICE) {
+    const int len = nc - lo < TG_PM_LDS_SLICE ? nc - lo : TG_PM_LDS_SLICE;
+    for (int i = threadIdx.x; i < len; i += 512) M[i] = H[i] = L[i] = 0ULL;
+    __syncthreads();
+    for (unsigned int q = threadIdx.x; q < n; q += 512)
+      pm_corners(B, x, y, z, m, blk, (int64_t)perm[o + q], [&](int64_t idx, double c) {
+        const int i = (int)(idx - base) - lo;
+        const unsigned long long bits = (unsigned long long)__double_as_longlong(fabs(c));
+        if (bits && i >= 0 && i < len) atomicMax(&M[i], bits);
+      });
+    __syncthreads();
+    for (unsigned int q = threadIdx.x; q < n; q += 512)
+      pm_corners(B, x, y, z, m, blk, (int64_t)perm[o + q], [&](int64_t idx, double c) {
+        const int i = (int)(idx - base) - lo;
+        if (i < 0 || i >= len) return;
+        unsigned long long h, l;
+        pm_split(c, pm_scale(M[i], np), h, l);
+        atomicAdd(&H[i], h);
+        atomicAdd(&L[i], l);
+      });
+    __syncthreads();
+    for (int i = threadIdx.x; i < len; i += 512) {
+      const double v = M[i] ? pm_value(H[i], L[i], pm_scale(M[i], np)) : 0.0;
+      const int64_t t = base + lo + i;
+      rho[t] = accumulate ? rho[t] + v : v;
+    }
+    __syncthreads();
+  }
 }
 
 __global__ void k_zero_u64(int64_t n, unsigned long long* a, unsigned long long* b,
@@ -200,7 +320,7 @@ __global__ __launch_bounds__(256) void k_pm_gradient(PmBlocks B, uint32_t magic,
 }
 
 // a_p = sum over the 8 corners of w g (corner order and roundings of the oracle).  A
-// particle outside its guarded block gets NaN and sets bit 0 of *err.
+// particle outside its guarded block gets NaN and sets *err (may be null).
 __global__ void k_pm_interpolate(int64_t np, const double* __restrict__ x,
                                  const double* __restrict__ y, const double* __restrict__ z,
                                  const int64_t* __restrict__ blk, PmBlocks B,
@@ -215,7 +335,7 @@ __global__ void k_pm_interpolate(int64_t np, const double* __restrict__ x,
   int c0[3];
   double w[3][2];
   if (!pm_particle(B, blk, p, x[p], y[p], z[p], b, del, c0, w)) {
-    atomicOr(err, 1ULL);
+    if (err) *err = 1ULL;        // every writer stores the same value
     ax[p] = ay[p] = az[p] = __longlong_as_double(0x7ff8000000000000LL);
     return;
   }
@@ -237,6 +357,56 @@ __global__ void k_pm_interpolate(int64_t np, const double* __restrict__ x,
   ax[p] = sx;
   ay[p] = sy;
   az[p] = sz;
+}
+
+// Particle accelerations straight from the potential: the row rule of k_pm_gradient at the 8 corners of
+// each particle's cloud, then the CIC sum of k_pm_interpolate, with the same operations in the same
+// order (same bits) and without the three block arrays between them: a whole gradient writes 24 B and
+// reads 8 B per cell (62 us for 8.2 million cells) for the few cells that particles touch.  8 lanes per
+// particle, one per corner (6 loads each instead of 48 in a chain): 10,000 particles in 6 us.
+__global__ __launch_bounds__(256) void k_pm_long_range(int64_t np, const double* __restrict__ x,
+                                                       const double* __restrict__ y, const double* __restrict__ z,
+                                                       const int64_t* __restrict__ blk, PmBlocks B,
+                                                       const double* __restrict__ phi, double* __restrict__ ax,
+                                                       double* __restrict__ ay, double* __restrict__ az,
+                                                       unsigned long long* err) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x, p = i >> 3;
+  const int corner = (int)(i & 7), first = (int)(threadIdx.x & 63) & ~7;
+  const bool in = p < np;        // whole groups of 8 lanes
+  int64_t b = 0;
+  double del = 1.0, w[3][2] = {{0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}};
+  int c0[3] = {0, 0, 0};
+  const bool ok = in && pm_particle(B, blk, p, x[p], y[p], z[p], b, del, c0, w);
+  double q[3] = {0.0, 0.0, 0.0};   // weight times the corner's acceleration
+  if (ok) {
+    const int n = B.nbg, d[3] = {corner & 1, (corner >> 1) & 1, corner >> 2};
+    const int c[3] = {c0[0] + d[0], c0[1] + d[1], c0[2] + d[2]};
+    const int stride[3] = {1, n, n * n};
+    const int r = (c[2] * n + c[1]) * n + c[0];
+    const double* f = phi + b * B.nc;
+    double delxinv = (double)B.nb / B.bs[b];
+    delxinv = 0.5 * delxinv;
+    const double wt = ((d[0] ? w[0][1] : w[0][0]) * (d[1] ? w[1][1] : w[1][0])) * (d[2] ? w[2][1] : w[2][0]);
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      const int ii = c[a] < 1 ? 1 : (c[a] > n - 2 ? n - 2 : c[a]);
+      const int ctr = r + (ii - c[a]) * stride[a];
+      q[a] = wt * (delxinv * (f[ctr - stride[a]] - f[ctr + stride[a]]));
+    }
+  }
+  double s[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+  for (int k = 0; k < 8; ++k)    // corners di fastest, dk slowest
+#pragma unroll
+    for (int a = 0; a < 3; ++a) s[a] = s[a] + __shfl(q[a], first + k);
+  if (!in || corner != 0) return;
+  if (!ok) {
+    if (err) *err = 1ULL;
+    s[0] = s[1] = s[2] = __longlong_as_double(0x7ff8000000000000LL);
+  }
+  ax[p] = s[0];
+  ay[p] = s[1];
+  az[p] = s[2];
 }
 
 }  // namespace tg

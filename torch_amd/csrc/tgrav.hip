@@ -345,7 +345,8 @@ struct tgrav_ctx {
   DevBuf in[12], outb[8], vel[3], part;      // staging for host pointers and scratch
   DevBuf colflag;            // explicit targets: 1 if they have 8^3 column structure
   DevBuf bp4, bpe2, bstat, bppart, bpgrp;   // fused passes: packed particles, partials
-  DevBuf pm[16], pm_acc[3], pm_stat;  // particle-mesh pieces: staging, fixed-point sums, stat
+  DevBuf pm[16], pm_acc[3];  // particle-mesh pieces: staging, fixed-point sums
+  DevBuf pm_cnt, pm_idx;     // particles by block: counts and offsets; ranks and permutation
   DevBuf pkey, pidx, ptmp, pbuf;   // periodic pairs: sort keys and indices (2 x each), sort scratch,
                                    //   per-pair image sums
   unsigned long long* host_flag = nullptr;   // pinned, kHostWords words
@@ -463,15 +464,6 @@ static int reduce_chunks(tgrav_ctx* c, const double* part, int64_t pstride, int 
     tg::k_reduce_chunks<<<grid1(n, 256), 256, 0, c->stream>>>(part, pstride, nsplit, n, fin);
     LAUNCHCHECK("k_reduce_chunks");
   }
-  return 0;
-}
-
-// Reads a device flag word (synchronous).
-static int read_flag(tgrav_ctx* c, const void* dflag, bool* bad) {
-  HIPCHECK(hipMemcpyAsync(c->host_flag + HW_FLAG, dflag, sizeof(unsigned long long), hipMemcpyDeviceToHost,
-                          c->stream));
-  HIPCHECK(hipStreamSynchronize(c->stream));
-  *bad = c->host_flag[HW_FLAG] != 0ULL;
   return 0;
 }
 
@@ -1229,7 +1221,8 @@ int tgrav_destroy(tgrav_ctx* c) {
   c->bpgrp.release();
   for (auto& b : c->pm) b.release();
   for (auto& b : c->pm_acc) b.release();
-  c->pm_stat.release();
+  c->pm_cnt.release();
+  c->pm_idx.release();
   c->pkey.release();
   c->pidx.release();
   c->ptmp.release();
@@ -2044,11 +2037,17 @@ static int pm_geometry(int64_t nblk, int nb, int ng, int64_t* ncell) {
   return 0;
 }
 
+// The error word of a particle kernel: pinned, cleared before the launch and read after the wait; null
+// without validation (nobody waits).
+static unsigned long long* pm_err_word(tgrav_ctx* c) {
+  if (!c->validate) return nullptr;
+  c->host_flag[HW_FLAG] = 0ULL;
+  return c->host_flag + HW_FLAG;
+}
 static int pm_read_err(tgrav_ctx* c, const char* what) {
-  bool bad = false;
-  int rc = read_flag(c, c->pm_stat.as<unsigned long long>() + 1, &bad);
-  if (rc) return rc;
-  if (bad)
+  if (!c->validate) return 0;
+  HIPCHECK(hipStreamSynchronize(c->stream));
+  if (c->host_flag[HW_FLAG] != 0ULL)
     return fail(TGRAV_EINVAL, "%s: a particle's block index is out of range or its cloud leaves "
                 "its guarded block", what);
   return 0;
@@ -2084,36 +2083,62 @@ int tgrav_pm_deposit(tgrav_ctx* c, int64_t np, const double* x, const double* y,
       (rc = pm_out(c, kind, 9, rho, ncell * 8, accumulate != 0, &drho)))
     return rc;
   if (ncell == 0) return 0;
-  if ((rc = c->pm_acc[0].ensure(ncell * 8)) || (rc = c->pm_acc[1].ensure(ncell * 8)) ||
-      (rc = c->pm_acc[2].ensure(ncell * 8)) || (rc = c->pm_stat.ensure(16)))
-    return rc;
   tg::PmBlocks B{(const double*)dox, (const double*)doy, (const double*)doz, (const double*)dbs,
                  nblk, nb, ng, nb + 2 * ng, (int64_t)(nb + 2 * ng) * (nb + 2 * ng) * (nb + 2 * ng)};
-  unsigned long long* H = c->pm_acc[0].as<unsigned long long>();
-  unsigned long long* L = c->pm_acc[1].as<unsigned long long>();
-  unsigned long long* M = c->pm_acc[2].as<unsigned long long>();
-  unsigned long long* st = c->pm_stat.as<unsigned long long>();
-  tg::k_zero_u64<<<grid1(ncell, 256), 256, 0, c->stream>>>(ncell, H, L, M);
-  tg::k_zero_u64<<<1, 64, 0, c->stream>>>(2, st, nullptr, nullptr);
-  LAUNCHCHECK("k_zero_u64");
-  if (np > 0) {
-    tg::k_pm_cell_max<<<grid1(np, 256), 256, 0, c->stream>>>(
-        np, (const double*)dx_, (const double*)dy_, (const double*)dz_, (const double*)dm_,
-        (const int64_t*)db_, B, M, st + 1);
-    LAUNCHCHECK("k_pm_cell_max");
-    if (c->validate && (rc = pm_read_err(c, "tgrav_pm_deposit"))) return rc;
+  unsigned long long* err = pm_err_word(c);
+  // Block by block in LDS where a guarded block is a few slices of it (k_pm_block); larger blocks would
+  // walk their particles once per slice and keep the passes over memory.
+  if (B.nc <= TG_PM_LDS_CELLS && nblk <= 0x7fffffffLL) {
+    if ((rc = c->pm_cnt.ensure((size_t)(2 * nblk + 1) * 4)) || (rc = c->pm_idx.ensure((size_t)std::max<int64_t>(np, 1) * 8)))
+      return rc;
+    unsigned int *cnt = c->pm_cnt.as<unsigned int>(), *total = cnt + nblk, *off = total + 1;
+    unsigned int *rank = c->pm_idx.as<unsigned int>(), *perm = rank + np;
+    tg::k_zero_u32<<<grid1(nblk + 1, 256), 256, 0, c->stream>>>(nblk + 1, cnt);
+    LAUNCHCHECK("k_zero_u32");
+    if (np > 0) {
+      tg::k_pm_bin<<<grid1(np, 256), 256, 0, c->stream>>>(np, (const double*)dx_, (const double*)dy_,
+                                                          (const double*)dz_, (const int64_t*)db_, B, cnt, rank, err);
+      LAUNCHCHECK("k_pm_bin");
+      tg::k_pm_offsets<<<grid1(nblk, 256), 256, 0, c->stream>>>(nblk, cnt, off, total);
+      tg::k_pm_scatter<<<grid1(np, 256), 256, 0, c->stream>>>(np, (const int64_t*)db_, rank, off, perm);
+      LAUNCHCHECK("k_pm_scatter");
+      if ((rc = pm_read_err(c, "tgrav_pm_deposit"))) return rc;
+    }
     rc = timed_launch(c, np, ncell, [&]() -> int {
-      tg::k_pm_deposit<<<grid1(np, 256), 256, 0, c->stream>>>(
-          np, (const double*)dx_, (const double*)dy_, (const double*)dz_, (const double*)dm_,
-          (const int64_t*)db_, B, M, H, L);
-      LAUNCHCHECK("k_pm_deposit");
+      tg::k_pm_block<<<(unsigned)nblk, 512, 0, c->stream>>>(
+          np, (const double*)dx_, (const double*)dy_, (const double*)dz_, (const double*)dm_, (const int64_t*)db_, B,
+          cnt, off, perm, (double*)drho, accumulate != 0);
+      LAUNCHCHECK("k_pm_block");
       return 0;
     });
     if (rc) return rc;
+  } else {
+    if ((rc = c->pm_acc[0].ensure(ncell * 8)) || (rc = c->pm_acc[1].ensure(ncell * 8)) ||
+        (rc = c->pm_acc[2].ensure(ncell * 8)))
+      return rc;
+    unsigned long long* H = c->pm_acc[0].as<unsigned long long>();
+    unsigned long long* L = c->pm_acc[1].as<unsigned long long>();
+    unsigned long long* M = c->pm_acc[2].as<unsigned long long>();
+    tg::k_zero_u64<<<grid1(ncell, 256), 256, 0, c->stream>>>(ncell, H, L, M);
+    LAUNCHCHECK("k_zero_u64");
+    if (np > 0) {
+      tg::k_pm_cell_max<<<grid1(np, 256), 256, 0, c->stream>>>(
+          np, (const double*)dx_, (const double*)dy_, (const double*)dz_, (const double*)dm_,
+          (const int64_t*)db_, B, M, err);
+      LAUNCHCHECK("k_pm_cell_max");
+      if ((rc = pm_read_err(c, "tgrav_pm_deposit"))) return rc;
+      rc = timed_launch(c, np, ncell, [&]() -> int {
+        tg::k_pm_deposit<<<grid1(np, 256), 256, 0, c->stream>>>(
+            np, (const double*)dx_, (const double*)dy_, (const double*)dz_, (const double*)dm_,
+            (const int64_t*)db_, B, M, H, L);
+        LAUNCHCHECK("k_pm_deposit");
+        return 0;
+      });
+      if (rc) return rc;
+    }
+    tg::k_pm_finalize<<<grid1(ncell, 256), 256, 0, c->stream>>>(ncell, H, L, M, np, (double*)drho, accumulate != 0);
+    LAUNCHCHECK("k_pm_finalize");
   }
-  tg::k_pm_finalize<<<grid1(ncell, 256), 256, 0, c->stream>>>(ncell, H, L, M, np, (double*)drho,
-                                                               accumulate != 0);
-  LAUNCHCHECK("k_pm_finalize");
   if ((rc = pm_back(c, kind, rho, drho, ncell * 8))) return rc;
   if (kind == TGRAV_HOST) HIPCHECK(hipStreamSynchronize(c->stream));
   return 0;
@@ -2202,22 +2227,69 @@ int tgrav_pm_interpolate(tgrav_ctx* c, int64_t np, const double* x, const double
       (rc = pm_out(c, kind, 12, ay, np * 8, false, &day)) ||
       (rc = pm_out(c, kind, 13, az, np * 8, false, &daz)))
     return rc;
-  if ((rc = c->pm_stat.ensure(16))) return rc;
-  unsigned long long* st = c->pm_stat.as<unsigned long long>();
-  tg::k_zero_u64<<<1, 64, 0, c->stream>>>(2, st, nullptr, nullptr);
-  LAUNCHCHECK("k_zero_u64");
+  unsigned long long* err = pm_err_word(c);
   tg::PmBlocks B{(const double*)dox, (const double*)doy, (const double*)doz, (const double*)dbs,
                  nblk, nb, ng, nb + 2 * ng, (int64_t)(nb + 2 * ng) * (nb + 2 * ng) * (nb + 2 * ng)};
   rc = timed_launch(c, np, ncell, [&]() -> int {
     tg::k_pm_interpolate<<<grid1(np, 256), 256, 0, c->stream>>>(
         np, (const double*)dx_, (const double*)dy_, (const double*)dz_, (const int64_t*)db_, B,
         (const double*)dgx, (const double*)dgy, (const double*)dgz, (double*)dax, (double*)day,
-        (double*)daz, st + 1);
+        (double*)daz, err);
     LAUNCHCHECK("k_pm_interpolate");
     return 0;
   });
   if (rc) return rc;
-  if (c->validate && (rc = pm_read_err(c, "tgrav_pm_interpolate"))) return rc;
+  if ((rc = pm_read_err(c, "tgrav_pm_interpolate"))) return rc;
+  if ((rc = pm_back(c, kind, ax, dax, np * 8)) || (rc = pm_back(c, kind, ay, day, np * 8)) ||
+      (rc = pm_back(c, kind, az, daz, np * 8)))
+    return rc;
+  if (kind == TGRAV_HOST) HIPCHECK(hipStreamSynchronize(c->stream));
+  return 0;
+}
+
+int tgrav_pm_long_range(tgrav_ctx* c, int64_t np, const double* x, const double* y, const double* z,
+                        const int64_t* blk, int64_t nblk, int nb, int ng, const double* ox,
+                        const double* oy, const double* oz, const double* bsize, const double* phi,
+                        double* ax, double* ay, double* az, int kind) {
+  if (!c) return fail(TGRAV_EINVAL, "context is NULL");
+  int rc;
+  int64_t ncell;
+  if ((rc = check_kind(kind)) || (rc = pm_geometry(nblk, nb, ng, &ncell))) return rc;
+  if (np < 0) return fail(TGRAV_EINVAL, "np must be >= 0");
+  if (nblk > 0 && (!bsize || !phi)) return fail(TGRAV_EINVAL, "bsize and phi are required");
+  if (np > 0 && (!x || !y || !z || !blk || !ax || !ay || !az))
+    return fail(TGRAV_EINVAL, "x, y, z, blk and ax, ay, az are required");
+  if (np > 0 && (nblk == 0 || !ox || !oy || !oz))
+    return fail(TGRAV_EINVAL, "blocks (ox, oy, oz, bsize, phi) are required");
+  if ((rc = set_device(c))) return rc;
+  if (kind == TGRAV_HOST && c->validate) {
+    const double* arr[8] = {x, y, z, ox, oy, oz, bsize, phi};
+    for (int q = 0; q < 8; ++q)
+      if (!host_finite(q < 3 ? np : q < 7 ? nblk : ncell, arr[q]))
+        return fail(TGRAV_ENONFINITE, "non-finite input %d", q);
+  }
+  if (np == 0) return 0;
+  const void *dx_, *dy_, *dz_, *db_, *dox, *doy, *doz, *dbs, *dphi;
+  void *dax, *day, *daz;
+  if ((rc = pm_in(c, kind, 0, x, np * 8, &dx_)) || (rc = pm_in(c, kind, 1, y, np * 8, &dy_)) ||
+      (rc = pm_in(c, kind, 2, z, np * 8, &dz_)) || (rc = pm_in(c, kind, 3, blk, np * 8, &db_)) ||
+      (rc = pm_in(c, kind, 4, ox, nblk * 8, &dox)) || (rc = pm_in(c, kind, 5, oy, nblk * 8, &doy)) ||
+      (rc = pm_in(c, kind, 6, oz, nblk * 8, &doz)) || (rc = pm_in(c, kind, 7, bsize, nblk * 8, &dbs)) ||
+      (rc = pm_in(c, kind, 8, phi, ncell * 8, &dphi)) || (rc = pm_out(c, kind, 11, ax, np * 8, false, &dax)) ||
+      (rc = pm_out(c, kind, 12, ay, np * 8, false, &day)) || (rc = pm_out(c, kind, 13, az, np * 8, false, &daz)))
+    return rc;
+  unsigned long long* err = pm_err_word(c);
+  tg::PmBlocks B{(const double*)dox, (const double*)doy, (const double*)doz, (const double*)dbs,
+                 nblk, nb, ng, nb + 2 * ng, (int64_t)(nb + 2 * ng) * (nb + 2 * ng) * (nb + 2 * ng)};
+  rc = timed_launch(c, np, ncell, [&]() -> int {
+    tg::k_pm_long_range<<<grid1(8 * np, 256), 256, 0, c->stream>>>(
+        np, (const double*)dx_, (const double*)dy_, (const double*)dz_, (const int64_t*)db_, B,
+        (const double*)dphi, (double*)dax, (double*)day, (double*)daz, err);
+    LAUNCHCHECK("k_pm_long_range");
+    return 0;
+  });
+  if (rc) return rc;
+  if ((rc = pm_read_err(c, "tgrav_pm_long_range"))) return rc;
   if ((rc = pm_back(c, kind, ax, dax, np * 8)) || (rc = pm_back(c, kind, ay, day, np * 8)) ||
       (rc = pm_back(c, kind, az, daz, np * 8)))
     return rc;

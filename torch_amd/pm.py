@@ -178,9 +178,21 @@ class ParticleMesh(GravityField):
 
     def long_range_force(self, x, y, z, blk, blocks, phi):
         """Particle accelerations from the block potential: finite differences, then CIC
-        (Particles_longRangeForce.F90:70-97)."""
-        g = self.accel_list_of_blocks(phi, blocks)
-        return self.map_mesh_to_particles(x, y, z, blk, blocks, *g)
+        (Particles_longRangeForce.F90:70-97), formed at the corners of the particles' clouds only
+        (bit for bit accel_list_of_blocks, then map_mesh_to_particles)."""
+        n = len(x) if not _is_torch(x) else int(x.shape[0])
+        dev = self._dev(x, y, z, blk, phi, blocks.origin, blocks.size)
+        xs = self._prep(dev, [x, y, z], n, ["x", "y", "z"])
+        b = self._prep(dev, [blk], n, ["blk"], dtype=np.int64)[0]
+        g = self._geom(blocks, dev)
+        f = self._prep(dev, [phi], blocks.ncell, ["phi"])[0]
+        outs = [self._empty(dev, n) for _ in range(3)]
+        kind = self._stream(dev)
+        rc = self.lib.tgrav_pm_long_range(self._ctx, n, *[self._ptr(a) for a in xs], self._ptr(b), blocks.nblk,
+                                          blocks.nb, blocks.ng, *[self._ptr(a) for a in g], self._ptr(f),
+                                          *[self._ptr(a) for a in outs], kind)
+        _lib.check(rc, "tgrav_pm_long_range")
+        return tuple(outs)
 
     @staticmethod
     def _check_out(a, n, dev, name):
