@@ -124,6 +124,38 @@ def test_blocks_match_explicit_and_oracle(mode, nblk, npart):
 
 
 @pytest.mark.parametrize("mode", ["fp64", "mixed"])
+@pytest.mark.parametrize("nblk,npart", [(4, 64), (5, 63), (9, 129), (66, 65)])
+@pytest.mark.parametrize("odd", ["none", "zero_eps", "z_reversed"])
+def test_workgroups_of_four_blocks(mode, nblk, npart, odd):
+    """Full and part workgroups of four blocks, and one whose blocks ask for different forms: a single
+    block with no softening (guarded pairs), or with its columns' z reversed (no shared dz).  66 blocks:
+    the particle sums of 17 workgroups are added in two levels."""
+    B, C, P = blocks_and_particles(nblk * 77 + npart, nblk, npart)
+    last = slice(512 * (nblk - 1), 512 * nblk)
+    if odd == "zero_eps":
+        C["eps"] = C["eps"].copy()
+        C["eps"][last] = 0.0
+        P["eps"] = np.zeros(npart)
+        for q in "xyz":                       # and one pair at no distance there
+            P[q][0] = C[q][512 * nblk - 5]
+    elif odd == "z_reversed":
+        for q in ("z", "m"):
+            C[q] = C[q].copy()
+            C[q][last][8:16] = C[q][last][8:16][::-1].copy()
+    with GravityField(mode) as f:
+        co, po = run(f, C, P)
+    (pa, pb, pc, pp), (ca, cb, cc, cp) = oracle.bidirectional(
+        C["x"], C["y"], C["z"], C["m"], C["eps"], P["x"], P["y"], P["z"], P["m"], P["eps"], G)
+    for name, got, ref in (("cells", co, (ca, cb, cc, cp)), ("particles", po, (pa, pb, pc, pp))):
+        s = _util.summary(got, ref)
+        print(mode, nblk, npart, odd, name, s, flush=True)
+        if mode == "fp64":
+            assert s["acc_max"] <= 1e-12 and s["pot_max"] <= 1e-12, (name, s)
+        else:
+            assert s["acc_median"] <= 1e-6 and s["acc_max"] <= 1e-4, (name, s)
+
+
+@pytest.mark.parametrize("mode", ["fp64", "mixed"])
 def test_shared_and_per_lane_dz_agree(mode):
     """Explicit cells in the blocks' C order, whose 64 columns per block hold the same 8 z, take the
     column kernel with each staged particle's 8 dz formed once; listing the 8 cells of one column per

@@ -13,7 +13,7 @@
 // wave order and written as this cell tile's partial sums; a second kernel adds the cell
 // tiles' partials per particle in tile order.  Everything is deterministic.
 #pragma once
-#include "kernels.hpp"
+#include "grid.hpp"
 
 namespace tg {
 
@@ -229,6 +229,7 @@ __global__ void k_bidir_group(const double* __restrict__ ppart, int ntiles, int 
   const int t0 = blockIdx.y * per;
   const int t1 = t0 + per < ntiles ? t0 + per : ntiles;
   double s0 = 0, s1 = 0, s2 = 0, s3 = 0;
+#pragma unroll 4
   for (int t = t0; t < t1; ++t) {
     const double* p = ppart + (int64_t)t * 4 * np;
     s0 += p[j];
@@ -249,6 +250,7 @@ __global__ void k_bidir_reduce(const double* __restrict__ ppart, int ntiles, int
   const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (j >= np || gated_off(O)) return;
   double s0 = 0, s1 = 0, s2 = 0, s3 = 0;
+#pragma unroll 4
   for (int t = 0; t < ntiles; ++t) {
     const double* p = ppart + (int64_t)t * 4 * np;
     s0 += p[j];
@@ -291,12 +293,19 @@ struct CellBlocks {
 #define TG_BIGRID_SUMW 3
 #endif
 
+// Blocks per workgroup: each wave has its own block, and the particle side of a tile is summed over the
+// workgroup's blocks before it is written, so a particle's partial sums are a quarter as many (80 MB
+// instead of 320 at 1,000 blocks x 10,000 particles).  The mixed kernel is held to three waves per SIMD,
+// 168 registers with 4 spilled: 1,761 us there against 2,001 at two waves and 1,850 with one block per
+// workgroup; FP64, 500 x 5,000, 1,141 against 1,221.
+#define TG_BIGRID_BLOCKS 4
 template <bool MIXED>
-struct LdsBiGrid {
+struct LdsBiGrid {               // one wave's
   typedef typename std::conditional<MIXED, float, double>::type T;
   typename std::conditional<MIXED, float4, double4>::type p4[64];
   T pe2[64];
-  typename std::conditional<MIXED, float4, double4>::type acc[64];   // particle sums of the tile
+  // particle sums of the tile; two copies in turn, so that the other waves may still read the last one
+  T acc[2][64][4];
   // ZROW (every lane holds the same 8 cell z): z_p - z_k of each staged particle, cells 0-3 in
   // dz[0], 4-7 in dz[1], formed once by the lane that stages the particle
   typename std::conditional<MIXED, float4, double4>::type dz[2][64];
@@ -304,7 +313,7 @@ struct LdsBiGrid {
 
 template <bool MIXED, bool GUARD, bool ZROW>
 __device__ __forceinline__ void bi_grid_tiles(
-    LdsBiGrid<MIXED>& L, const double4* __restrict__ p4, const double* __restrict__ pe2,
+    LdsBiGrid<MIXED>* LL, bool on, const double4* __restrict__ p4, const double* __restrict__ pe2,
     int64_t pb, int64_t pe, double e2c, double ax_, double ay_, double az_,
     typename std::conditional<MIXED, float, double>::type qx,
     typename std::conditional<MIXED, float, double>::type qy,
@@ -313,126 +322,135 @@ __device__ __forceinline__ void bi_grid_tiles(
     double (&hx)[8], double (&hy)[8], double (&hz)[8], double (&hp)[8],
     double* __restrict__ ppart, int64_t np) {
   typedef typename std::conditional<MIXED, float, double>::type T;
-  const int lane = threadIdx.x;
-  for (int64_t base = pb; base < pe; base += 64) {
-    __syncthreads();
-    const int64_t j = base + lane;
-    T pz = (T)0;
-    if (j < pe) {
-      const double4 s = p4[j];
-      if constexpr (MIXED)
-        L.p4[lane] = make_float4((float)(s.x - ax_), (float)(s.y - ay_), (float)(s.z - az_), (float)s.w);
-      else
-        L.p4[lane] = s;
-      pz = MIXED ? (T)(s.z - az_) : (T)s.z;
-      L.pe2[lane] = (T)(pe2[j] + e2c);
-    } else {                      // padding particle: zero mass, eps^2 = 1
-      if constexpr (MIXED) L.p4[lane] = make_float4(0.f, 0.f, 0.f, 0.f);
-      else L.p4[lane] = make_double4(0.0, 0.0, 0.0, 0.0);
-      L.pe2[lane] = (T)1.0;
-    }
-    if constexpr (ZROW) {         // this lane's qz are every lane's: the dz the loop would form
-      L.dz[0][lane] = {pz - qz[0], pz - qz[1], pz - qz[2], pz - qz[3]};
-      L.dz[1][lane] = {pz - qz[4], pz - qz[5], pz - qz[6], pz - qz[7]};
-    }
-    if constexpr (MIXED) L.acc[lane] = make_float4(0.f, 0.f, 0.f, 0.f);
-    else L.acc[lane] = make_double4(0.0, 0.0, 0.0, 0.0);
-    __syncthreads();
-    T cx[8], cy[8], cz[8], cp[8];
+  typedef typename std::conditional<MIXED, float4, double4>::type T4;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  LdsBiGrid<MIXED>& L = LL[wave];
+  int cur = 0;
+  for (int64_t base = pb; base < pe; base += 64, cur ^= 1) {
+    T4* acc = reinterpret_cast<T4*>(L.acc[cur]);
+    if (on) {                     // this wave has a block (uniform over the wave)
+      const int64_t j = base + lane;
+      T pz = (T)0;
+      if (j < pe) {
+        const double4 s = p4[j];
+        if constexpr (MIXED)
+          L.p4[lane] = make_float4((float)(s.x - ax_), (float)(s.y - ay_), (float)(s.z - az_), (float)s.w);
+        else
+          L.p4[lane] = s;
+        pz = MIXED ? (T)(s.z - az_) : (T)s.z;
+        L.pe2[lane] = (T)(pe2[j] + e2c);
+      } else {                      // padding particle: zero mass, eps^2 = 1
+        if constexpr (MIXED) L.p4[lane] = make_float4(0.f, 0.f, 0.f, 0.f);
+        else L.p4[lane] = make_double4(0.0, 0.0, 0.0, 0.0);
+        L.pe2[lane] = (T)1.0;
+      }
+      if constexpr (ZROW) {         // this lane's qz are every lane's: the dz the loop would form
+        L.dz[0][lane] = {pz - qz[0], pz - qz[1], pz - qz[2], pz - qz[3]};
+        L.dz[1][lane] = {pz - qz[4], pz - qz[5], pz - qz[6], pz - qz[7]};
+      }
+      acc[lane] = T4{(T)0, (T)0, (T)0, (T)0};
+      stage_sync<TG_BIGRID_BLOCKS>();
+      T cx[8], cy[8], cz[8], cp[8];
 #pragma unroll
-    for (int k = 0; k < 8; ++k) cx[k] = cy[k] = cz[k] = cp[k] = (T)0;
+      for (int k = 0; k < 8; ++k) cx[k] = cy[k] = cz[k] = cp[k] = (T)0;
 #pragma unroll TG_BIGRID_UNROLL
-    for (int s = 0; s < 64; ++s) {
-      const int jj = (lane + s) & 63;
-      const auto P = L.p4[jj];
-      const T dx = P.x - qx, dy = P.y - qy;
-      const T base2 = fma(dx, dx, fma(dy, dy, L.pe2[jj]));
-      constexpr bool sumw = TG_BIGRID_SUMW == 2 || (TG_BIGRID_SUMW == 1 && !MIXED) ||
-                            (TG_BIGRID_SUMW == 3 && MIXED);
-      T ux = 0, uy = 0, uz = 0, up = 0, uw = 0;
-      T zr[8];
-      if constexpr (ZROW) {
-        const auto d0 = L.dz[0][jj], d1 = L.dz[1][jj];
-        zr[0] = d0.x; zr[1] = d0.y; zr[2] = d0.z; zr[3] = d0.w;
-        zr[4] = d1.x; zr[5] = d1.y; zr[6] = d1.z; zr[7] = d1.w;
-      }
-      T y[8];
-      bool near[8];                 // GUARD: r^2 == 0 (the pair contributes 0)
-#pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        if constexpr (!ZROW) zr[k] = P.z - qz[k];
-        const T r2 = fma(zr[k], zr[k], base2);
-        if constexpr (MIXED) {
-          y[k] = r2;
-          near[k] = !(r2 > (T)0);
-        } else {
-          y[k] = rsqrt_f64<GUARD ? F_GUARD : 0>(r2);
+      for (int s = 0; s < 64; ++s) {
+        const int jj = (lane + s) & 63;
+        const auto P = L.p4[jj];
+        const T dx = P.x - qx, dy = P.y - qy;
+        const T base2 = fma(dx, dx, fma(dy, dy, L.pe2[jj]));
+        constexpr bool sumw = TG_BIGRID_SUMW == 2 || (TG_BIGRID_SUMW == 1 && !MIXED) ||
+                              (TG_BIGRID_SUMW == 3 && MIXED);
+        T ux = 0, uy = 0, uz = 0, up = 0, uw = 0;
+        T zr[8];
+        if constexpr (ZROW) {
+          const auto d0 = L.dz[0][jj], d1 = L.dz[1][jj];
+          zr[0] = d0.x; zr[1] = d0.y; zr[2] = d0.z; zr[3] = d0.w;
+          zr[4] = d1.x; zr[5] = d1.y; zr[6] = d1.z; zr[7] = d1.w;
         }
-      }
-      // one run of 8 v_rsq_f32 per particle (rsq_run): 2.02 ms per call on 1,000 blocks x 10,000
-      // particles against 2.28 with the v_rsq_f32 spread over the column
-      if constexpr (MIXED) rsq_run(y);
+        T y[8];
+        bool near[8];                 // GUARD: r^2 == 0 (the pair contributes 0)
 #pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        if constexpr (MIXED && GUARD) y[k] = near[k] ? (T)0 : y[k];
-        const T y3 = (y[k] * y[k]) * y[k];
-        const T wp = P.w * y3;
-        cp[k] = fma(P.w, y[k], cp[k]);
-        cx[k] = fma(wp, dx, cx[k]);
-        cy[k] = fma(wp, dy, cy[k]);
-        cz[k] = fma(wp, zr[k], cz[k]);
-        const T wc = qm[k] * y3;
-        up = fma(qm[k], y[k], up);
+        for (int k = 0; k < 8; ++k) {
+          if constexpr (!ZROW) zr[k] = P.z - qz[k];
+          const T r2 = fma(zr[k], zr[k], base2);
+          if constexpr (MIXED) {
+            y[k] = r2;
+            near[k] = !(r2 > (T)0);
+          } else {
+            y[k] = rsqrt_f64<GUARD ? F_GUARD : 0>(r2);
+          }
+        }
+        // one run of 8 v_rsq_f32 per particle (rsq_run): 2.02 ms per call on 1,000 blocks x 10,000
+        // particles against 2.28 with the v_rsq_f32 spread over the column
+        if constexpr (MIXED) rsq_run(y);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          if constexpr (MIXED && GUARD) y[k] = near[k] ? (T)0 : y[k];
+          const T y3 = (y[k] * y[k]) * y[k];
+          const T wp = P.w * y3;
+          cp[k] = fma(P.w, y[k], cp[k]);
+          cx[k] = fma(wp, dx, cx[k]);
+          cy[k] = fma(wp, dy, cy[k]);
+          cz[k] = fma(wp, zr[k], cz[k]);
+          const T wc = qm[k] * y3;
+          up = fma(qm[k], y[k], up);
+          if constexpr (sumw) {
+            uw += wc;
+          } else {
+            ux = fma(wc, dx, ux);
+            uy = fma(wc, dy, uy);
+          }
+          uz = fma(wc, zr[k], uz);
+        }
         if constexpr (sumw) {
-          uw += wc;
-        } else {
-          ux = fma(wc, dx, ux);
-          uy = fma(wc, dy, uy);
+          ux = uw * dx;
+          uy = uw * dy;
         }
-        uz = fma(wc, zr[k], uz);
+        T4 a = acc[jj];             // the tile's sum for this particle (FP32 in mixed mode)
+        a.x += ux;
+        a.y += uy;
+        a.z += uz;
+        a.w += up;
+        acc[jj] = a;
       }
-      if constexpr (sumw) {
-        ux = uw * dx;
-        uy = uw * dy;
-      }
-      auto a = L.acc[jj];         // the tile's sum for this particle (FP32 in mixed mode)
-      a.x += ux;
-      a.y += uy;
-      a.z += uz;
-      a.w += up;
-      L.acc[jj] = a;
-    }
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      hx[k] += (double)cx[k];
-      hy[k] += (double)cy[k];
-      hz[k] += (double)cz[k];
-      hp[k] += (double)cp[k];
+      for (int k = 0; k < 8; ++k) {
+        hx[k] += (double)cx[k];
+        hy[k] += (double)cy[k];
+        hz[k] += (double)cz[k];
+        hp[k] += (double)cp[k];
+      }
+    } else {
+      acc[lane] = T4{(T)0, (T)0, (T)0, (T)0};
     }
     __syncthreads();
-    if (j < pe) {                 // this block's partial sums for particle j
-      const auto a = L.acc[lane];
-      ppart[j] = (double)a.x;
-      ppart[np + j] = (double)a.y;
-      ppart[2 * np + j] = (double)a.z;
-      ppart[3 * np + j] = (double)a.w;
+    // lane: component `wave` of the tile's particle `lane`, over the workgroup's blocks in order
+    const int64_t j = base + lane;
+    if (j < pe) {
+      double s = (double)LL[0].acc[cur][lane][wave];
+#pragma unroll
+      for (int w = 1; w < TG_BIGRID_BLOCKS; ++w) s += (double)LL[w].acc[cur][lane][wave];
+      ppart[wave * np + j] = s;
     }
   }
 }
 
-// blockIdx.x = leaf block, blockIdx.y = particle chunk.  Cell results (C order inside the
-// block) go to CO (final, or chunk partials when CO.part is set); particle partials go to
-// ppart[(block * 4 + q) * np + j], summed by k_bidir_reduce in block order.
+// blockIdx.x = group of TG_BIGRID_BLOCKS leaf blocks (one per wave), blockIdx.y = particle chunk.  Cell
+// results (C order inside the block) go to CO (final, or chunk partials when CO.part is set); particle
+// partials go to ppart[(group * 4 + q) * np + j], summed by k_bidir_reduce in group order.
 template <bool MIXED>
-__global__ __launch_bounds__(64) void k_bidir_grid(CellBlocks C, const double4* __restrict__ p4,
-                                                   const double* __restrict__ pe2, int64_t np,
-                                                   int64_t chunk, const double* e2p_min_p, Out CO,
-                                                   double* __restrict__ ppart) {
+__global__ __launch_bounds__(64 * TG_BIGRID_BLOCKS, MIXED ? 3 : 1) void k_bidir_grid(
+    CellBlocks C, const double4* __restrict__ p4, const double* __restrict__ pe2, int64_t np, int64_t chunk,
+    const double* e2p_min_p, Out CO, double* __restrict__ ppart) {
   typedef typename std::conditional<MIXED, float, double>::type T;
-  __shared__ LdsBiGrid<MIXED> L;
+  static_assert(TG_BIGRID_BLOCKS == 4, "one wave per component of a particle's sums");
+  __shared__ LdsBiGrid<MIXED> L[TG_BIGRID_BLOCKS];
   if (gated_off(CO)) return;    // explicit cells that are not 8^3 block columns
-  const int lane = threadIdx.x;
-  const int64_t b = blockIdx.x;
+  const int lane = threadIdx.x & 63;
+  const int64_t bw = (int64_t)blockIdx.x * TG_BIGRID_BLOCKS + (threadIdx.x >> 6);
+  const bool on = bw < C.nblk;
+  const int64_t b = on ? bw : C.nblk - 1;
   const int i = lane >> 3, jj = lane & 7;
   const int64_t pb = (int64_t)blockIdx.y * chunk;
   const int64_t pe = pb + chunk < np ? pb + chunk : np;
@@ -489,23 +507,25 @@ __global__ __launch_bounds__(64) void k_bidir_grid(CellBlocks C, const double4* 
     qm[k] = (T)C.m[t0 + k];
   }
   const double lo = *e2p_min_p + e2c;
-  const bool guard = MIXED ? !(lo > TG_F32_TINY_E2) : !(lo > 0.0);
+  const bool guard = __syncthreads_or(MIXED ? !(lo > TG_F32_TINY_E2) : !(lo > 0.0)) != 0;
   double hx[8], hy[8], hz[8], hp[8];
 #pragma unroll
   for (int k = 0; k < 8; ++k) hx[k] = hy[k] = hz[k] = hp[k] = 0.0;
-  double* pp = ppart + b * 4 * np;
+  double* pp = ppart + (int64_t)blockIdx.x * 4 * np;
   // the same 8 z in every lane: leaf blocks always, explicit cells in their C order (wave vote)
   bool same = true;
 #pragma unroll
   for (int k = 0; k < 8; ++k) same = same && z[k] == __shfl(z[k], 0);
-  const bool zrow = !C.cx || __all(same) != 0;
+  // (both choices are the workgroup's: its waves meet at the tiles' barriers)
+  const bool zrow = !C.cx || __syncthreads_and(same) != 0;
   if (zrow) {
-    if (guard) bi_grid_tiles<MIXED, true, true>(L, p4, pe2, pb, pe, e2c, ax_, ay_, az_, qx, qy, qz, qm, hx, hy, hz, hp, pp, np);
-    else bi_grid_tiles<MIXED, false, true>(L, p4, pe2, pb, pe, e2c, ax_, ay_, az_, qx, qy, qz, qm, hx, hy, hz, hp, pp, np);
+    if (guard) bi_grid_tiles<MIXED, true, true>(L, on, p4, pe2, pb, pe, e2c, ax_, ay_, az_, qx, qy, qz, qm, hx, hy, hz, hp, pp, np);
+    else bi_grid_tiles<MIXED, false, true>(L, on, p4, pe2, pb, pe, e2c, ax_, ay_, az_, qx, qy, qz, qm, hx, hy, hz, hp, pp, np);
   } else {
-    if (guard) bi_grid_tiles<MIXED, true, false>(L, p4, pe2, pb, pe, e2c, ax_, ay_, az_, qx, qy, qz, qm, hx, hy, hz, hp, pp, np);
-    else bi_grid_tiles<MIXED, false, false>(L, p4, pe2, pb, pe, e2c, ax_, ay_, az_, qx, qy, qz, qm, hx, hy, hz, hp, pp, np);
+    if (guard) bi_grid_tiles<MIXED, true, false>(L, on, p4, pe2, pb, pe, e2c, ax_, ay_, az_, qx, qy, qz, qm, hx, hy, hz, hp, pp, np);
+    else bi_grid_tiles<MIXED, false, false>(L, on, p4, pe2, pb, pe, e2c, ax_, ay_, az_, qx, qy, qz, qm, hx, hy, hz, hp, pp, np);
   }
+  if (!on) return;
   Out o = CO;
   if (o.part) o.part += (int64_t)blockIdx.y * 4 * o.pstride;
 #pragma unroll

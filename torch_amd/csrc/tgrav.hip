@@ -970,15 +970,15 @@ static int launch_flash(tgrav_ctx* c, int mode, const tg::Tgt& T, const tg::Out&
 }
 
 // Particle side of the fused passes: sums the ntiles cell-tile partials per particle in a
-// fixed order.  Above 64 tiles the sum runs in two levels (64 groups of consecutive tiles, then
-// the groups in order), so the partial buffer is read by ~64x more workgroups than particles
-// alone would give.
+// fixed order.  Above 16 tiles the sum runs in two levels, groups of ~sqrt(ntiles) consecutive tiles
+// and then the groups in order: the chains of loads are short and the partial buffer is read by that
+// many times more workgroups than particles alone would give (250 tiles x 10,000 particles: 16.5 + 4.3
+// us; 79 + 22 us for 1,000 tiles in 63 groups).
 static int reduce_particle_partials(tgrav_ctx* c, int64_t ntiles, int64_t np, const tg::Out& PO) {
   const double* src = c->bppart.as<double>();
   int64_t nt = ntiles;
-  if (ntiles > 64) {
-    const int G = 64;
-    const int per = (int)((ntiles + G - 1) / G);
+  if (ntiles > 16) {
+    const int per = (int)ceil(sqrt((double)ntiles));
     const int groups = (int)((ntiles + per - 1) / per);
     int rc = c->bpgrp.ensure((size_t)groups * 4 * np * sizeof(double));
     if (rc) return rc;
@@ -1688,9 +1688,21 @@ static int bidir_grid_shape(const tgrav_ctx* c, int mode, int64_t nblk, int64_t 
                             int* nsplit) {
   int64_t want = c->bnsplit[mode];
   if (want <= 0) {
-    const int64_t target = 8LL * 12 * c->num_cu;
-    want = std::min<int64_t>((target + nblk - 1) / nblk,
-                             std::min<int64_t>(12, std::max<int64_t>(1, np / 256)));
+    // A compute unit takes ceil(workgroups / units) turns of `t` particle tiles each; a turn costs about a
+    // tile more (its start, and the cell sums written and read again), and few turns cost up to 1/3
+    // (one wave per SIMD, and every wave ending at once).  2,000 stars x 120 blocks in FP64: 187 us at the
+    // 8 chunks this picks, 215 at 7, 223 at 13; 5,000 x 500: 1,141 at 8, 1,300 at 5, 1,194 at 12.
+    const int64_t ngrp = (nblk + TG_BIGRID_BLOCKS - 1) / TG_BIGRID_BLOCKS, tiles = (np + 63) / 64;
+    double best = 0.0;
+    for (int64_t n = 1; n <= std::min<int64_t>(tiles, 64); ++n) {
+      const int64_t t = (tiles + n - 1) / n, cnt = (tiles + t - 1) / t;
+      const double turns = (double)((ngrp * cnt + c->num_cu - 1) / c->num_cu);
+      const double cost = turns * (t + 0.75) * (1.0 + 0.3 / turns);
+      if (n == 1 || cost < best) {
+        best = cost;
+        want = cnt;
+      }
+    }
   }
   want = std::max<int64_t>(1, std::min<int64_t>(want, 65535));
   *chunk = (np + want - 1) / want;
@@ -1705,15 +1717,15 @@ static int bidir_grid_shape(const tgrav_ctx* c, int mode, int64_t nblk, int64_t 
 
 static void bidir_grid_kernel(tgrav_ctx* c, int mode, const tg::CellBlocks& C, int64_t np, int64_t chunk,
                               int nsplit, const tg::Out& o) {
-  const dim3 g((unsigned)C.nblk, (unsigned)nsplit);
+  const dim3 g((unsigned)((C.nblk + TG_BIGRID_BLOCKS - 1) / TG_BIGRID_BLOCKS), (unsigned)nsplit);
   if (mode == TGRAV_MIXED)
-    tg::k_bidir_grid<true><<<g, 64, 0, c->stream>>>(C, c->bp4.as<double4>(), c->bpe2.as<double>(), np,
-                                                   chunk, c->bstat.as<const double>(), o,
-                                                   c->bppart.as<double>());
+    tg::k_bidir_grid<true><<<g, 64 * TG_BIGRID_BLOCKS, 0, c->stream>>>(
+        C, c->bp4.as<double4>(), c->bpe2.as<double>(), np, chunk, c->bstat.as<const double>(), o,
+        c->bppart.as<double>());
   else
-    tg::k_bidir_grid<false><<<g, 64, 0, c->stream>>>(C, c->bp4.as<double4>(), c->bpe2.as<double>(), np,
-                                                    chunk, c->bstat.as<const double>(), o,
-                                                    c->bppart.as<double>());
+    tg::k_bidir_grid<false><<<g, 64 * TG_BIGRID_BLOCKS, 0, c->stream>>>(
+        C, c->bp4.as<double4>(), c->bpe2.as<double>(), np, chunk, c->bstat.as<const double>(), o,
+        c->bppart.as<double>());
 }
 
 // The fused pass with the cells as 8^3 block descriptors (k_bidir_grid).
@@ -1724,7 +1736,8 @@ static int bidir_grid_pass(tgrav_ctx* c, int mode, const tg::CellBlocks& C, int6
   int64_t chunk;
   int nsplit;
   if ((rc = bidir_grid_shape(c, mode, nblk, np, &chunk, &nsplit))) return rc;
-  if ((rc = c->bppart.ensure((size_t)nblk * 4 * np * sizeof(double)))) return rc;
+  const int64_t ngrp = (nblk + TG_BIGRID_BLOCKS - 1) / TG_BIGRID_BLOCKS;
+  if ((rc = c->bppart.ensure((size_t)ngrp * 4 * np * sizeof(double)))) return rc;
   tg::Out o = CO;
   if (nsplit > 1) {
     if ((rc = c->part.ensure((size_t)nsplit * 4 * nc * sizeof(double)))) return rc;
@@ -1740,7 +1753,7 @@ static int bidir_grid_pass(tgrav_ctx* c, int mode, const tg::CellBlocks& C, int6
   if (nsplit > 1) {
     if ((rc = reduce_chunks(c, c->part.as<double>(), nc, nsplit, nc, CO))) return rc;
   }
-  return reduce_particle_partials(c, nblk, np, PO);
+  return reduce_particle_partials(c, ngrp, np, PO);
 }
 
 int tgrav_bidirectional(tgrav_ctx* c, int64_t nc, const double* cx, const double* cy,
@@ -1871,7 +1884,7 @@ int tgrav_bidirectional(tgrav_ctx* c, int64_t nc, const double* cx, const double
     if (rc) return rc;
     if (cand) {
       if (nsplit_g > 1 && (rc = reduce_chunks(c, c->part.as<double>(), nc, nsplit_g, nc, CG))) return rc;
-      if ((rc = reduce_particle_partials(c, nblk, np, PG))) return rc;
+      if ((rc = reduce_particle_partials(c, (nblk + TG_BIGRID_BLOCKS - 1) / TG_BIGRID_BLOCKS, np, PG))) return rc;
     }
     if (generic) {
       if (nsplit > 1 && (rc = reduce_chunks(c, c->part.as<double>(), nc, nsplit, nc, CX))) return rc;
