@@ -679,3 +679,30 @@ def test_library_applies_the_tune_cache(c2):
     assert any(not np.array_equal(res[0][q], res[2][q]) for q in range(4))
     with pytest.raises(TgravError):
         GravityField("fp64", tune_cache=os.path.join(HERE, "conftest.py"))
+
+
+@pytest.mark.parametrize("ns", [1, 7, 8, 9, 63, 64, 65, 257, 2000])
+@pytest.mark.parametrize("variant", [0, 1, 2, 5])
+def test_fp64_slices_and_zero_pairs(ns, variant):
+    """The generic FP64 kernel at the edges of its groups of pairs, 64-source slices and 256-source
+    tiles, with unsoftened sources and targets that lie on some of them (those pairs add nothing)."""
+    rng = np.random.default_rng(ns)
+    S = [rng.normal(size=ns) for _ in range(3)] + [rng.uniform(0.5, 2.0, ns), np.zeros(ns)]
+    nt = 777
+    T = [rng.normal(size=nt) for _ in range(3)]
+    on = rng.choice(nt, min(ns, 40), replace=False)
+    at = rng.choice(ns, on.size, replace=False)
+    for q in range(3):
+        T[q][on] = S[q][at]
+    ref = oracle.eval_plummer(*S, *T, np.zeros(nt), W.G_PC_MSUN_KMS, mode=oracle.NEUMAIER)
+    with StellarGravityField("fp64") as f:
+        f.set_stars(*S)
+        for nsplit in (0, 1, 3):
+            f.set_config(variant=variant, nsplit=nsplit)
+            got = f.evaluate(None, *T)
+            # a coordinate of a close pair carries ~eps |x| / |d|: bounded against the sum of the terms
+            size = oracle.eval_plummer(*S, *T, np.full(nt, 1e-3), W.G_PC_MSUN_KMS)[3]
+            for q in range(4):
+                err = np.abs(got[q] - ref[q])
+                scale = np.abs(ref[q]) if q == 3 else np.sqrt(ref[0] ** 2 + ref[1] ** 2 + ref[2] ** 2)
+                assert np.all(err <= 1e-12 * (scale + np.abs(size))), (q, nsplit, err.max())

@@ -550,29 +550,50 @@ static int expand_sources(tgrav_ctx* c) {
   return 0;
 }
 
-// Launch shape: the variant's target tile and a source split that gives about
-// 4 workgroups per CU when the target set alone cannot fill the chip.
+// Chunks for nwg workgroups (per chunk) of at least one of `units` source units each, on `slots` workgroup
+// places of four waves (one wave per SIMD of a CU).  A place takes ceil(workgroups / slots) turns of a
+// chunk's units and `start` units' worth of start and of partial sums written and read again; k turns
+// cost a part few / k more (few waves per SIMD, and all of them ending at once).  For each count of turns
+// the most chunks that fit are tried.
+static int turns_split(int64_t nwg, int64_t units, double slots, double start, double few, int64_t most) {
+  const int64_t first = (int64_t)ceil((double)nwg / slots);
+  int64_t best_n = 1;
+  double best = 0.0;
+  for (int64_t k = first; k < first + 16; ++k) {
+    int64_t n = std::min<int64_t>((int64_t)((double)k * slots / (double)nwg), std::min<int64_t>(units, most));
+    n = std::max<int64_t>(1, std::min<int64_t>(n, 65535));
+    const int64_t t = (units + n - 1) / n;
+    n = (units + t - 1) / t;
+    const double turns = ceil((double)(nwg * n) / slots);
+    const double cost = (turns + few) * ((double)t + start);
+    if (k == first || cost < best) {
+      best = cost;
+      best_n = n;
+    }
+  }
+  return (int)best_n;
+}
+
+// Launch shape: the variant's target tile and the source split.
 static void choose_split(const tgrav_ctx* c, int mode, const Variant* v, int64_t nt, int64_t ns,
                          int64_t* ntiles, int* nsplit, int64_t* chunk, int force = -1) {
   const int64_t tile = (int64_t)v->k * v->nt;
   *ntiles = (nt + tile - 1) / tile;
   int want = force >= 0 ? force : c->nsplit[mode];
-  if (want <= 0) {
-    // About 8 rounds of workgroups at ~3 resident waves per SIMD, at least 4 source tiles a
-    // chunk (1 when that would leave fewer workgroups than CUs: small problems, where the
-    // partial sums are few), and at most 12 x 2^20 target-chunks of partial sums (32 B each).
-    const int64_t target_wg = 8LL * 12 * c->num_cu / (v->nt / 64);
-    int64_t s = (target_wg + *ntiles - 1) / *ntiles;
-    int64_t maxs = (ns + 4LL * v->ts - 1) / (4LL * v->ts);
-    if (*ntiles * maxs < c->num_cu) maxs = (ns + v->ts - 1) / v->ts;
-    const int64_t maxp = std::max<int64_t>(1, (12LL << 20) / std::max<int64_t>(nt, 1));
-    s = std::min<int64_t>(s, std::min<int64_t>(maxs, maxp));
-    want = (int)(s < 1 ? 1 : s);
-  }
+  // Whole source tiles, or 64-source slices where the tiles are too few for the CUs (FP64 only: a part tile
+  // costs only its own sources there, and the mixed tiles' FP32 sums stay what they are).  FP64, per call:
+  // 20,011 points x 5,003 sources 145 us at the 20 chunks this picks, 151 at 12, 161 at 6, 182 at 8;
+  // 3,000 x 300 74 us at 5 slices against 86 at one tile; 90,000 x 17,000 1,113 at 16, 1,131 at 40, 1,157
+  // at 20, 1,276 at 6.
+  const bool few = mode != TGRAV_MIXED && *ntiles * ((ns + v->ts - 1) / v->ts) < c->num_cu;
+  const int64_t unit = few ? 64 : v->ts;
+  if (want <= 0)                // at most 12 x 2^20 target-chunks of partial sums (32 B each)
+    want = turns_split(*ntiles, (ns + unit - 1) / unit, c->num_cu * (256.0 / v->nt), few ? 0.75 : 0.2, 0.8,
+                       std::max<int64_t>(1, (12LL << 20) / std::max<int64_t>(nt, 1)));
   if (want > 65535) want = 65535;
   int64_t ch = (ns + want - 1) / want;
-  ch = (ch + v->ts - 1) / v->ts * v->ts;
-  if (ch < v->ts) ch = v->ts;
+  ch = (ch + unit - 1) / unit * unit;
+  if (ch < unit) ch = unit;
   *chunk = ch;
   *nsplit = (int)((ns + ch - 1) / ch);
   if (*nsplit < 1) *nsplit = 1;
@@ -1688,21 +1709,10 @@ static int bidir_grid_shape(const tgrav_ctx* c, int mode, int64_t nblk, int64_t 
                             int* nsplit) {
   int64_t want = c->bnsplit[mode];
   if (want <= 0) {
-    // A compute unit takes ceil(workgroups / units) turns of `t` particle tiles each; a turn costs about a
-    // tile more (its start, and the cell sums written and read again), and few turns cost up to 1/3
-    // (one wave per SIMD, and every wave ending at once).  2,000 stars x 120 blocks in FP64: 187 us at the
-    // 8 chunks this picks, 215 at 7, 223 at 13; 5,000 x 500: 1,141 at 8, 1,300 at 5, 1,194 at 12.
-    const int64_t ngrp = (nblk + TG_BIGRID_BLOCKS - 1) / TG_BIGRID_BLOCKS, tiles = (np + 63) / 64;
-    double best = 0.0;
-    for (int64_t n = 1; n <= std::min<int64_t>(tiles, 64); ++n) {
-      const int64_t t = (tiles + n - 1) / n, cnt = (tiles + t - 1) / t;
-      const double turns = (double)((ngrp * cnt + c->num_cu - 1) / c->num_cu);
-      const double cost = turns * (t + 0.75) * (1.0 + 0.3 / turns);
-      if (n == 1 || cost < best) {
-        best = cost;
-        want = cnt;
-      }
-    }
+    // 2,000 stars x 120 blocks in FP64: 187 us at 8 chunks, 215 at 7, 223 at 13; 5,000 x 500: 1,141 at
+    // 8, 1,300 at 5, 1,194 at 12.
+    want = turns_split((nblk + TG_BIGRID_BLOCKS - 1) / TG_BIGRID_BLOCKS, (np + 63) / 64, c->num_cu, 0.75, 0.3,
+                       64);
   }
   want = std::max<int64_t>(1, std::min<int64_t>(want, 65535));
   *chunk = (np + want - 1) / want;
