@@ -244,3 +244,28 @@ def test_thin_launches_give_the_column_kernels_bits(mode, ns):
                 assert torch.equal(a[q], b[q]) and torch.equal(a[q], c[q])
                 assert torch.equal(a[q], phi if q == 3 else acc[q])
             assert torch.isfinite(a[3]).all()
+
+
+@pytest.mark.parametrize("mode", ["fp64", "mixed"])
+@pytest.mark.parametrize("nblk,nt", [(1, 1), (3, 127), (4, 128), (5, 129), (37, 300), (130, 640)])
+def test_block_source_chunks_match_oracle(mode, nblk, nt):
+    """The automatic source split of the block-source kernel, in whole rounds of a block per wave: part
+    rounds, part target tiles, and as many chunks as rounds; the unsplit evaluation gives the same sums
+    of the same blocks."""
+    rng = W.rng_for(nblk * 1000 + nt)
+    o = rng.uniform(-2.0, 1.5, (nblk, 3))
+    size = rng.choice([0.125, 0.25, 0.5], nblk)
+    x, y, z, dx = W.block_cell_centres(o, size)
+    m = 50.0 * np.exp(rng.normal(size=x.size)) * dx ** 3
+    st = W.star_cluster(rng, max(nt, 2), binary_frac=0.0)
+    T = [st[k][:nt] for k in "xyz"]
+    ref = oracle.eval_plummer(x, y, z, m, dx, *T, np.zeros(nt), G, mode=oracle.NEUMAIER, threads=8)
+    with GravityField(mode) as f:
+        for waves in (1, 2, 4):
+            f.set_column_waves(waves)
+            f.set_sources(x, y, z, m, dx)              # recognised as 8^3 blocks
+            for nsplit in (0, 1):
+                f.set_config(nsplit=nsplit)
+                s = _util.summary(f.evaluate(None, *T), ref)
+                print(mode, nblk, nt, waves, nsplit, s, flush=True)
+                check_bar(mode, s)

@@ -701,14 +701,15 @@ static int launch_grid(tgrav_ctx* c, int mode, const tg::Tgt& T, const tg::Out& 
 
 // Explicit targets against 8^3 source blocks: K targets per lane, tiles of 64 K targets, a
 // workgroup of W = col_waves waves per tile (splitting its source blocks), source blocks split
-// further over blockIdx.y.  K = 2 in the mixed kernel, 4 in the FP64 one: measured on c5's reverse
-// (plan) 87.7 against 90.2 ms (mixed, K = 2 against 4) and 204.8 against 206.4 ms (FP64, K = 4
-// against 2); the FP64 kernel holds each block's dz for its K targets and already needs 240 VGPRs.
+// further over blockIdx.y.  K = 2: in the mixed kernel c5's reverse (plan) took 87.7 ms against 90.2 with
+// 4; the FP64 kernel holds each block's dz for its K targets, 240 VGPRs and two waves per SIMD at K = 4:
+// 10,000 stars x 1,000 blocks 2,741 us per call with 2, 2,960 with 4, 2,781 with 1; 5,000 x 500 804 / 980 /
+// 788.
 #ifndef TG_GS_K_MIXED
 #define TG_GS_K_MIXED 2
 #endif
 #ifndef TG_GS_K_FP64
-#define TG_GS_K_FP64 4
+#define TG_GS_K_FP64 2
 #endif
 template <bool MIXED>
 static constexpr int gs_k() { return MIXED ? TG_GS_K_MIXED : TG_GS_K_FP64; }
@@ -722,13 +723,14 @@ static void gridsrc_shape(const tgrav_ctx* c, int mode, int64_t nt, int64_t nblk
   const int tuned = tuned_block_split(c, mode, "blocksrc", nt, nblk, W);
   if (tuned > 0) want = tuned;
   if (want <= 0) {
-    // ~12 waves resident per CU: aim at ~16 rounds of waves, with at least 4 source blocks per
-    // wave and chunk (1 when that leaves fewer waves than CUs).
-    const int64_t target = 16LL * 12 * c->num_cu;
-    const int64_t per = (target + *ntiles * W - 1) / (*ntiles * W);
-    int64_t w = std::min<int64_t>(per, std::max<int64_t>(1, nblk / (4 * W)));
-    if (*ntiles * W * w < c->num_cu) w = std::min<int64_t>(per, nblk);
-    want = (int)std::min<int64_t>(w, 65535);
+    // Whole rounds of a block per wave, by turns.  Per call at the chunks this picks, against ~16 rounds of
+    // waves of at least 4 blocks each: 5,000 stars x 500 blocks 714 / 802 us, x 1,000 1,309 / 1,434 (FP64),
+    // 3,000 x 300 212 / 288 (mixed), 10,000 x 2,000 1,954 / 1,956 (mixed).
+    const int64_t rounds = (nblk + W - 1) / W;
+    const int n = turns_split(*ntiles, rounds, c->num_cu * 4.0 / W, 0.1, 0.8, 65535);
+    *chunk = (rounds + n - 1) / n * W;
+    *nsplit = (int)((nblk + *chunk - 1) / *chunk);
+    return;
   }
   if (want > 65535) want = 65535;
   *chunk = (nblk + want - 1) / want;
@@ -800,16 +802,17 @@ static double sqrt_lt_threshold(double r) {
 
 // FLASH kernel, isolated, explicit targets against 8^3 source blocks: K targets per lane
 // (TG_FLASH_GS_K), 256 lanes, source blocks split over blockIdx.y (about 16 rounds of
-// workgroups, or the chunk count of tgrav_set_config).
+// workgroups, or the chunk count of tgrav_set_config).  K = 1: a wave's targets come near fewer blocks and
+// flag fewer cells than with 2, 10,000 stars x 1,000 blocks 2,786 us per call against 2,898.  (Chunks by turns
+// as the Plummer kernel's, longer ones, took 2,908: the blocks' near cells make workgroups uneven.)
 #ifndef TG_FLASH_GS_K
-#define TG_FLASH_GS_K 2
+#define TG_FLASH_GS_K 1
 #endif
 static void flash_gridsrc_shape(const tgrav_ctx* c, int64_t nt, int64_t nblk, int64_t* ntiles,
                                 int* nsplit, int64_t* chunk) {
   const int K = TG_FLASH_GS_K, NT = 256;
   *ntiles = (nt + K * NT - 1) / (K * NT);
-  // As the Plummer block-source kernel: about 16 rounds of workgroups, at least 4 blocks a chunk
-  // (1 when that leaves fewer workgroups than CUs).
+  // at least 4 blocks a chunk (1 when that leaves fewer workgroups than CUs)
   const int64_t target = 16LL * 3 * c->num_cu;
   const int64_t per = (target + *ntiles - 1) / *ntiles;
   int64_t want = std::min<int64_t>(per, std::max<int64_t>(1, nblk / 4));
