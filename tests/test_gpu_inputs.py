@@ -123,3 +123,37 @@ def test_block_sources_expand_where_needed(nblk):
                 torch.cuda.synchronize()
                 for q, r in zip(outs, b):
                     assert torch.equal(q, r)
+
+
+def test_scalar_softening_and_origin_layouts():
+    """Numbers for the softening (zero among them) and corners in any order or stride give the bits of
+    whole vectors; a number that is not finite is still refused."""
+    import torch
+    rng = np.random.default_rng(12)
+    st = [torch.as_tensor(rng.normal(size=200), device="cuda") for _ in range(3)]
+    m = torch.ones(200, dtype=torch.float64, device="cuda")
+    T = [torch.as_tensor(rng.normal(size=700), device="cuda") for _ in range(3)]
+    o = torch.as_tensor(rng.uniform(-2, 2, (5, 3)), device="cuda")
+    dx = torch.full((5,), 0.03, dtype=torch.float64, device="cuda")
+    wide = torch.zeros(5, 7, dtype=torch.float64, device="cuda")
+    wide[:, 1:4] = o
+    layouts = [o, o.t().contiguous().t(), wide[:, 1:4], wide[:, 1:], o.cpu(), o.flip(0).flip(0)]
+    with StellarGravityField("fp64") as f:
+        for eps in (0.0, 0, -0.0, 0.02, np.float64(0.02), np.array(0.02), torch.tensor(0.02, dtype=torch.float64)):
+            vec = torch.full((200,), float(eps), dtype=torch.float64, device="cuda")
+            f.set_sources(*st, m, eps)
+            got = f.evaluate(eps, *T)
+            f.set_sources(*st, m, vec)
+            ref = f.evaluate(torch.full((700,), float(eps), dtype=torch.float64, device="cuda"), *T)
+            for a, b in zip(got, ref):
+                assert torch.equal(a, b), eps
+        with pytest.raises(TgravError):
+            f.evaluate(float("nan"), *T)
+        ref = None
+        for q, lay in enumerate(layouts):
+            got = f.evaluate_blocks(lay, dx)
+            ref = ref or got
+            for a, b in zip(got, ref):
+                assert torch.equal(a, b), q
+        with pytest.raises(TgravError):
+            f.evaluate_blocks(o, dx[:4])

@@ -49,6 +49,14 @@ def _is_torch(a):
     return type(a).__module__.startswith("torch")
 
 
+def _columns(a, dev):
+    """Columns 0-2 of a[n, >= 3] as the rows of one contiguous tensor on dev; None: not a case for it."""
+    if dev is None or not _is_torch(a) or a.dim() != 2 or a.shape[1] < 3:
+        return None
+    import torch
+    return a[:, :3].to(device=dev, dtype=torch.float64).t().contiguous().unbind(0)
+
+
 class _Arrays:
     """Normalises a group of same-length inputs to one backend (numpy host / torch device)."""
 
@@ -65,11 +73,18 @@ class _Arrays:
         if self.dev is not None:
             import torch
             if not torch.is_tensor(a):
-                a = torch.as_tensor(np.asarray(a, dtype=np.float64), device=self.dev)
-            a = a.to(device=self.dev, dtype=torch.float64)
-            if a.dim() == 0:
-                a = a.expand(self.n)
-            a = a.contiguous().reshape(-1)
+                a = np.asarray(a, dtype=np.float64)
+                if a.ndim == 0:        # a number: filled in on the device (a copy of it waits for the GPU)
+                    if allow_none and a == 0.0:
+                        return None
+                    a = torch.full((self.n,), float(a), dtype=torch.float64, device=self.dev)
+                else:
+                    a = torch.as_tensor(a, device=self.dev)
+            if not (a.dtype is torch.float64 and a.dim() == 1 and a.device == self.dev and a.is_contiguous()):
+                a = a.to(device=self.dev, dtype=torch.float64)
+                if a.dim() == 0:
+                    a = a.expand(self.n)
+                a = a.contiguous().reshape(-1)
         else:
             a = np.asarray(a, dtype=np.float64)
             if a.ndim == 0:
@@ -80,6 +95,13 @@ class _Arrays:
                              f"{name} has length {a.shape[0]}, expected {self.n}")
         self.keep.append(a)
         return a
+
+    def columns(self, a, name):
+        """The three columns of a[n, 3], each contiguous; on the device one transposing copy."""
+        cols = _columns(a, self.dev)
+        if cols is None:
+            return [self.inp(a[:, q], name) for q in range(3)]
+        return [self.inp(c, name) for c in cols]
 
     def out(self):
         if self.dev is not None:
@@ -244,7 +266,7 @@ class GravityField:
         nblk = int(origin.shape[0])
         dev = _torch_device(origin, dx, mass, eps)
         A, B = _Arrays(nblk, dev), _Arrays(nblk * nb ** 3, dev)
-        o = [A.inp(origin[:, q], "origin") for q in range(3)]
+        o = A.columns(origin, "origin")
         d = A.inp(dx, "dx")
         e = A.inp(dx if eps is None else eps, "eps")
         m = B.inp(mass, "mass")
@@ -300,7 +322,7 @@ class GravityField:
         nblk = int(origin.shape[0])
         ncell = nblk * nb ** 3
         A = _Arrays(nblk, _torch_device(origin, dx, eps))
-        ox, oy, oz = (A.inp(origin[:, q], "origin") for q in range(3))
+        ox, oy, oz = A.columns(origin, "origin")
         d = A.inp(dx, "dx")
         e = A.inp(eps, "eps", allow_none=True)
         B = _Arrays(ncell, A.dev)
@@ -353,7 +375,7 @@ class GravityField:
         np_ = _length(px, py, pz, pm)
         dev = _torch_device(origin, dx, cm, ceps, px, py, pz, pm, pe)
         A, M, B = _Arrays(nblk, dev), _Arrays(nblk * 512, dev), _Arrays(np_, dev)
-        ba = [A.inp(origin[:, q], "origin") for q in range(3)] + [A.inp(dx, "dx")]
+        ba = A.columns(origin, "origin") + [A.inp(dx, "dx")]
         m = M.inp(cm, "cm")
         e = A.inp(ceps, "ceps", allow_none=True)
         pa = [B.inp(px, "px"), B.inp(py, "py"), B.inp(pz, "pz"), B.inp(pm, "pm"),

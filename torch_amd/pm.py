@@ -27,7 +27,7 @@ import numpy as np
 
 from . import _lib
 from ._lib import DEVICE, HOST
-from .field import GravityField, _is_torch
+from .field import GravityField, _columns, _is_torch
 
 
 class LeafBlocks:
@@ -80,8 +80,9 @@ class ParticleMesh(GravityField):
             if dev is not None:
                 import torch
                 t = a if torch.is_tensor(a) else torch.as_tensor(np.asarray(a), device=dev)
-                t = t.to(device=dev, dtype=torch.int64 if dtype == np.int64 else torch.float64)
-                t = t.contiguous().reshape(-1)
+                want = torch.int64 if dtype == np.int64 else torch.float64
+                if not (t.dtype is want and t.dim() == 1 and t.device == dev and t.is_contiguous()):
+                    t = t.to(device=dev, dtype=want).contiguous().reshape(-1)
             else:
                 t = np.ascontiguousarray(np.asarray(a, dtype=dtype)).reshape(-1)
             if t.shape[0] != n:
@@ -117,8 +118,8 @@ class ParticleMesh(GravityField):
 
     def _geom(self, blocks, dev):
         o = blocks.origin
-        o = [o[:, q] for q in range(3)]
-        return self._prep(dev, o + [blocks.size], blocks.nblk, ["origin x", "origin y", "origin z", "size"])
+        o = _columns(o, dev) or [o[:, q] for q in range(3)]
+        return self._prep(dev, [*o, blocks.size], blocks.nblk, ["origin x", "origin y", "origin z", "size"])
 
     # -- the reference's operations ---------------------------------------------------
     def update_grid_var(self, x, y, z, m, blk, blocks, rho=None, accumulate=False):
