@@ -371,3 +371,29 @@ def test_flash_errors_and_plummer_restored(c1):
         f.set_softening("spline", 0.2)
         with pytest.raises(TgravError):
             f.evaluate(st["eps"], st["x"], st["y"], st["z"])
+
+
+@pytest.mark.parametrize("quirks", [False, True])
+@pytest.mark.parametrize("far", [0.0, 5.0])
+def test_pair_keys_of_near_and_far_sets(quirks, far):
+    """Pairs grouped by separation with the short key (sets known to lie within two boxes of each other)
+    give the bits of the long key (not known: validation off), and the sums of the per-target walk; a
+    set shifted by whole boxes takes the long key."""
+    rng = W.rng_for(99)
+    L = np.array([2.0, 2.5, 3.0])
+    S = [rng.uniform(-0.5, 0.5, 70) * L[q] for q in range(3)]
+    T = [rng.uniform(-0.5, 0.5, 65) * L[q] + far * L[q] for q in range(3)]
+    T[0][:3], T[1][:3], T[2][:3] = S[0][:3] + far * L[0], S[1][:3] + far * L[1], S[2][:3] + far * L[2]
+    m = rng.uniform(0.5, 2.0, 70)
+    outs = {}
+    for name, validate, walk in (("known", True, False), ("unknown", False, False), ("walk", True, True)):
+        with GasGravityField("fp64", validate=validate) as f:
+            f.set_sources(*S, m, np.zeros(70))
+            f.set_softening("spline", 0.05, quirks=quirks)
+            f.set_periodic(tuple(L), nrep=6, per_target=walk)
+            outs[name] = f.evaluate(None, *T)
+    for a, b in zip(outs["known"], outs["unknown"]):
+        np.testing.assert_array_equal(a, b)
+    # sum of the terms' sizes: images of density 1 / (Lx Ly Lz) out to R = nrep min(L) add 4 pi R / V per mass
+    sa = W.G_PC_MSUN_KMS * m.sum() * 4 * np.pi * 6 * L.min() / L.prod()
+    check(outs["known"], outs["walk"], sa, np.abs(outs["walk"][3]).max())

@@ -348,8 +348,11 @@ __global__ __launch_bounds__(NT) void k_eval_flash(Tgt T, const double4* __restr
 // the pair's index t * ns + c; k_pair_reduce sums them per target with the masses.
 #define TG_PAIR_NREP 7                                   // rows of the table: (2 N + 1)^2 <= 225
 #ifndef TG_PAIR_BITS
-#define TG_PAIR_BITS 10      // separation key: bits per axis (bins of L / 2^(bits - 4), 8 boxes either way)
+#define TG_PAIR_BITS 10      // separation key: bits per axis (bins of L / 64, 8 boxes either way)
 #endif
+// Bits per axis where no separation exceeds 2 boxes (the same bins, and the same order of the pairs): the
+// radix sort takes 3 passes over 24 bits instead of 4 over 30.
+#define TG_PAIR_BITS_NEAR 8
 #define TG_PAIR_SLACK 1e-4   // image spacings; the square roots (v_rsq_f64, ~2^-24) are off by < 1e-5
 #define TG_PAIR_ROWS ((2 * TG_PAIR_NREP + 1) * (2 * TG_PAIR_NREP + 1))
 // nrep 8 .. 10: a table of (2 nrep + 1)^2 rows in dynamic LDS (<= 21.2 KB).  On c1's inputs it ran at
@@ -378,8 +381,8 @@ __device__ __forceinline__ unsigned int morton_spread10(unsigned int v) {
   return v;
 }
 
-__device__ __forceinline__ unsigned int sep_bin(double d, double ibin) {
-  const double h = (double)(1 << (TG_PAIR_BITS - 1));
+__device__ __forceinline__ unsigned int sep_bin(double d, double ibin, int bits) {
+  const double h = (double)(1 << (bits - 1));
   const double q = fmin(fmax(floor(d * ibin) + h, 0.0), 2.0 * h - 1.0);   // NaN -> 0
   return (unsigned int)q;
 }
@@ -388,7 +391,7 @@ __device__ __forceinline__ unsigned int sep_bin(double d, double ibin) {
 // separation, and i.
 __global__ __launch_bounds__(256) void k_pair_keys(Tgt T, int64_t t0, const double4* __restrict__ src4,
                                                    int64_t ns, int64_t npairs, double ibx, double iby,
-                                                   double ibz, unsigned int* __restrict__ keys,
+                                                   double ibz, int bits, unsigned int* __restrict__ keys,
                                                    unsigned int* __restrict__ idx) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= npairs) return;
@@ -396,8 +399,8 @@ __global__ __launch_bounds__(256) void k_pair_keys(Tgt T, int64_t t0, const doub
   double tx, ty, tz, e2;
   load_target(T, t0 + t, tx, ty, tz, e2);
   const double4 s = src4[c];
-  keys[i] = morton_spread10(sep_bin(tx - s.x, ibx)) | (morton_spread10(sep_bin(ty - s.y, iby)) << 1) |
-            (morton_spread10(sep_bin(tz - s.z, ibz)) << 2);
+  keys[i] = morton_spread10(sep_bin(tx - s.x, ibx, bits)) | (morton_spread10(sep_bin(ty - s.y, iby, bits)) << 1) |
+            (morton_spread10(sep_bin(tz - s.z, ibz, bits)) << 2);
   idx[i] = (unsigned int)i;
 }
 
@@ -424,6 +427,19 @@ __device__ __forceinline__ void sq_range(double lo, double hi, double c, double&
   const double a2 = a * a, b2 = b * b;
   mx = fmax(a2, b2);
   mn = (a <= 0.0 && b >= 0.0) ? 0.0 : fmin(a2, b2);
+}
+
+// kv = r2^(-3/2) without forming 1/sqrt(r2): with y the hardware estimate and e = 1 - r2 y^2 (~2^-23),
+// y^3 (1 + 3/2 e + 15/8 e^2), the next term below 2^-67.  One operation less than the cube of the refined
+// 1/sqrt(r2); its rounding error is smaller too (the cube takes three times that of the root).  With quirks
+// the walk needs no 1/sqrt(r2) per image: with the short key, 1,024 stars x 16^3 cells at nrep 6 2,138 ->
+// 2,048 us per call.
+__device__ __forceinline__ double rsqrt3_f64(double r2) {
+  const double y = __builtin_amdgcn_rsq(r2);
+  const double y2 = y * y;
+  const double e = fma(-r2, y2, 1.0);
+  const double c = y2 * y;
+  return fma(c, e * fma(e, 1.875, 1.5), c);
 }
 
 // One wave per workgroup: sorted pairs [64 w, 64 w + 64) of `idx`.  DYN = false: a static table of
@@ -523,7 +539,22 @@ __global__ __launch_bounds__(64) void k_eval_flash_pairs(Tgt T, int64_t t0, cons
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  double px = 0.0, py = 0.0, pz = 0.0, pp = 0.0;
+  // pp: the sum of pk; with quirks the pk of the last image, formed at the end from its r2 (r2l, or the
+  // softened pk in pp with r2l = 0): the walk then needs kv only
+  double px = 0.0, py = 0.0, pz = 0.0, pp = 0.0, r2l = 0.0;
+  auto add = [&](double r2, double dz, double& skv) {
+    double kv;
+    if (QUIRKS) {
+      kv = rsqrt3_f64(r2);
+      r2l = r2;
+    } else {
+      const double y = rsqrt_f64<0>(r2);
+      kv = (y * y) * y;
+      pp += y;
+    }
+    skv += kv;
+    pz = fma(kv, dz, pz);
+  };
   // the rows in (nx, ny) order (the quirk's potential is the last image's): the runs of rows without
   // a soft row, each followed by the soft row that ends it
   int r = 0;
@@ -550,14 +581,7 @@ __global__ __launch_bounds__(64) void k_eval_flash_pairs(Tgt T, int64_t t0, cons
           dz = dzi + fz * P.lz;
           r2 = xy + dz * dz;
         }
-        if (r2 <= cut) {
-          const double y = rsqrt_f64<0>(r2);
-          const double kv = (y * y) * y;
-          skv += kv;
-          pz = fma(kv, dz, pz);
-          if (QUIRKS) pp = y;
-          else pp += y;
-        }
+        if (r2 <= cut) add(r2, dz, skv);
       };
       double fz = R.zu0;
       for (int i = 0; i < nlo; ++i, fz += 1.0) tested(fz);
@@ -565,14 +589,7 @@ __global__ __launch_bounds__(64) void k_eval_flash_pairs(Tgt T, int64_t t0, cons
       // index step and an FMA (4% of the walk); the steps round dz to within nc/2 ulps of the row's
       // largest |dz|
       double dz = fma(fz, P.lz, dzi);
-      for (int i = 0; i < nc; ++i, dz += P.lz) {
-        const double y = rsqrt_f64<0>(fma(dz, dz, xy));
-        const double kv = (y * y) * y;
-        skv += kv;
-        pz = fma(kv, dz, pz);
-        if (QUIRKS) pp = y;
-        else pp += y;
-      }
+      for (int i = 0; i < nc; ++i, dz += P.lz) add(fma(dz, dz, xy), dz, skv);
       fz = R.zh0;
       for (int i = 0; i < nhi; ++i, fz += 1.0) tested(fz);
       px = fma(skv, dx, px);
@@ -602,14 +619,19 @@ __global__ __launch_bounds__(64) void k_eval_flash_pairs(Tgt T, int64_t t0, cons
           flash_pair(P, r2, kv, pk);
           skv += kv;
           pz = fma(kv, dz, pz);
-          if (QUIRKS) pp = pk;
-          else pp += pk;
+          if (QUIRKS) {
+            pp = pk;
+            r2l = 0.0;
+          } else {
+            pp += pk;
+          }
         }
       }
       px = fma(skv, dx, px);
       py = fma(skv, dy, py);
     }
   }
+  if (QUIRKS && r2l > 0.0) pp = rsqrt_f64<0>(r2l);
   if (valid) pairbuf[pr] = make_double4(px, py, pz, pp);
 }
 

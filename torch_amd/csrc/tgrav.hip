@@ -510,6 +510,7 @@ static int mixed_range_ok(const double* S, const double* T, const char* what) {
 // waited for), the kernels are then gated on the device.
 struct Known {
   bool valid = false, cols = false, srcb = false;
+  double span = 0.0;    // largest |coordinate| of the sources plus that of the targets
 };
 
 // One pass over the (device) targets of an evaluation and one wait: NaN/Inf, column structure and, mixed,
@@ -532,6 +533,7 @@ static int check_targets(tgrav_ctx* c, const tg::Tgt& T, int64_t nin, int mode, 
   k->valid = true;
   k->cols = !T.blocks && c->host_flag[HW_EVAL + tg::ST_WORDS] == 0ULL;
   k->srcb = c->ns > 0 && c->host_flag[HW_EVAL + 8 + tg::ST_WORDS] == 1ULL;
+  k->span = host_stats(c, HW_EVAL)[tg::ST_RMAX] + (c->ns > 0 ? host_stats(c, HW_EVAL + 8)[tg::ST_RMAX] : 0.0);
   return 0;
 }
 
@@ -837,13 +839,16 @@ static int flash_gridsrc_kernel(tgrav_ctx* c, const tg::Tgt& T, const tg::Out& o
 // targets of at most kMaxPairs pairs: pair keys, a stable radix sort of them, the grouped walk
 // (the timed kernel), the per-target sums.  ns <= kMaxPairs (the caller checks).
 static const int64_t kMaxPairs = 1LL << 25;
-static int launch_flash_pairs(tgrav_ctx* c, const tg::Tgt& T, const tg::Out& O, const tg::Flash& P) {
+static int launch_flash_pairs(tgrav_ctx* c, const tg::Tgt& T, const tg::Out& O, const tg::Flash& P,
+                              const Known& known) {
+  const int bits = known.valid && known.span <= 2.0 * std::min(P.lx, std::min(P.ly, P.lz)) ? TG_PAIR_BITS_NEAR
+                                                                                          : TG_PAIR_BITS;
   const int64_t nt = T.n, ns = c->ns;
   const int64_t tb = std::max<int64_t>(1, std::min<int64_t>(nt, kMaxPairs / ns)), nmax = tb * ns;
   size_t tmp = 0;
   HIPCHECK(hipcub::DeviceRadixSort::SortPairs(nullptr, tmp, (const unsigned int*)nullptr, (unsigned int*)nullptr,
                                              (const unsigned int*)nullptr, (unsigned int*)nullptr, (int)nmax, 0,
-                                             3 * TG_PAIR_BITS, c->stream));
+                                             3 * bits, c->stream));
   int rc;
   if ((rc = c->pkey.ensure((size_t)nmax * 2 * sizeof(unsigned int))) ||
       (rc = c->pidx.ensure((size_t)nmax * 2 * sizeof(unsigned int))) || (rc = c->ptmp.ensure(tmp)) ||
@@ -859,10 +864,10 @@ static int launch_flash_pairs(tgrav_ctx* c, const tg::Tgt& T, const tg::Out& O, 
   for (int64_t t0 = 0; t0 < nt; t0 += tb) {
     const int64_t nb = std::min<int64_t>(tb, nt - t0), np = nb * ns;
     tg::k_pair_keys<<<grid1(np, 256), 256, 0, c->stream>>>(T, t0, s4, ns, np, bins / P.lx, bins / P.ly,
-                                                           bins / P.lz, k0, i0);
+                                                           bins / P.lz, bits, k0, i0);
     LAUNCHCHECK("k_pair_keys");
     size_t tmp_b = tmp;
-    HIPCHECK(hipcub::DeviceRadixSort::SortPairs(c->ptmp.p, tmp_b, k0, k1, i0, i1, (int)np, 0, 3 * TG_PAIR_BITS,
+    HIPCHECK(hipcub::DeviceRadixSort::SortPairs(c->ptmp.p, tmp_b, k0, k1, i0, i1, (int)np, 0, 3 * bits,
                                                c->stream));
     rc = timed_launch(c, nb, ns, [&]() -> int {
       const unsigned int nw = (unsigned int)((np + 63) / 64);
@@ -915,7 +920,7 @@ static int launch_flash(tgrav_ctx* c, int mode, const tg::Tgt& T, const tg::Out&
   // arrays); tgrav_set_periodic(on = 2) keeps the per-target walk.
   if (per && c->periodic == 1 && c->nrep <= TG_PAIR_NREP_DYN && nt > 0 && ns > 0 && ns <= kMaxPairs &&
       nt <= 0x7fffffffLL)
-    return launch_flash_pairs(c, T, O, P);
+    return launch_flash_pairs(c, T, O, P, known);
   // Sources given as 8^3 blocks take the block-source kernel.  Explicit sources that may be
   // C-ordered 8^3 blocks (flagged on the device when they were set) launch it too, gated against
   // the generic kernel on that flag, as in the Plummer path.
