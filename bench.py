@@ -858,7 +858,7 @@ def main():
                                        "max_rel_acc_vs_grouped": float(ea_t.max()),
                                        "max_rel_pot_vs_grouped": float(ep_t.max())}
         line["roofline"] = {"bound": "valu", "kernel": ("k_eval_flash_pairs (pairs grouped by separation)"
-                                                          if periodic else "k_eval_flash_gridsrc<2,256>"),
+                                                          if periodic else "k_eval_flash_gridsrc<1,256>"),
                             "achieved": achieved, "peak": PEAK_FP64_TFLOPS, "unit": "TFLOP/s",
                             "frac": achieved / PEAK_FP64_TFLOPS, "traffic": None, "kernel_ms": r["kernel_ms"],
                             "flop_per_interaction": FLOP_PER_INTERACTION,

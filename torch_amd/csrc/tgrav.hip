@@ -706,20 +706,15 @@ static int launch_grid(tgrav_ctx* c, int mode, const tg::Tgt& T, const tg::Out& 
 // further over blockIdx.y.  K = 2: in the mixed kernel c5's reverse (plan) took 87.7 ms against 90.2 with
 // 4; the FP64 kernel holds each block's dz for its K targets, 240 VGPRs and two waves per SIMD at K = 4:
 // 10,000 stars x 1,000 blocks 2,741 us per call with 2, 2,960 with 4, 2,781 with 1; 5,000 x 500 804 / 980 /
-// 788.
-#ifndef TG_GS_K_MIXED
-#define TG_GS_K_MIXED 2
-#endif
-#ifndef TG_GS_K_FP64
-#define TG_GS_K_FP64 2
-#endif
+// 788.  The persistent FP64 kernel of the batch plans, whose workgroups never start anew, keeps K = 4 (the
+// same sums): c5's reverse 196.1 ms against 198.9 with 2.
+#define TG_GS_K 2
 template <bool MIXED>
-static constexpr int gs_k() { return MIXED ? TG_GS_K_MIXED : TG_GS_K_FP64; }
-static int gs_k_mode(int mode) { return mode == TGRAV_MIXED ? TG_GS_K_MIXED : TG_GS_K_FP64; }
+static constexpr int gs_plan_k() { return MIXED ? TG_GS_K : 4; }
 
 static void gridsrc_shape(const tgrav_ctx* c, int mode, int64_t nt, int64_t nblk, int64_t* ntiles,
                           int* nsplit, int64_t* chunk) {
-  const int K = gs_k_mode(mode), W = c->col_waves;
+  const int K = TG_GS_K, W = c->col_waves;
   *ntiles = (nt + K * 64 - 1) / (K * 64);
   int want = c->nsplit[mode];
   const int tuned = tuned_block_split(c, mode, "blocksrc", nt, nblk, W);
@@ -742,7 +737,7 @@ static void gridsrc_shape(const tgrav_ctx* c, int mode, int64_t nt, int64_t nblk
 template <bool MIXED, int W>
 static void gridsrc_kernel_w(tgrav_ctx* c, dim3 g, const tg::Tgt& T, const tg::Out& o, int64_t chunk,
                              int64_t nblk) {
-  tg::k_eval_gridsrc<gs_k<MIXED>(), W, MIXED><<<g, 64 * W, 0, c->stream>>>(
+  tg::k_eval_gridsrc<TG_GS_K, W, MIXED><<<g, 64 * W, 0, c->stream>>>(
       T, c->sax.as<double>(), c->sbe2.as<double>(), c->sms.as<double>(), nblk, chunk,
       c->stat.as<const double>(), o);
 }
@@ -1075,7 +1070,7 @@ static int launch_eval(tgrav_ctx* c, int mode, const tg::Tgt& T, const tg::Out& 
   // structure is decided on the device (k_check_cols sets a flag); both kernels are launched
   // and the flag lets exactly one of them (and its chunk reduction) run, so nothing waits for
   // the host.
-  // Likewise explicit sources that are C-ordered 8^3 blocks (k_detect_source_blocks flagged
+  // Likewise explicit sources that are C-ordered 8^3 blocks (k_pack_sources flagged
   // them when they were set) run the block-source kernel: gate value 2 wins over the column
   // test (1) and the generic kernel (0).
   // An evaluation that validated its inputs knows both answers already (Known) and launches the one
@@ -2427,7 +2422,7 @@ static void batch_free(tgrav_batch* b) {
   delete b;
 }
 
-// Block-source work items: tiles of K x 64 targets (gs_k), the eager kernel's shape.
+// Block-source work items: tiles of K x 64 targets (gs_plan_k).
 
 // The persistent column kernel for W waves per workgroup.
 static const void* batch_grid_kernel(bool mixed, int W) {
@@ -2438,16 +2433,16 @@ static const void* batch_grid_kernel(bool mixed, int W) {
 
 template <bool MIXED, int W>
 static void batch_gridsrc_launch(tgrav_batch* b, hipStream_t s) {
-  tg::k_batch_eval_gridsrc<gs_k<MIXED>(), W, MIXED><<<b->sgrid, 64 * W, 0, s>>>(
+  tg::k_batch_eval_gridsrc<gs_plan_k<MIXED>(), W, MIXED><<<b->sgrid, 64 * W, 0, s>>>(
       b->probs.as<tg::BProb>(), b->sitems.as<tg::BItem>(), b->sgoff.as<int>(), b->counter.as<unsigned int>() + 4,
       b->bms.as<double>(), b->sax.as<double>(), b->be2.as<double>(), b->stats.as<unsigned long long>(),
       b->part.as<double>());
 }
 
 static const void* batch_gridsrc_kernel(bool mixed, int W) {
-  if (W == 4) return mixed ? (const void*)tg::k_batch_eval_gridsrc<gs_k<true>(), 4, true> : (const void*)tg::k_batch_eval_gridsrc<gs_k<false>(), 4, false>;
-  if (W == 2) return mixed ? (const void*)tg::k_batch_eval_gridsrc<gs_k<true>(), 2, true> : (const void*)tg::k_batch_eval_gridsrc<gs_k<false>(), 2, false>;
-  return mixed ? (const void*)tg::k_batch_eval_gridsrc<gs_k<true>(), 1, true> : (const void*)tg::k_batch_eval_gridsrc<gs_k<false>(), 1, false>;
+  if (W == 4) return mixed ? (const void*)tg::k_batch_eval_gridsrc<gs_plan_k<true>(), 4, true> : (const void*)tg::k_batch_eval_gridsrc<gs_plan_k<false>(), 4, false>;
+  if (W == 2) return mixed ? (const void*)tg::k_batch_eval_gridsrc<gs_plan_k<true>(), 2, true> : (const void*)tg::k_batch_eval_gridsrc<gs_plan_k<false>(), 2, false>;
+  return mixed ? (const void*)tg::k_batch_eval_gridsrc<gs_plan_k<true>(), 1, true> : (const void*)tg::k_batch_eval_gridsrc<gs_plan_k<false>(), 1, false>;
 }
 
 template <bool MIXED, int W>
@@ -2626,7 +2621,7 @@ int tgrav_batch_create(tgrav_ctx* c, int32_t n, const tgrav_problem* pr, int mod
   const int CW = c->col_waves;
   const int gslots = occupancy(batch_grid_kernel(mode == TGRAV_MIXED, CW), 64 * CW, 0);
   const int sslots = occupancy(batch_gridsrc_kernel(mode == TGRAV_MIXED, CW), 64 * CW, 0);
-  const int64_t GT = (int64_t)gs_k_mode(mode) * 64;   // targets per block-source tile
+  const int64_t GT = (int64_t)(mode == TGRAV_MIXED ? gs_plan_k<true>() : gs_plan_k<false>()) * 64;   // targets per block-source tile
   // Form of each problem's work items.
   std::vector<int> form(n, tg::FORM_GENERIC);
   double tot_list[3] = {0.0, 0.0, 0.0};   // interactions on the generic, column, block-source lists
