@@ -181,3 +181,45 @@ def test_deposit_and_long_range_at_block_sizes(pm, nb, ng, nblk, crowd):
         with pytest.raises(TgravError):
             pm.update_grid_var(*a[:4], bad, B, rho=keep)
         np.testing.assert_array_equal(keep, base)
+
+
+# the deposit in LDS (at most 8,192 cells a block) and through memory
+@pytest.mark.parametrize("nb,ng", [(8, 2), (8, 4), (16, 4), (18, 2)])
+@pytest.mark.parametrize("bad", ["block_low", "block_high", "cloud"])
+def test_bad_particles_without_validation(nb, ng, bad):
+    """A particle whose block index or cloud is outside: with validation an error (and rho untouched), without
+    it the deposit is the other particles', and the forces are theirs with NaN for it."""
+    rng = W.rng_for(nb + ng)
+    nblk, n = 3, 200
+    B = LeafBlocks(rng.uniform(-2, 2, (nblk, 3)), rng.uniform(0.1, 1.0, nblk), nb=nb, ng=ng)
+    blk = rng.integers(0, nblk, n)
+    pos = B.origin[blk] + B.size[blk][:, None] * rng.uniform(0.0, 1.0, (n, 3))
+    m = rng.uniform(0.1, 2.0, n)
+    phi = rng.normal(size=B.ncell)
+    out = [0, 77, n - 1]
+    good = np.setdiff1d(np.arange(n), out)
+    b2, p2 = blk.copy(), pos.copy()
+    if bad == "cloud":
+        p2[out] = B.origin[blk[out]] - 1.5 * B.size[blk[out]][:, None] * ng
+    else:
+        b2[out] = -1 if bad == "block_low" else nblk
+    base = rng.uniform(-1, 1, B.ncell)
+    with ParticleMesh(validate=False) as f:
+        ref = f.update_grid_var(*[np.ascontiguousarray(pos[good, q]) for q in range(3)], m[good], blk[good], B)
+        got = f.update_grid_var(*[np.ascontiguousarray(p2[:, q]) for q in range(3)], m, b2, B)
+        # each cell's fixed point is scaled by the number of particles, so the sums may round differently
+        np.testing.assert_allclose(got, ref, rtol=1e-13, atol=0)
+        g = f.accel_list_of_blocks(phi, B)
+        want = f.map_mesh_to_particles(*[np.ascontiguousarray(pos[:, q]) for q in range(3)], blk, B, *g)
+        for a in (f.long_range_force(*[np.ascontiguousarray(p2[:, q]) for q in range(3)], b2, B, phi),
+                  f.map_mesh_to_particles(*[np.ascontiguousarray(p2[:, q]) for q in range(3)], b2, B, *g)):
+            for u, v in zip(a, want):
+                np.testing.assert_array_equal(u[good], v[good])
+                assert np.isnan(u[out]).all()
+    with ParticleMesh() as f:
+        keep = base.copy()
+        with pytest.raises(TgravError):
+            f.update_grid_var(*[np.ascontiguousarray(p2[:, q]) for q in range(3)], m, b2, B, rho=keep)
+        np.testing.assert_array_equal(keep, base)
+        with pytest.raises(TgravError):
+            f.long_range_force(*[np.ascontiguousarray(p2[:, q]) for q in range(3)], b2, B, phi)

@@ -109,7 +109,7 @@ __device__ __forceinline__ bool pm_corners(const PmBlocks& B, const double* x, c
 }
 
 // Pass 1: cmax[cell] = max |c| over the cell's contributions (as non-negative double bits,
-// whose unsigned order is the numeric order); a bad particle sets *err.
+// whose unsigned order is the numeric order); a bad particle sets *err (may be null).
 __global__ void k_pm_cell_max(int64_t np, const double* __restrict__ x, const double* __restrict__ y,
                               const double* __restrict__ z, const double* __restrict__ m,
                               const int64_t* __restrict__ blk, PmBlocks B, unsigned long long* cmax,
@@ -120,7 +120,7 @@ __global__ void k_pm_cell_max(int64_t np, const double* __restrict__ x, const do
     const unsigned long long bits = (unsigned long long)__double_as_longlong(fabs(c));
     if (bits) atomicMax(&cmax[idx], bits);
   });
-  if (!ok) atomicOr(err, 1ULL);
+  if (!ok && err) *err = 1ULL;   // every writer stores the same value
 }
 
 // Pass 2: accH / accL += the exact integer split c 2^S = H 2^32 + L of every contribution,
