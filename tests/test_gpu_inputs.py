@@ -157,3 +157,65 @@ def test_scalar_softening_and_origin_layouts():
                 assert torch.equal(a, b), q
         with pytest.raises(TgravError):
             f.evaluate_blocks(o, dx[:4])
+
+
+@pytest.mark.parametrize("nblk", [1, 40])
+def test_captured_block_sets_are_whole(nblk):
+    """A graph that sets block sources (and evaluates them block by block) sets them for every later call:
+    after each replay, eager calls that read the set cell by cell see the masses of that replay."""
+    rng = W.rng_for(nblk)
+    from torch_amd.blocks import block_centres
+    o, d = rng.uniform(-1, 1, (nblk, 3)), rng.uniform(0.02, 0.1, nblk)
+    x, y, z, dx = block_centres(o, d)
+    to, td = dev(rng.uniform(-1, 1, (2, 3)), np.full(2, 0.03))
+    t = dev(*rng.uniform(-1, 1, (3, 300)))
+    od, dd, m = dev(o, d, np.ones(x.size))
+    with GasGravityField("fp64", validate=False) as g, GasGravityField("fp64") as p:
+        g.set_blocks(od, dd, m)
+        g.evaluate(None, *t)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            g.set_blocks(od, dd, m)
+            outs = g.evaluate(None, *t)
+        for step in range(4):
+            m.copy_(dev(rng.uniform(0.5, 1, x.size))[0])
+            graph.replay()
+            torch.cuda.synchronize()
+            p.set_blocks(od, dd, m)
+            p.set_block_kernel(True)
+            for a, b in zip(outs, p.evaluate(None, *t)):
+                assert torch.equal(a, b)
+            for on in (True, False):                  # block targets, then the generic kernel
+                g.set_block_kernel(on)
+                p.set_block_kernel(on)
+                for a, b in zip(g.evaluate_blocks(to, td), p.evaluate_blocks(to, td)):
+                    assert torch.equal(a, b), (step, on)
+
+
+def test_block_set_read_on_two_streams():
+    """Block sources set on one stream and read cell by cell on two others that wait for it."""
+    rng = W.rng_for(5)
+    from torch_amd.blocks import block_centres
+    nblk = 600
+    o, d, m = dev(rng.uniform(-1, 1, (nblk, 3)), rng.uniform(0.02, 0.1, nblk), rng.uniform(0.5, 1, nblk * 512))
+    to, td = dev(rng.uniform(-1, 1, (1, 3)), np.full(1, 0.03))
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    with GasGravityField("fp64", validate=False) as g, GasGravityField("fp64") as p:
+        for f in (g, p):
+            f.set_config(nsplit=1)                    # no partial sums, which calls of a context share
+        p.set_blocks(o, d, m)
+        ref = p.evaluate_blocks(to, td)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(streams[0]):
+            g.set_blocks(o, d, m)
+            ready = streams[0].record_event()
+        got = []
+        for s in streams[1:]:
+            s.wait_event(ready)
+            with torch.cuda.stream(s):
+                got.append(g.evaluate_blocks(to, td))
+        torch.cuda.synchronize()
+        for a in got:
+            for u, v in zip(a, ref):
+                assert torch.equal(u, v)

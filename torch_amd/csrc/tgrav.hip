@@ -337,10 +337,6 @@ struct tgrav_ctx {
   DevBuf sbe2, sax, sms;     // source blocks: eps^2, cell-centre axes (24 per block), cell masses
   int64_t src_cols = 0;      // > 0: explicit sources that may be 8^3 blocks (scolflag says)
   DevBuf scolflag;
-  // Block sources: whether s4 / se2 hold the packed per-cell form of the current set, and whether any
-  // evaluation ever needed it (then every later set is expanded at once, so that a captured graph that
-  // reads it stays valid when the blocks are set again).
-  bool expanded = false, expand_used = false;
   DevBuf pub;                // slots and ticket of the one-pass reductions (tg::Publish)
   DevBuf in[12], outb[8], vel[3], part;      // staging for host pointers and scratch
   DevBuf colflag;            // explicit targets: 1 if they have 8^3 column structure
@@ -534,21 +530,6 @@ static int check_targets(tgrav_ctx* c, const tg::Tgt& T, int64_t nin, int mode, 
   k->cols = !T.blocks && c->host_flag[HW_EVAL + tg::ST_WORDS] == 0ULL;
   k->srcb = c->ns > 0 && c->host_flag[HW_EVAL + 8 + tg::ST_WORDS] == 1ULL;
   k->span = host_stats(c, HW_EVAL)[tg::ST_RMAX] + (c->ns > 0 ? host_stats(c, HW_EVAL + 8)[tg::ST_RMAX] : 0.0);
-  return 0;
-}
-
-// The packed per-cell form of block sources, for the kernels that read s4 / se2.
-static int expand_sources(tgrav_ctx* c) {
-  if (c->src_nblk == 0) return 0;
-  c->expand_used = true;
-  if (c->expanded) return 0;
-  tg::k_expand_source_blocks<<<grid1(c->src_nblk * 512, 256), 256, 0, c->stream>>>(
-      c->src_nblk, c->sbe2.as<double>(), c->sax.as<double>(), c->sms.as<double>(), c->s4.as<double4>(),
-      c->se2.as<double>());
-  LAUNCHCHECK("k_expand_source_blocks");
-  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  HIPCHECK(hipStreamIsCapturing(c->stream, &cap));
-  c->expanded = cap == hipStreamCaptureStatusNone;   // a captured launch has not run yet
   return 0;
 }
 
@@ -1054,8 +1035,6 @@ static int launch_eval(tgrav_ctx* c, int mode, const tg::Tgt& T, const tg::Out& 
     LAUNCHCHECK("k_fill");
     return 0;
   }
-  int rcx;
-  if (!(c->block_kernel && !T.blocks && !c->periodic) && (rcx = expand_sources(c))) return rcx;
   if (c->soft != TGRAV_SOFT_PLUMMER) return launch_flash(c, mode, T, O, known);
   if (T.blocks && T.nb == 8 && c->block_kernel) return launch_grid(c, mode, T, O);
   if (!T.blocks && c->src_nblk > 0 && c->block_kernel) return launch_gridsrc(c, mode, T, O);
@@ -1423,15 +1402,15 @@ int tgrav_set_source_blocks(tgrav_ctx* c, int64_t nblk, int nb, const double* ox
     return rc;
   const bool wait = kind == TGRAV_DEVICE && c->validate;
   tg::k_pack_source_blocks<<<pub_grid(n), 256, 0, c->stream>>>(
-      nblk, a[0], a[1], a[2], a[3], a[5], a[4], c->sbe2.as<double>(), c->sax.as<double>(), c->sms.as<double>(), wait,
+      nblk, a[0], a[1], a[2], a[3], a[5], a[4], c->s4.as<double4>(), c->se2.as<double>(), c->sbe2.as<double>(),
+      c->sax.as<double>(), c->sms.as<double>(), wait,
       publish_to(c, c->stat.as<unsigned long long>(), nullptr, wait ? HW_A : -1));
   LAUNCHCHECK("k_pack_source_blocks");
   if (kind == TGRAV_HOST || wait) HIPCHECK(hipStreamSynchronize(c->stream));
   if (wait && host_bad(c, HW_A)) return fail(TGRAV_ENONFINITE, "non-finite value in a source block array");
   c->ns = n;
   c->src_nblk = nblk;
-  c->expanded = false;
-  return c->expand_used ? expand_sources(c) : 0;
+  return 0;
 }
 
 // Shared body of tgrav_eval / tgrav_eval_kick / tgrav_eval_blocks.
