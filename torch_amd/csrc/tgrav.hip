@@ -58,12 +58,15 @@ static int fail(int code, const char* fmt, ...) {
 // One array per GPU the library runs on, held until the process ends.  Host code never passes
 // `scratch` itself (on the host it names a stand-in, not device memory): it passes the device
 // address hipGetSymbolAddress gave for the current device, kept per device in g_scratch_ptr.
+// Behind the TG_STATIC_SCRATCH_BYTES that calls share out: the slots and the ticket with which their packing
+// launch reduces its statistics, here so that a captured call needs nothing of its context at a replay.
 #define TG_STATIC_SCRATCH_BYTES (64ull << 20)
+#define TG_PUB_BYTES (TG_PUB_WG * 64 + 64)
 #define TG_MAX_DEVICES 64
 #ifndef TG_COL_WAVES
 #define TG_COL_WAVES 4   // default waves per column workgroup (tgrav_set_column_waves)
 #endif
-static __device__ __align__(256) unsigned char scratch[TG_STATIC_SCRATCH_BYTES];
+static __device__ __align__(256) unsigned char scratch[TG_STATIC_SCRATCH_BYTES + TG_PUB_BYTES];
 static std::mutex g_scratch_mu;
 static void* g_scratch_ptr[TG_MAX_DEVICES] = {};
 
@@ -464,15 +467,18 @@ static int reduce_chunks(tgrav_ctx* c, const double* part, int64_t pstride, int 
 }
 
 // Where a one-pass reduction writes: device words (stat, flag; may be null) and, with hw >= 0, the
-// pinned host words from hw on.
-static tg::Publish publish_to(tgrav_ctx* c, unsigned long long* stat, int* flag, int hw) {
+// pinned host words from hw on.  pub: TG_PUB_BYTES of device memory, slots and then the ticket.
+static tg::Publish publish_in(tgrav_ctx* c, void* pub, unsigned long long* stat, int* flag, int hw) {
   tg::Publish P{};
-  P.slots = c->pub.as<unsigned long long>();
+  P.slots = (unsigned long long*)pub;
   P.ticket = (unsigned int*)(P.slots + (size_t)TG_PUB_WG * 8);
   P.stat = stat;
   P.flag = flag;
   P.host = hw >= 0 ? c->host_flag + hw : nullptr;
   return P;
+}
+static tg::Publish publish_to(tgrav_ctx* c, unsigned long long* stat, int* flag, int hw) {
+  return publish_in(c, c->pub.p, stat, flag, hw);
 }
 static unsigned pub_grid(int64_t n) { return (unsigned)std::max<int64_t>(1, std::min<int64_t>(TG_PUB_WG, (n + 255) / 256)); }
 static bool host_bad(const tgrav_ctx* c, int hw) { return c->host_flag[hw + tg::ST_BAD] != 0ULL; }
@@ -1185,7 +1191,7 @@ int tgrav_create(tgrav_ctx** out, int device, const char* tune_cache_path) {
     return fail(TGRAV_EHIP, "tgrav_create: %s", hipGetErrorString(e));
   }
   int rs = scratch_init(device);
-  if (!rs) rs = c->pub.ensure((size_t)TG_PUB_WG * 64 + 64);
+  if (!rs) rs = c->pub.ensure(TG_PUB_BYTES);
   if (!rs && hipMemset(c->pub.p, 0, c->pub.cap) != hipSuccess) rs = fail(TGRAV_EHIP, "tgrav_create: hipMemset failed");
   if (rs) {
     c->pub.release();
@@ -1530,7 +1536,7 @@ int tgrav_eval_blocks(tgrav_ctx* c, int64_t nblk, int nb, const double* ox, cons
 // The allocation-free variant of tgrav_eval (device pointers, sources passed in): packed sources,
 // their statistics and the chunk partial sums live in the fixed per-device array `scratch`
 // (layout: ST_WORDS statistics words padded to 256 B, then {x,y,z,m} and eps^2 of the sources,
-// then the partials); the kernels and the launch shape are tgrav_eval's generic ones.
+// then the partials, and past those the packing launch's slots); the kernels and the launch shape are tgrav_eval's generic ones.
 int tgrav_eval_static(tgrav_ctx* c, int64_t ns, const double* sx, const double* sy, const double* sz,
                       const double* sm, const double* se, int64_t nt, const double* eps_t,
                       const double* x, const double* y, const double* z, double* ax, double* ay,
@@ -1582,8 +1588,13 @@ int tgrav_eval_static(tgrav_ctx* c, int64_t ns, const double* sx, const double* 
   tg::Out o = O;
   o.part = nsplit > 1 ? part : nullptr;
   o.pstride = nt;
+  // Slots and ticket of this array, and the ticket set here, not by the call before: calls that overlap
+  // against the rule spoil their own results only.
+  const tg::Publish pub = publish_in(c, base + TG_STATIC_SCRATCH_BYTES, stat, nullptr, -1);
+  tg::k_zero_u32<<<1, 64, 0, c->stream>>>(1, pub.ticket);
+  LAUNCHCHECK("k_zero_u32");
   tg::k_pack_sources<<<pub_grid(ns), 256, 0, c->stream>>>(ns, sx, sy, sz, sm, se, s4, se2, 0, nullptr, nullptr,
-                                                          nullptr, 0, publish_to(c, stat, nullptr, -1));
+                                                          nullptr, 0, pub);
   LAUNCHCHECK("k_pack_sources");
   v->fn(dim3((unsigned)ntiles, (unsigned)nsplit), dim3(v->nt), c->stream, T, s4, se2, ns, chunk,
         (const double*)stat, o);
