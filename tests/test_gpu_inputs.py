@@ -219,3 +219,52 @@ def test_block_set_read_on_two_streams():
         for a in got:
             for u, v in zip(a, ref):
                 assert torch.equal(u, v)
+
+
+def test_contexts_made_while_the_null_stream_is_busy():
+    """A context is ready for calls on its own stream when it is made, whatever the null stream still has to do."""
+    rng = W.rng_for(3)
+    st = [rng.uniform(-1, 1, 5000) for _ in range(3)] + [rng.uniform(0.1, 1, 5000), np.full(5000, 0.01)]
+    t = [rng.uniform(-1, 1, 400) for _ in range(3)]
+    ref = None
+    a = torch.ones(4096, 4096, device="cuda")
+    for step in range(4):
+        with torch.cuda.stream(torch.cuda.default_stream()):
+            for _ in range(200 if step else 0):
+                a = a * 1.0001
+        with StellarGravityField("fp64", validate=bool(step & 1)) as f:
+            f.set_stars(*st)                      # host arrays: the context's own stream
+            got = f.evaluate(None, *t)
+        torch.cuda.synchronize()
+        ref = ref or got
+        for u, v in zip(got, ref):
+            np.testing.assert_array_equal(u, v)
+
+
+def test_set_and_fused_pass_on_two_streams():
+    """A source set and the particles of a fused pass packed at once on two streams of one context: their
+    results, and those of the calls after them, are the ones of calls in a row."""
+    rng = W.rng_for(4)
+    n = 120000
+    S = dev(*rng.uniform(-1, 1, (3, n)), rng.uniform(0.1, 1, n), np.full(n, 0.01))
+    o, d, m = dev(rng.uniform(-1, 1, (1, 3)), np.full(1, 0.03), rng.uniform(0.5, 1, 512))
+    t = dev(*rng.uniform(-1, 1, (3, 40)))
+    P = [a[: n - 777].clone() for a in S]
+    with StellarGravityField("fp64", validate=False) as f:
+        f.set_bidir_config(nsplit=1)               # no chunk sums, which calls of a context share
+        f.set_sources(*S)
+        want = f.evaluate(None, *t), f.bidirectional_blocks(o, d, m, d, *P)
+        torch.cuda.synchronize()
+        one, two = torch.cuda.Stream(), torch.cuda.Stream()
+        for _ in range(20):
+            with torch.cuda.stream(one):
+                f.set_sources(*S)
+            with torch.cuda.stream(two):
+                fused = f.bidirectional_blocks(o, d, m, d, *P)
+        torch.cuda.synchronize()
+        got = f.evaluate(None, *t)
+        for u, v in zip(got, want[0]):
+            assert torch.equal(u, v)
+        for side in range(2):
+            for u, v in zip(fused[side], want[1][side]):
+                assert torch.equal(u, v)

@@ -340,7 +340,7 @@ struct tgrav_ctx {
   DevBuf sbe2, sax, sms;     // source blocks: eps^2, cell-centre axes (24 per block), cell masses
   int64_t src_cols = 0;      // > 0: explicit sources that may be 8^3 blocks (scolflag says)
   DevBuf scolflag;
-  DevBuf pub;                // slots and ticket of the one-pass reductions (tg::Publish)
+  DevBuf pub;                // slots and tickets of the one-pass reductions (tg::Publish)
   DevBuf in[12], outb[8], vel[3], part;      // staging for host pointers and scratch
   DevBuf colflag;            // explicit targets: 1 if they have 8^3 column structure
   DevBuf bp4, bpe2, bstat, bppart, bpgrp;   // fused passes: packed particles, partials
@@ -477,8 +477,11 @@ static tg::Publish publish_in(tgrav_ctx* c, void* pub, unsigned long long* stat,
   P.host = hw >= 0 ? c->host_flag + hw : nullptr;
   return P;
 }
-static tg::Publish publish_to(tgrav_ctx* c, unsigned long long* stat, int* flag, int hw) {
-  return publish_in(c, c->pub.p, stat, flag, hw);
+// Each kind of launch has slots and a ticket of its own in c->pub, as it has buffers of its own for what it
+// packs: the source set, the particles of the fused passes, and the checks (always waited for).
+enum { PUB_SOURCES, PUB_PARTICLES, PUB_CHECK, kNumPub };
+static tg::Publish publish_to(tgrav_ctx* c, int use, unsigned long long* stat, int* flag, int hw) {
+  return publish_in(c, c->pub.as<unsigned char>() + (size_t)use * TG_PUB_BYTES, stat, flag, hw);
 }
 static unsigned pub_grid(int64_t n) { return (unsigned)std::max<int64_t>(1, std::min<int64_t>(TG_PUB_WG, (n + 255) / 256)); }
 static bool host_bad(const tgrav_ctx* c, int hw) { return c->host_flag[hw + tg::ST_BAD] != 0ULL; }
@@ -518,7 +521,7 @@ struct Known {
 // One pass over the (device) targets of an evaluation and one wait: NaN/Inf, column structure and, mixed,
 // the range check against the source set.
 static int check_targets(tgrav_ctx* c, const tg::Tgt& T, int64_t nin, int mode, bool finite, Known* k) {
-  tg::Publish P = publish_to(c, nullptr, nullptr, HW_EVAL);
+  tg::Publish P = publish_to(c, PUB_CHECK, nullptr, nullptr, HW_EVAL);
   P.src_stat = c->ns > 0 ? c->stat.as<unsigned long long>() : nullptr;
   P.src_flag = c->src_cols > 0 ? c->scolflag.as<int>() : nullptr;
   if (T.blocks)
@@ -1191,8 +1194,12 @@ int tgrav_create(tgrav_ctx** out, int device, const char* tune_cache_path) {
     return fail(TGRAV_EHIP, "tgrav_create: %s", hipGetErrorString(e));
   }
   int rs = scratch_init(device);
-  if (!rs) rs = c->pub.ensure(TG_PUB_BYTES);
-  if (!rs && hipMemset(c->pub.p, 0, c->pub.cap) != hipSuccess) rs = fail(TGRAV_EHIP, "tgrav_create: hipMemset failed");
+  if (!rs) rs = c->pub.ensure(kNumPub * TG_PUB_BYTES);
+  // on the context's stream, which does not wait for the null stream, and waited for: calls may come on any
+  // stream
+  if (!rs && (hipMemsetAsync(c->pub.p, 0, c->pub.cap, c->own) != hipSuccess ||
+              hipStreamSynchronize(c->own) != hipSuccess))
+    rs = fail(TGRAV_EHIP, "tgrav_create: clearing the context's words failed");
   if (rs) {
     c->pub.release();
     (void)hipHostFree(c->host_flag);
@@ -1342,7 +1349,7 @@ int tgrav_set_sources(tgrav_ctx* c, int64_t n, const double* x, const double* y,
   tg::k_pack_sources<<<pub_grid(n), 256, 0, c->stream>>>(
       n, a[0], a[1], a[2], a[3], a[4], c->s4.as<double4>(), c->se2.as<double>(), nb8, c->sax.as<double>(),
       c->sbe2.as<double>(), c->sms.as<double>(), wait,
-      publish_to(c, c->stat.as<unsigned long long>(), nb8 > 0 ? c->scolflag.as<int>() : nullptr, wait ? HW_A : -1));
+      publish_to(c, PUB_SOURCES, c->stat.as<unsigned long long>(), nb8 > 0 ? c->scolflag.as<int>() : nullptr, wait ? HW_A : -1));
   LAUNCHCHECK("k_pack_sources");
   if (kind == TGRAV_DEVICE) {
     if (wait) {
@@ -1410,7 +1417,7 @@ int tgrav_set_source_blocks(tgrav_ctx* c, int64_t nblk, int nb, const double* ox
   tg::k_pack_source_blocks<<<pub_grid(n), 256, 0, c->stream>>>(
       nblk, a[0], a[1], a[2], a[3], a[5], a[4], c->s4.as<double4>(), c->se2.as<double>(), c->sbe2.as<double>(),
       c->sax.as<double>(), c->sms.as<double>(), wait,
-      publish_to(c, c->stat.as<unsigned long long>(), nullptr, wait ? HW_A : -1));
+      publish_to(c, PUB_SOURCES, c->stat.as<unsigned long long>(), nullptr, wait ? HW_A : -1));
   LAUNCHCHECK("k_pack_source_blocks");
   if (kind == TGRAV_HOST || wait) HIPCHECK(hipStreamSynchronize(c->stream));
   if (wait && host_bad(c, HW_A)) return fail(TGRAV_ENONFINITE, "non-finite value in a source block array");
@@ -1664,7 +1671,7 @@ static int bidir_pack_particles(tgrav_ctx* c, int64_t np, const double* const* p
     return rc;
   tg::k_pack_sources<<<pub_grid(np), 256, 0, c->stream>>>(
       np, pa[0], pa[1], pa[2], pa[3], pa[4], c->bp4.as<double4>(), c->bpe2.as<double>(), 0, nullptr, nullptr, nullptr,
-      hw >= 0, publish_to(c, c->bstat.as<unsigned long long>(), nullptr, hw));
+      hw >= 0, publish_to(c, PUB_PARTICLES, c->bstat.as<unsigned long long>(), nullptr, hw));
   LAUNCHCHECK("k_pack_sources");
   return 0;
 }
@@ -1681,7 +1688,7 @@ static int bidir_inputs(tgrav_ctx* c, int mode, int kind, int64_t n, const doubl
   int rc;
   if (wait && n > 0) {
     tg::k_check_set<<<pub_grid(std::max(n, nm)), 256, 0, c->stream>>>(n, x, y, z, dx, e, nm, m, dx ? 0 : 1,
-                                                                     publish_to(c, nullptr, nullptr, HW_A));
+                                                                     publish_to(c, PUB_CHECK, nullptr, nullptr, HW_A));
     LAUNCHCHECK("k_check_set");
   }
   if (np > 0 && (rc = bidir_pack_particles(c, np, pa, wait ? HW_B : -1))) return rc;
