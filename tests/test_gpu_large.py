@@ -140,3 +140,65 @@ def test_c5_explicit_arrays_equal_block_form(c5, fields):
             np.testing.assert_array_equal(p.cpu().numpy(), q)
         for p, q in zip(rev, fields["mixed"][1]):
             np.testing.assert_array_equal(p.cpu().numpy(), q)
+
+
+def test_mesh_deposit_of_many_small_blocks():
+    """More blocks than a launch of 512 lanes per block can take: a few particles, in the first, a middle and
+    the last block, deposit their mass there and nowhere else."""
+    import torch
+    from torch_amd import LeafBlocks, ParticleMesh
+    nblk, h = (1 << 23) + 3, 0.5
+    o = torch.zeros(nblk, 3, dtype=torch.float64, device="cuda")
+    o[:, 0] = torch.arange(nblk, dtype=torch.float64, device="cuda")
+    B = LeafBlocks(o, torch.full((nblk,), h, dtype=torch.float64, device="cuda"), nb=1, ng=1)
+    blk = torch.tensor([0, nblk // 2, nblk - 1, nblk - 1], device="cuda")
+    x, y, z = (o[blk, 0] + 0.5 * h), torch.full((4,), 0.5 * h, dtype=torch.float64, device="cuda"), \
+        torch.full((4,), 0.5 * h, dtype=torch.float64, device="cuda")
+    m = torch.tensor([1.0, 2.0, 3.0, 4.0], dtype=torch.float64, device="cuda")
+    with ParticleMesh() as f:
+        rho = f.update_grid_var(x, y, z, m, blk, B)
+    at = torch.nonzero(rho).reshape(-1).tolist()      # each particle at its cell's centre: that cell alone
+    assert at == [13, (nblk // 2) * 27 + 13, (nblk - 1) * 27 + 13]
+    assert rho[at].tolist() == [1.0 / h ** 3, 2.0 / h ** 3, 7.0 / h ** 3]
+    del rho, o, B
+    torch.cuda.empty_cache()
+
+
+def test_mesh_forces_of_very_many_particles():
+    """More particles than a launch of 8 lanes per particle can take (2^29): the first, the last and those
+    beside the launches' limits get the force of a call with them alone."""
+    import ctypes
+
+    import torch
+    from torch_amd import LeafBlocks, ParticleMesh, _lib
+    n = (1 << 29) + 5
+    at = torch.tensor([0, 1, (1 << 28) - 1, 1 << 28, (1 << 28) + 1, (1 << 29) - 1, 1 << 29, n - 1], device="cuda")
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    B = LeafBlocks(torch.zeros(2, 3, dtype=torch.float64, device="cuda"),
+                   torch.ones(2, dtype=torch.float64, device="cuda"), nb=8, ng=1)
+    phi = torch.randn(B.ncell, dtype=torch.float64, device="cuda", generator=gen)
+    some = torch.rand(3, at.numel(), dtype=torch.float64, device="cuda", generator=gen)
+    xs = []
+    for q in range(3):
+        a = torch.full((n,), 0.25, dtype=torch.float64, device="cuda")
+        a[at] = some[q]
+        xs.append(a)
+    blk = torch.zeros(n, dtype=torch.int64, device="cuda")
+    blk[at] = torch.arange(at.numel(), device="cuda") % 2
+    out = [torch.empty(n, dtype=torch.float64, device="cuda") for _ in range(3)]
+    p = lambda a: ctypes.c_void_p(a.data_ptr())  # noqa: E731
+    g = [B.origin[:, q].contiguous() for q in range(3)] + [B.size]
+    with ParticleMesh() as f:
+        want = f.long_range_force(*[a[at] for a in xs], blk[at], B, phi)
+        mid = f.long_range_force(*[a[7:8] for a in xs], blk[7:8], B, phi)
+        torch.cuda.synchronize()
+        rc = f.lib.tgrav_pm_long_range(f.handle, n, *[p(a) for a in xs], p(blk), 2, 8, 1, *[p(a) for a in g], p(phi),
+                                       *[p(a) for a in out], _lib.DEVICE)
+        _lib.check(rc, "tgrav_pm_long_range")
+        torch.cuda.synchronize()
+    for a, w, v in zip(out, want, mid):
+        assert torch.equal(a[at], w)
+        a[at] = v[0]
+        assert bool((a == v[0]).all())
+    del xs, blk, out, a
+    torch.cuda.empty_cache()

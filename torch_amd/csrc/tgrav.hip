@@ -2110,8 +2110,9 @@ int tgrav_pm_deposit(tgrav_ctx* c, int64_t np, const double* x, const double* y,
                  nblk, nb, ng, nb + 2 * ng, (int64_t)(nb + 2 * ng) * (nb + 2 * ng) * (nb + 2 * ng)};
   unsigned long long* err = pm_err_word(c);
   // Block by block in LDS where a guarded block is a few slices of it (k_pm_block); larger blocks would
-  // walk their particles once per slice and keep the passes over memory.
-  if (B.nc <= TG_PM_LDS_CELLS && nblk <= 0x7fffffffLL) {
+  // walk their particles once per slice and keep the passes over memory, and so do sets beyond what a
+  // launch of 512 lanes per block (2^32 lanes) and 32-bit counts of particles can hold.
+  if (B.nc <= TG_PM_LDS_CELLS && nblk <= 0xffffffffLL / 512 && np < 0xffffffffLL) {
     if ((rc = c->pm_cnt.ensure((size_t)(2 * nblk + 1) * 4)) || (rc = c->pm_idx.ensure((size_t)std::max<int64_t>(np, 1) * 8)))
       return rc;
     unsigned int *cnt = c->pm_cnt.as<unsigned int>(), *total = cnt + nblk, *off = total + 1;
@@ -2305,10 +2306,14 @@ int tgrav_pm_long_range(tgrav_ctx* c, int64_t np, const double* x, const double*
   tg::PmBlocks B{(const double*)dox, (const double*)doy, (const double*)doz, (const double*)dbs,
                  nblk, nb, ng, nb + 2 * ng, (int64_t)(nb + 2 * ng) * (nb + 2 * ng) * (nb + 2 * ng)};
   rc = timed_launch(c, np, ncell, [&]() -> int {
-    tg::k_pm_long_range<<<grid1(8 * np, 256), 256, 0, c->stream>>>(
-        np, (const double*)dx_, (const double*)dy_, (const double*)dz_, (const int64_t*)db_, B,
-        (const double*)dphi, (double*)dax, (double*)day, (double*)daz, err);
-    LAUNCHCHECK("k_pm_long_range");
+    const int64_t most = 1LL << 28;          // particles of a launch: 8 lanes each, below 2^32 lanes
+    for (int64_t p = 0; p < np; p += most) {
+      const int64_t n = std::min(most, np - p);
+      tg::k_pm_long_range<<<grid1(8 * n, 256), 256, 0, c->stream>>>(
+          n, (const double*)dx_ + p, (const double*)dy_ + p, (const double*)dz_ + p, (const int64_t*)db_ + p, B,
+          (const double*)dphi, (double*)dax + p, (double*)day + p, (double*)daz + p, err);
+      LAUNCHCHECK("k_pm_long_range");
+    }
     return 0;
   });
   if (rc) return rc;
