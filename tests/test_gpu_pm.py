@@ -223,3 +223,43 @@ def test_bad_particles_without_validation(nb, ng, bad):
         np.testing.assert_array_equal(keep, base)
         with pytest.raises(TgravError):
             f.long_range_force(*[np.ascontiguousarray(p2[:, q]) for q in range(3)], b2, B, phi)
+
+
+# particles in the crowded blocks: around the line to several workgroups, and whole and part stretches of them
+@pytest.mark.parametrize("counts", [(1023, 1024), (1025,), (1025, 2047, 2048, 2049), (5000, 1, 1024, 9000), (70000,)])
+@pytest.mark.parametrize("nb,ng,nblk", [(8, 1, 40), (8, 4, 40), (16, 2, 9), (8, 1, 16385)])
+def test_crowded_blocks(pm, counts, nb, ng, nblk):
+    """Some blocks with many particles among others with few: the oracle's densities, the same bits under a
+    permutation, without validation, and added to what is there."""
+    rng = W.rng_for(sum(counts) + nb + nblk)
+    B = LeafBlocks(rng.uniform(-2, 2, (nblk, 3)), rng.uniform(0.1, 1.0, nblk), nb=nb, ng=ng)
+    where = rng.choice(nblk, len(counts), replace=False)
+    blk = np.concatenate([np.full(n, b) for n, b in zip(counts, where)] + [rng.integers(0, nblk, 4100)])
+    rng.shuffle(blk)
+    h = (B.size / nb)[blk]
+    pos = B.origin[blk] + h[:, None] * rng.uniform(0.6 - ng, nb + ng - 0.6, (blk.size, 3))
+    m = rng.uniform(0.1, 2.0, blk.size) * 10.0 ** rng.uniform(-8, 8, blk.size)
+    a = [np.ascontiguousarray(pos[:, q]) for q in range(3)] + [m, blk]
+    got = pm.update_grid_var(*a, B)
+    ref = oracle.pm_deposit(*a, oblocks(B))
+    # the oracle's sequential sums of up to a few thousand positive terms a cell
+    np.testing.assert_allclose(got, ref, rtol=1e-12, atol=1e-300)
+    p = rng.permutation(blk.size)
+    np.testing.assert_array_equal(pm.update_grid_var(*[q[p] for q in a], B), got)
+    base = rng.uniform(-1, 1, B.ncell)
+    np.testing.assert_array_equal(pm.update_grid_var(*a, B, rho=base.copy(), accumulate=True), base + got)
+    with ParticleMesh(validate=False) as f:
+        np.testing.assert_array_equal(f.update_grid_var(*a, B), got)
+        few = [q[:37] for q in a]                      # nothing of the crowded call is left behind
+        np.testing.assert_array_equal(f.update_grid_var(*few, B), pm.update_grid_var(*few, B))
+
+
+@pytest.mark.parametrize("np_", [4095, 4096, 4097])
+def test_deposit_routes_agree(pm, np_):
+    """Few particles in very few cells go through memory, one more through LDS: the same densities."""
+    rng = W.rng_for(np_)
+    B = LeafBlocks(rng.uniform(-2, 2, (4, 3)), rng.uniform(0.1, 1.0, 4), nb=8, ng=4)
+    blk = rng.integers(0, 4, np_)
+    pos = B.origin[blk] + B.size[blk][:, None] * rng.uniform(0, 1, (np_, 3))
+    a = [np.ascontiguousarray(pos[:, q]) for q in range(3)] + [rng.uniform(0.1, 2.0, np_), blk]
+    np.testing.assert_allclose(pm.update_grid_var(*a, B), oracle.pm_deposit(*a, oblocks(B)), rtol=1e-13, atol=1e-300)

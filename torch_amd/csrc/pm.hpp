@@ -168,30 +168,65 @@ __global__ void k_zero_u32(int64_t n, unsigned int* a) {
 }
 
 // rank[p] = particle p's place among its block's particles (any order); ~0u and *err for a bad particle.
+// The lanes of a wave that share a block take one atomic, for up to 8 blocks.
 __global__ __launch_bounds__(256) void k_pm_bin(int64_t np, const double* __restrict__ x, const double* __restrict__ y,
                                                 const double* __restrict__ z, const int64_t* __restrict__ blk,
-                                                PmBlocks B, unsigned int* cnt, unsigned int* __restrict__ rank,
-                                                unsigned long long* err) {
+                                                PmBlocks B, unsigned int* cnt, int cs,
+                                                unsigned int* __restrict__ rank, unsigned long long* err) {
   const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (p >= np) return;
-  int64_t b;
+  const int lane = threadIdx.x & 63;
+  const bool in = p < np;        // every lane stays for the wave's shuffle
+  int64_t b = 0;
   double del, w[3][2];
   int c0[3];
-  if (!pm_particle(B, blk, p, x[p], y[p], z[p], b, del, c0, w)) {
-    rank[p] = ~0u;
-    if (err) *err = 1ULL;        // every writer stores the same value
-    return;
+  const bool ok = in && pm_particle(B, blk, p, x[p], y[p], z[p], b, del, c0, w);
+  const unsigned int mine = ok ? (unsigned int)b : ~0u;
+  unsigned long long left = __builtin_amdgcn_ballot_w64(ok);
+  int lead = lane;               // the lane that counts for this one, for how many, and this one's place
+  unsigned int n = 1u, r = 0u;
+  for (int i = 0; i < 8 && left; ++i) {
+    const int first = __builtin_ctzll(left);
+    const bool same = mine == (unsigned int)__builtin_amdgcn_readlane((int)mine, first);
+    const unsigned long long group = __builtin_amdgcn_ballot_w64(same);
+    if (same) {
+      lead = first;
+      n = (unsigned int)__builtin_popcountll(group);
+      r = (unsigned int)__builtin_popcountll(group & ((1ULL << lane) - 1ULL));
+    }
+    left &= ~group;
   }
-  rank[p] = atomicAdd(&cnt[b], 1u);
+  unsigned int base = 0u;
+  if (ok && lead == lane) base = atomicAdd(&cnt[b * cs], n);
+  base = (unsigned int)__shfl((int)base, lead);
+  if (!in) return;
+  rank[p] = ok ? base + r : ~0u;
+  if (!ok && err) *err = 1ULL;   // every writer stores the same value
 }
 
-// off[b]: a stretch of perm for each block with particles, in whatever order the workgroups come.
-__global__ __launch_bounds__(256) void k_pm_offsets(int64_t nblk, const unsigned int* __restrict__ cnt,
-                                                    unsigned int* __restrict__ off, unsigned int* total) {
+// Blocks of more than TG_PM_HEAVY particles ("heavy") are summed by several workgroups, TG_PM_SEG particles
+// each (k_pm_heavy_max, k_pm_heavy_sum), into words in memory: one workgroup takes ~30 ns per particle, and a
+// cluster inside one or a few blocks left the rest of the chip idle.  A call of 2,000 blocks of 16^3 cells with
+// all of its particles in one: 10,000 86 us (315 by one workgroup, 118 by the passes over memory), 100,000 91
+// (3,248; 311), 1,000,000 357 (33,000; 2,306); in eight of them 86 (75; 111), 92 (475; 212), 405 (4,645;
+// 1,288).  The line at 512: 1,000 particles in one block 86 us against 50; at 2,048: 2,000 in one 53 against 40.
+#define TG_PM_HEAVY 1024
+#define TG_PM_SEG 1024
+struct PmHeavy {
+  unsigned int block, seg;       // its first workgroup among all heavy blocks'
+  unsigned int off, cnt;         // its stretch of perm
+};
+
+// off[b]: a stretch of perm for each block with particles, in whatever order the workgroups come.  slot[b]: a
+// heavy block's place in `list` (ascending in seg: one counter, blocks in its high word and workgroups in its
+// low word, gives both), else ~0u; *any (may be null) is set if there is one.
+__global__ __launch_bounds__(256) void k_pm_offsets(int64_t nblk, const unsigned int* __restrict__ cnt, int cs,
+                                                    unsigned int* __restrict__ off, unsigned int* total,
+                                                    unsigned int* __restrict__ slot, unsigned long long* nheavy,
+                                                    PmHeavy* __restrict__ list, unsigned long long* any) {
   __shared__ unsigned int wsum[4], start;
   const int64_t b = (int64_t)blockIdx.x * 256 + threadIdx.x;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const unsigned int n = b < nblk ? cnt[b] : 0u;
+  const unsigned int n = b < nblk ? cnt[b * cs] : 0u;
   unsigned int s = n;            // inclusive sum over the wave
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
@@ -204,33 +239,167 @@ __global__ __launch_bounds__(256) void k_pm_offsets(int64_t nblk, const unsigned
   __syncthreads();
   unsigned int at = start + s - n;
   for (int q = 0; q < w; ++q) at += wsum[q];
-  if (b < nblk) off[b] = at;
+  if (b >= nblk) return;
+  off[b] = at;
+  unsigned int h = ~0u;
+  if (n > TG_PM_HEAVY) {
+    const unsigned long long r = atomicAdd(nheavy, (1ULL << 32) | ((n + TG_PM_SEG - 1) / TG_PM_SEG));
+    h = (unsigned int)(r >> 32);
+    list[h] = {(unsigned int)b, (unsigned int)r, at, n};
+    if (any) *any = 1ULL;        // every writer stores the same value
+  }
+  slot[b] = h;
 }
 
+// perm from the ranks; workgroups from nscatter on clear one heavy block's words each (block h's at h * nc).
 __global__ __launch_bounds__(256) void k_pm_scatter(int64_t np, const int64_t* __restrict__ blk,
                                                     const unsigned int* __restrict__ rank,
                                                     const unsigned int* __restrict__ off,
-                                                    unsigned int* __restrict__ perm) {
+                                                    unsigned int* __restrict__ perm, unsigned int nscatter,
+                                                    const unsigned long long* __restrict__ nheavy, int64_t nc,
+                                                    unsigned long long* M, unsigned long long* H,
+                                                    unsigned long long* L) {
+  if (blockIdx.x >= nscatter) {
+    const unsigned int h = blockIdx.x - nscatter;
+    if (h >= (unsigned int)(*nheavy >> 32)) return;
+    const int64_t at = (int64_t)h * nc;
+    for (int64_t i = at + threadIdx.x; i < at + nc; i += 256) M[i] = H[i] = L[i] = 0ULL;
+    return;
+  }
   const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (p >= np) return;
   const unsigned int r = rank[p];
   if (r != ~0u) perm[off[blk[p]] + r] = (unsigned int)p;
 }
 
-// One workgroup of 512 lanes per block.
+// The cells [lo, lo + len) of block b in LDS: M = max |c|, then H and L += the split of every contribution
+// of particles perm[q0 ... q1).  512 lanes.
+__device__ __forceinline__ void pm_lds_max(unsigned long long* M, int lo, int len, int64_t base, unsigned int q0,
+                                           unsigned int q1, const unsigned int* __restrict__ perm,
+                                           const double* __restrict__ x, const double* __restrict__ y,
+                                           const double* __restrict__ z, const double* __restrict__ m,
+                                           const int64_t* __restrict__ blk, const PmBlocks& B) {
+  for (unsigned int q = q0 + threadIdx.x; q < q1; q += 512)
+    pm_corners(B, x, y, z, m, blk, (int64_t)perm[q], [&](int64_t idx, double c) {
+      const int i = (int)(idx - base) - lo;
+      const unsigned long long bits = (unsigned long long)__double_as_longlong(fabs(c));
+      if (bits && i >= 0 && i < len) atomicMax(&M[i], bits);
+    });
+}
+__device__ __forceinline__ void pm_lds_sum(const unsigned long long* M, unsigned long long* H, unsigned long long* L,
+                                           int lo, int len, int64_t base, unsigned int q0, unsigned int q1,
+                                           const unsigned int* __restrict__ perm, int64_t np,
+                                           const double* __restrict__ x, const double* __restrict__ y,
+                                           const double* __restrict__ z, const double* __restrict__ m,
+                                           const int64_t* __restrict__ blk, const PmBlocks& B) {
+  for (unsigned int q = q0 + threadIdx.x; q < q1; q += 512)
+    pm_corners(B, x, y, z, m, blk, (int64_t)perm[q], [&](int64_t idx, double c) {
+      const int i = (int)(idx - base) - lo;
+      if (i < 0 || i >= len) return;
+      unsigned long long h, l;
+      pm_split(c, pm_scale(M[i], np), h, l);
+      atomicAdd(&H[i], h);
+      atomicAdd(&L[i], l);
+    });
+}
+
+// Workgroup i of the heavy blocks': its block's entry and its particles perm[q0 ... q1); false past the last.
+__device__ __forceinline__ bool pm_heavy_part(const unsigned long long* __restrict__ nheavy,
+                                              const PmHeavy* __restrict__ list, unsigned int i, unsigned int& h,
+                                              PmHeavy& e, unsigned int& q0, unsigned int& q1) {
+  const unsigned long long n = *nheavy;
+  if (i >= (unsigned int)n) return false;
+  unsigned int lo = 0, hi = (unsigned int)(n >> 32);   // list[lo].seg <= i < list[hi].seg
+  while (hi - lo > 1) {
+    const unsigned int mid = (lo + hi) / 2;
+    if (list[mid].seg <= i) lo = mid;
+    else hi = mid;
+  }
+  h = lo;
+  e = list[lo];
+  q0 = e.off + (i - e.seg) * TG_PM_SEG;
+  q1 = e.off + e.cnt;
+  if (q1 - q0 > TG_PM_SEG) q1 = q0 + TG_PM_SEG;
+  return true;
+}
+
+// blockIdx.x = workgroup of the heavy blocks', blockIdx.y = slice of TG_PM_LDS_SLICE cells.
+__global__ __launch_bounds__(512) void k_pm_heavy_max(const unsigned long long* __restrict__ nheavy,
+                                                      const PmHeavy* __restrict__ list, const double* __restrict__ x,
+                                                      const double* __restrict__ y, const double* __restrict__ z,
+                                                      const double* __restrict__ m, const int64_t* __restrict__ blk,
+                                                      PmBlocks B, const unsigned int* __restrict__ perm,
+                                                      unsigned long long* Mg) {
+  __shared__ unsigned long long M[TG_PM_LDS_SLICE];
+  unsigned int h, q0, q1;
+  PmHeavy e;
+  if (!pm_heavy_part(nheavy, list, blockIdx.x, h, e, q0, q1)) return;   // uniform over the workgroup
+  const int lo = (int)blockIdx.y * TG_PM_LDS_SLICE, nc = (int)B.nc;
+  const int len = nc - lo < TG_PM_LDS_SLICE ? nc - lo : TG_PM_LDS_SLICE;
+  for (int i = threadIdx.x; i < len; i += 512) M[i] = 0ULL;
+  __syncthreads();
+  pm_lds_max(M, lo, len, (int64_t)e.block * B.nc, q0, q1, perm, x, y, z, m, blk, B);
+  __syncthreads();
+  for (int i = threadIdx.x; i < len; i += 512)
+    if (M[i]) atomicMax(&Mg[(int64_t)h * B.nc + lo + i], M[i]);
+}
+
+__global__ __launch_bounds__(512) void k_pm_heavy_sum(const unsigned long long* __restrict__ nheavy,
+                                                      const PmHeavy* __restrict__ list, int64_t np,
+                                                      const double* __restrict__ x, const double* __restrict__ y,
+                                                      const double* __restrict__ z, const double* __restrict__ m,
+                                                      const int64_t* __restrict__ blk, PmBlocks B,
+                                                      const unsigned int* __restrict__ perm,
+                                                      const unsigned long long* __restrict__ Mg,
+                                                      unsigned long long* Hg, unsigned long long* Lg) {
+  __shared__ unsigned long long M[TG_PM_LDS_SLICE], H[TG_PM_LDS_SLICE], L[TG_PM_LDS_SLICE];
+  unsigned int h, q0, q1;
+  PmHeavy e;
+  if (!pm_heavy_part(nheavy, list, blockIdx.x, h, e, q0, q1)) return;
+  const int lo = (int)blockIdx.y * TG_PM_LDS_SLICE, nc = (int)B.nc;
+  const int len = nc - lo < TG_PM_LDS_SLICE ? nc - lo : TG_PM_LDS_SLICE;
+  const int64_t at = (int64_t)h * B.nc + lo;
+  for (int i = threadIdx.x; i < len; i += 512) {
+    M[i] = Mg[at + i];
+    H[i] = L[i] = 0ULL;
+  }
+  __syncthreads();
+  pm_lds_sum(M, H, L, lo, len, (int64_t)e.block * B.nc, q0, q1, perm, np, x, y, z, m, blk, B);
+  __syncthreads();
+  for (int i = threadIdx.x; i < len; i += 512)
+    if (M[i]) {
+      if (H[i]) atomicAdd(&Hg[at + i], H[i]);
+      if (L[i]) atomicAdd(&Lg[at + i], L[i]);
+    }
+}
+
+// One workgroup of 512 lanes per block; a heavy block's sums are in memory already (Mg, Hg, Lg).
 __global__ __launch_bounds__(512) void k_pm_block(int64_t np, const double* __restrict__ x,
                                                   const double* __restrict__ y, const double* __restrict__ z,
                                                   const double* __restrict__ m, const int64_t* __restrict__ blk,
-                                                  PmBlocks B, const unsigned int* __restrict__ cnt,
+                                                  PmBlocks B, const unsigned int* __restrict__ cnt, int cs,
                                                   const unsigned int* __restrict__ off,
                                                   const unsigned int* __restrict__ perm,
+                                                  const unsigned int* __restrict__ slot,
+                                                  const unsigned long long* __restrict__ Mg,
+                                                  const unsigned long long* __restrict__ Hg,
+                                                  const unsigned long long* __restrict__ Lg,
                                                   double* __restrict__ rho, int accumulate) {
   __shared__ unsigned long long M[TG_PM_LDS_SLICE], H[TG_PM_LDS_SLICE], L[TG_PM_LDS_SLICE];
   const int64_t b = blockIdx.x, base = b * B.nc;
   const int nc = (int)B.nc;
-  const unsigned int n = cnt[b];
-  if (n == 0u) {                 // uniform over the workgroup
+  const unsigned int n = cnt[b * cs];
+  if (n == 0u) {                 // uniform over the workgroup, as the next test
     for (int i = threadIdx.x; i < nc; i += 512) rho[base + i] = accumulate ? rho[base + i] + 0.0 : 0.0;
+    return;
+  }
+  if (n > TG_PM_HEAVY) {
+    const int64_t at = (int64_t)slot[b] * B.nc;
+    for (int i = threadIdx.x; i < nc; i += 512) {
+      const unsigned long long mx = Mg[at + i];
+      const double v = mx ? pm_value(Hg[at + i], Lg[at + i], pm_scale(mx, np)) : 0.0;
+      rho[base + i] = accumulate ? rho[base + i] + v : v;
+    }
     return;
   }
   const unsigned int o = off[b];
@@ -238,22 +407,9 @@ __global__ __launch_bounds__(512) void k_pm_block(int64_t np, const double* __re
     const int len = nc - lo < TG_PM_LDS_SLICE ? nc - lo : TG_PM_LDS_SLICE;
     for (int i = threadIdx.x; i < len; i += 512) M[i] = H[i] = L[i] = 0ULL;
     __syncthreads();
-    for (unsigned int q = threadIdx.x; q < n; q += 512)
-      pm_corners(B, x, y, z, m, blk, (int64_t)perm[o + q], [&](int64_t idx, double c) {
-        const int i = (int)(idx - base) - lo;
-        const unsigned long long bits = (unsigned long long)__double_as_longlong(fabs(c));
-        if (bits && i >= 0 && i < len) atomicMax(&M[i], bits);
-      });
+    pm_lds_max(M, lo, len, base, o, o + n, perm, x, y, z, m, blk, B);
     __syncthreads();
-    for (unsigned int q = threadIdx.x; q < n; q += 512)
-      pm_corners(B, x, y, z, m, blk, (int64_t)perm[o + q], [&](int64_t idx, double c) {
-        const int i = (int)(idx - base) - lo;
-        if (i < 0 || i >= len) return;
-        unsigned long long h, l;
-        pm_split(c, pm_scale(M[i], np), h, l);
-        atomicAdd(&H[i], h);
-        atomicAdd(&L[i], l);
-      });
+    pm_lds_sum(M, H, L, lo, len, base, o, o + n, perm, np, x, y, z, m, blk, B);
     __syncthreads();
     for (int i = threadIdx.x; i < len; i += 512) {
       const double v = M[i] ? pm_value(H[i], L[i], pm_scale(M[i], np)) : 0.0;

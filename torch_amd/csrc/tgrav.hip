@@ -382,7 +382,7 @@ static int tuned_block_split(const tgrav_ctx* c, int mode, const char* dir, int6
 static const int kTimingSlots = 256;
 // Pinned host words: results of the one-pass reductions (tg::Publish::host), by use.
 static const int kHostWords = 32;
-enum { HW_EVAL = 0, HW_A = 16, HW_B = 24, HW_FLAG = 31 };
+enum { HW_EVAL = 0, HW_A = 16, HW_B = 24, HW_HEAVY = 30, HW_FLAG = 31 };
 
 template <class F>
 static int timed_launch_on(tgrav_ctx* c, hipStream_t s, int64_t nt, int64_t ns, F launch) {
@@ -2110,28 +2110,56 @@ int tgrav_pm_deposit(tgrav_ctx* c, int64_t np, const double* x, const double* y,
                  nblk, nb, ng, nb + 2 * ng, (int64_t)(nb + 2 * ng) * (nb + 2 * ng) * (nb + 2 * ng)};
   unsigned long long* err = pm_err_word(c);
   // Block by block in LDS where a guarded block is a few slices of it (k_pm_block); larger blocks would
-  // walk their particles once per slice and keep the passes over memory, and so do sets beyond what a
-  // launch of 512 lanes per block (2^32 lanes) and 32-bit counts of particles can hold.
-  if (B.nc <= TG_PM_LDS_CELLS && nblk <= 0xffffffffLL / 512 && np < 0xffffffffLL) {
-    if ((rc = c->pm_cnt.ensure((size_t)(2 * nblk + 1) * 4)) || (rc = c->pm_idx.ensure((size_t)std::max<int64_t>(np, 1) * 8)))
+  // walk their particles once per slice and keep the passes over memory, and so do sets of more blocks than a
+  // launch of 512 lanes each (2^32 lanes) can take, and few particles in very few cells, where either way is
+  // launches and the passes are two or three fewer: 1 block of 16^3, 1,000 / 3,000 / 5,000 / 10,000 particles
+  // 18 / 21 / 27 / 42 us against 28 / 30 / 30 / 31; 4 blocks 23 / 22 / 24 / 33 against 21 / 32 / 31 / 32.
+  if (B.nc <= TG_PM_LDS_CELLS && nblk <= 0xffffffffLL / 512 && !(np <= 4096 && ncell <= 16384)) {
+    const int64_t hmax = std::min<int64_t>(nblk, np / (TG_PM_HEAVY + 1));   // heavy blocks there can be
+    const size_t hbytes = (size_t)std::max<int64_t>(hmax, 1) * B.nc * 8, list_bytes = (size_t)hmax * sizeof(tg::PmHeavy);
+    // A block's counter has 128 bytes to itself where that is little memory (2 MB): neighbouring counters are
+    // in one L2 channel, which takes their atomics one by one (1,000,000 particles in 64 blocks: 340 us against 1,380).
+    const int cs = nblk <= 16384 ? 32 : 1;
+    if ((rc = c->pm_cnt.ensure((size_t)((cs + 2) * nblk + 4) * 4)) ||
+        (rc = c->pm_idx.ensure(list_bytes + (size_t)std::max<int64_t>(np, 1) * 8)) ||
+        (hmax > 0 && ((rc = c->pm_acc[0].ensure(hbytes)) || (rc = c->pm_acc[1].ensure(hbytes)) ||
+                      (rc = c->pm_acc[2].ensure(hbytes)))))
       return rc;
-    unsigned int *cnt = c->pm_cnt.as<unsigned int>(), *total = cnt + nblk, *off = total + 1;
-    unsigned int *rank = c->pm_idx.as<unsigned int>(), *perm = rank + np;
-    tg::k_zero_u32<<<grid1(nblk + 1, 256), 256, 0, c->stream>>>(nblk + 1, cnt);
+    unsigned long long* nheavy = c->pm_cnt.as<unsigned long long>();
+    unsigned int *total = (unsigned int*)(nheavy + 1), *cnt = total + 2, *off = cnt + cs * nblk, *slot = off + nblk;
+    tg::PmHeavy* list = c->pm_idx.as<tg::PmHeavy>();
+    unsigned int *rank = (unsigned int*)(list + hmax), *perm = rank + np;
+    unsigned long long *H = c->pm_acc[0].as<unsigned long long>(), *L = c->pm_acc[1].as<unsigned long long>(),
+                       *M = c->pm_acc[2].as<unsigned long long>();
+    unsigned long long* any = c->validate && hmax > 0 ? c->host_flag + HW_HEAVY : nullptr;
+    if (any) *any = 0ULL;
+    tg::k_zero_u32<<<grid1(cs * nblk + 4, 256), 256, 0, c->stream>>>(cs * nblk + 4, (unsigned int*)nheavy);
     LAUNCHCHECK("k_zero_u32");
     if (np > 0) {
       tg::k_pm_bin<<<grid1(np, 256), 256, 0, c->stream>>>(np, (const double*)dx_, (const double*)dy_,
-                                                          (const double*)dz_, (const int64_t*)db_, B, cnt, rank, err);
+                                                          (const double*)dz_, (const int64_t*)db_, B, cnt, cs, rank, err);
       LAUNCHCHECK("k_pm_bin");
-      tg::k_pm_offsets<<<grid1(nblk, 256), 256, 0, c->stream>>>(nblk, cnt, off, total);
-      tg::k_pm_scatter<<<grid1(np, 256), 256, 0, c->stream>>>(np, (const int64_t*)db_, rank, off, perm);
+      tg::k_pm_offsets<<<grid1(nblk, 256), 256, 0, c->stream>>>(nblk, cnt, cs, off, total, slot, nheavy, list, any);
+      tg::k_pm_scatter<<<grid1(np, 256) + (unsigned)hmax, 256, 0, c->stream>>>(
+          np, (const int64_t*)db_, rank, off, perm, grid1(np, 256), nheavy, B.nc, M, H, L);
       LAUNCHCHECK("k_pm_scatter");
       if ((rc = pm_read_err(c, "tgrav_pm_deposit"))) return rc;
     }
     rc = timed_launch(c, np, ncell, [&]() -> int {
+      // validated calls have waited and know whether there is a heavy block
+      if (hmax > 0 && (!any || *any)) {
+        const dim3 g((unsigned)(np / TG_PM_SEG + hmax), (unsigned)((B.nc + TG_PM_LDS_SLICE - 1) / TG_PM_LDS_SLICE));
+        tg::k_pm_heavy_max<<<g, 512, 0, c->stream>>>(nheavy, list, (const double*)dx_, (const double*)dy_,
+                                                     (const double*)dz_, (const double*)dm_, (const int64_t*)db_, B,
+                                                     perm, M);
+        tg::k_pm_heavy_sum<<<g, 512, 0, c->stream>>>(nheavy, list, np, (const double*)dx_, (const double*)dy_,
+                                                     (const double*)dz_, (const double*)dm_, (const int64_t*)db_, B,
+                                                     perm, M, H, L);
+        LAUNCHCHECK("k_pm_heavy_sum");
+      }
       tg::k_pm_block<<<(unsigned)nblk, 512, 0, c->stream>>>(
           np, (const double*)dx_, (const double*)dy_, (const double*)dz_, (const double*)dm_, (const int64_t*)db_, B,
-          cnt, off, perm, (double*)drho, accumulate != 0);
+          cnt, cs, off, perm, slot, M, H, L, (double*)drho, accumulate != 0);
       LAUNCHCHECK("k_pm_block");
       return 0;
     });
