@@ -263,3 +263,31 @@ def test_deposit_routes_agree(pm, np_):
     pos = B.origin[blk] + B.size[blk][:, None] * rng.uniform(0, 1, (np_, 3))
     a = [np.ascontiguousarray(pos[:, q]) for q in range(3)] + [rng.uniform(0.1, 2.0, np_), blk]
     np.testing.assert_allclose(pm.update_grid_var(*a, B), oracle.pm_deposit(*a, oblocks(B)), rtol=1e-13, atol=1e-300)
+
+
+@pytest.mark.parametrize("nblk", [146, 147])              # 598,016 and 602,112 cells
+@pytest.mark.parametrize("n", [600_000, 600_001])
+def test_force_routes_agree(n, nblk):
+    """Many particles in few cells take the gradient first: on either side of the line the same bits, phi and
+    blocks as host arrays among the particles' tensors included."""
+    import torch
+    rng = W.rng_for(n + nblk)
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    o, size = rng.uniform(-2, 2, (nblk, 3)), rng.uniform(0.1, 1.0, nblk)
+    phi = rng.normal(size=nblk * 4096)
+    B = LeafBlocks(*[torch.as_tensor(a, device="cuda") for a in (o, size)], nb=8, ng=4)
+    blk = torch.randint(0, nblk, (n,), device="cuda", generator=gen)
+    x, y, z = [B.origin[:, q][blk] + B.size[blk] * torch.rand(n, dtype=torch.float64, device="cuda", generator=gen)
+               for q in range(3)]
+    f_d = torch.as_tensor(phi, device="cuda")
+    with ParticleMesh() as f:
+        got = f.long_range_force(x, y, z, blk, B, f_d)
+        mixed = f.long_range_force(x, y, z, blk, LeafBlocks(o, size, nb=8, ng=4), phi)
+        few = f.long_range_force(x[:1000], y[:1000], z[:1000], blk[:1000], B, f_d)
+        two = f.map_mesh_to_particles(x, y, z, blk, B, *f.accel_list_of_blocks(f_d, B))
+        bad = blk.clone()
+        bad[-1] = nblk
+        with pytest.raises(TgravError):
+            f.long_range_force(x, y, z, bad, B, f_d)
+    for a, m_, b, c in zip(got, mixed, two, few):
+        assert torch.equal(a, b) and torch.equal(m_, b) and torch.equal(a[:1000], c)

@@ -180,9 +180,15 @@ class ParticleMesh(GravityField):
     def long_range_force(self, x, y, z, blk, blocks, phi):
         """Particle accelerations from the block potential: finite differences, then CIC
         (Particles_longRangeForce.F90:70-97), formed at the corners of the particles' clouds only
-        (bit for bit accel_list_of_blocks, then map_mesh_to_particles)."""
+        (bit for bit accel_list_of_blocks, then map_mesh_to_particles).  Many particles in few cells
+        take those two calls: every cell's acceleration is then formed once instead of at each of its
+        particles, and read from cache.  Per call, one step / two: 600,000 particles in 262,144 cells
+        93 / 91 us, 4,000,000 362 / 254, in 4,096 cells 328 / 138; 400,000 in 409,600 cells 78 / 87;
+        4,000,000 in 737,280 cells 381 / 366, in 1,048,576 cells 399 / 487."""
         n = len(x) if not _is_torch(x) else int(x.shape[0])
         dev = self._dev(x, y, z, blk, phi, blocks.origin, blocks.size)
+        if dev is not None and n > 600_000 and blocks.ncell <= 600_000:
+            return self.map_mesh_to_particles(x, y, z, blk, blocks, *self.accel_list_of_blocks(phi, blocks))
         xs = self._prep(dev, [x, y, z], n, ["x", "y", "z"])
         b = self._prep(dev, [blk], n, ["blk"], dtype=np.int64)[0]
         g = self._geom(blocks, dev)
