@@ -268,3 +268,42 @@ def test_empty_sides():
         assert all(np.all(a == 0) for a in co) and all(a.size == 0 for a in po)
         co, po = f.bidirectional([], [], [], [], None, P["x"], P["y"], P["z"], P["m"], P["eps"])
         assert all(np.all(a == 0) for a in po)
+
+
+@pytest.mark.parametrize("explicit", [False, True])
+def test_size_limit_does_not_move_with_the_launch_shape(explicit):
+    """100 blocks with just fewer particles than 64 GiB of partial sums at one row per block and 12 chunks:
+    taken (the kernel's own chunks are more), and right; a few more particles are refused as blocks."""
+    import torch
+    from torch_amd import TgravError
+    from torch_amd.blocks import block_centres
+    nblk, n, few = 100, 21_462_336, 300
+    gen = torch.Generator(device="cuda").manual_seed(8)
+    r = lambda *s: torch.rand(*s, dtype=torch.float64, device="cuda", generator=gen)  # noqa: E731
+    o, d, cm = 3.0 * r(nblk, 3), 0.01 + 0.02 * r(nblk), 0.5 + r(nblk * 512)
+    big = 21_480_000
+    p = [3.0 * r(big) for _ in range(3)] + [1e-6 * (0.5 + r(big)), torch.full((big,), 0.01, dtype=torch.float64, device="cuda")]
+    x, y, z = [torch.as_tensor(a, device="cuda") for a in block_centres(o.cpu().numpy(), d.cpu().numpy())[:3]]
+    e = d.repeat_interleave(512)
+    with GravityField("mixed", G=1.0) as f:
+        q = [a[:n].contiguous() for a in p]
+        if explicit:
+            cells, parts = f.bidirectional(x, y, z, cm, e, *q)
+        else:
+            cells, parts = f.bidirectional_blocks(o, d, cm, d, *q)
+            with pytest.raises(TgravError) as err:
+                f.bidirectional_blocks(o, d, cm, d, *p)
+            assert err.value.code == _lib.ELIMIT
+    at = torch.randint(0, n, (few,), device="cuda", generator=gen)
+    with GravityField("fp64", G=1.0) as f:
+        f.set_sources(x, y, z, cm, e)
+        ref = f.evaluate(q[4][at], *[a[at] for a in q[:3]])
+        s = _util.summary([a[at].cpu().numpy() for a in parts], [a.cpu().numpy() for a in ref])
+        assert s["acc_median"] <= 1e-6 and s["acc_max"] <= 1e-4, s
+        f.set_sources(*q)
+        c = torch.arange(0, nblk * 512, 171, device="cuda")
+        ref = f.evaluate(e[c], x[c], y[c], z[c])
+        s = _util.summary([a[c].cpu().numpy() for a in cells], [a.cpu().numpy() for a in ref])
+        assert s["acc_median"] <= 1e-6 and s["acc_max"] <= 1e-4, s
+    del p, q, cells, parts
+    torch.cuda.empty_cache()

@@ -264,9 +264,9 @@ __global__ void k_bidir_reduce(const double* __restrict__ ppart, int ntiles, int
 }
 
 // ------------------------------------------------------------- 8^3 cell blocks ----
-// The fused pass with the cells handed over as 8^3 leaf blocks: one 64-lane workgroup per
-// block, lane l owns the cell column (i, j) = (l / 8, l % 8) and its 8 cells along z (as
-// k_eval_grid).  Particles stream through LDS 64 at a time and are walked in the rotated
+// The fused pass with the cells handed over as 8^3 leaf blocks: one wave per block
+// (TG_BIGRID_BLOCKS to a workgroup), lane l owns the cell column (i, j) = (l / 8, l % 8) and its 8
+// cells along z (as k_eval_grid).  Particles stream through LDS 64 at a time and are walked in the rotated
 // order of k_bidir (lane l takes particle (l + s) mod 64 at step s), so each lane meets one
 // particle per step with its whole column: dx, dy and dx^2 + dy^2 + eps^2 are formed once
 // per (column, particle), the cell side accumulates in registers, and the particle side sums

@@ -1703,31 +1703,48 @@ static int bidir_inputs(tgrav_ctx* c, int mode, int kind, int64_t n, const doubl
   return 0;
 }
 
-// Launch shape of the block-column fused kernel: particle chunks over blockIdx.y, about 8 rounds
-// of one-wave workgroups, at most 12 chunks, at least 4 particle tiles a chunk.
+// Workgroups of the block-column fused kernel, and rows of particle partials they write.
+static int64_t bidir_groups(int64_t nblk) { return (nblk + TG_BIGRID_BLOCKS - 1) / TG_BIGRID_BLOCKS; }
+
+// Partial sums a fused pass by blocks is counted at for its size limit: a row per block and at most 12
+// chunks of at least 4 particle tiles, more than the kernel's groups of blocks write, so which sizes are
+// refused does not move with the launch shape.  *chunks: that many chunks.
+static double bidir_grid_bytes(const tgrav_ctx* c, int mode, int64_t nblk, int64_t np, int64_t* chunks) {
+  int64_t want = c->bnsplit[mode];
+  if (want <= 0)
+    want = std::min<int64_t>((8LL * 12 * c->num_cu + nblk - 1) / nblk,
+                             std::min<int64_t>(12, std::max<int64_t>(1, np / 256)));
+  want = std::max<int64_t>(1, std::min<int64_t>(want, 65535));
+  const int64_t chunk = ((np + want - 1) / want + 63) / 64 * 64;
+  *chunks = (np + chunk - 1) / chunk;
+  return (double)nblk * 4 * np * 8 + (*chunks > 1 ? (double)*chunks * 4 * nblk * 512 * 8 : 0.0);
+}
+static const double kFusedLimit = 64.0 * (1ULL << 30);
+
+// Launch shape of the block-column fused kernel: particle chunks over blockIdx.y, by turns of its workgroups
+// of TG_BIGRID_BLOCKS waves, at most 64 chunks of at least one particle tile.
 static int bidir_grid_shape(const tgrav_ctx* c, int mode, int64_t nblk, int64_t np, int64_t* chunk,
                             int* nsplit) {
-  int64_t want = c->bnsplit[mode];
+  int64_t want = c->bnsplit[mode], counted;
+  if (bidir_grid_bytes(c, mode, nblk, np, &counted) > kFusedLimit)
+    return fail(TGRAV_ELIMIT, "%lld blocks x %lld particles are more than a fused pass takes (a row of partial "
+                "sums per block within 64 GiB); evaluate the two directions separately", (long long)nblk,
+                (long long)np);
   if (want <= 0) {
     // 2,000 stars x 120 blocks in FP64: 187 us at 8 chunks, 215 at 7, 223 at 13; 5,000 x 500: 1,141 at
     // 8, 1,300 at 5, 1,194 at 12.
-    want = turns_split((nblk + TG_BIGRID_BLOCKS - 1) / TG_BIGRID_BLOCKS, (np + 63) / 64, c->num_cu, 0.75, 0.3,
-                       64);
+    want = turns_split(bidir_groups(nblk), (np + 63) / 64, c->num_cu, 0.75, 0.3, 64);
   }
   want = std::max<int64_t>(1, std::min<int64_t>(want, 65535));
   *chunk = (np + want - 1) / want;
   *chunk = (*chunk + 63) / 64 * 64;
   *nsplit = (int)((np + *chunk - 1) / *chunk);
-  const double part_bytes = (double)nblk * 4 * np * 8 + (*nsplit > 1 ? (double)*nsplit * 4 * nblk * 512 * 8 : 0.0);
-  if (part_bytes > 64.0 * (1ULL << 30))
-    return fail(TGRAV_ELIMIT, "fused pass would need %.1f GiB of partial sums; evaluate the two "
-                "directions separately", part_bytes / (1ULL << 30));
   return 0;
 }
 
 static void bidir_grid_kernel(tgrav_ctx* c, int mode, const tg::CellBlocks& C, int64_t np, int64_t chunk,
                               int nsplit, const tg::Out& o) {
-  const dim3 g((unsigned)((C.nblk + TG_BIGRID_BLOCKS - 1) / TG_BIGRID_BLOCKS), (unsigned)nsplit);
+  const dim3 g((unsigned)bidir_groups(C.nblk), (unsigned)nsplit);
   if (mode == TGRAV_MIXED)
     tg::k_bidir_grid<true><<<g, 64 * TG_BIGRID_BLOCKS, 0, c->stream>>>(
         C, c->bp4.as<double4>(), c->bpe2.as<double>(), np, chunk, c->bstat.as<const double>(), o,
@@ -1746,7 +1763,7 @@ static int bidir_grid_pass(tgrav_ctx* c, int mode, const tg::CellBlocks& C, int6
   int64_t chunk;
   int nsplit;
   if ((rc = bidir_grid_shape(c, mode, nblk, np, &chunk, &nsplit))) return rc;
-  const int64_t ngrp = (nblk + TG_BIGRID_BLOCKS - 1) / TG_BIGRID_BLOCKS;
+  const int64_t ngrp = bidir_groups(nblk);
   if ((rc = c->bppart.ensure((size_t)ngrp * 4 * np * sizeof(double)))) return rc;
   tg::Out o = CO;
   if (nsplit > 1) {
@@ -1842,7 +1859,7 @@ int tgrav_bidirectional(tgrav_ctx* c, int64_t nc, const double* cx, const double
     chunk = (chunk + v.nt - 1) / v.nt * v.nt;
     const int nsplit = (int)((np + chunk - 1) / chunk);
     const double part_bytes = (double)ntiles * 4 * np * 8 + (nsplit > 1 ? (double)nsplit * 4 * nc * 8 : 0.0);
-    if (part_bytes > 64.0 * (1ULL << 30))
+    if (part_bytes > kFusedLimit)
       return fail(TGRAV_ELIMIT, "fused pass would need %.1f GiB of partial sums; evaluate the two "
                   "directions separately", part_bytes / (1ULL << 30));
     const int64_t nblk = nc / 512;
@@ -1851,16 +1868,18 @@ int tgrav_bidirectional(tgrav_ctx* c, int64_t nc, const double* cx, const double
     // The size limit is the generic pipeline's; a column pipeline that would exceed it is simply
     // not offered (the generic one then runs whatever the structure).
     if (cand && bidir_grid_shape(c, mode, nblk, np, &chunk_g, &nsplit_g) != 0) cand = false;
-    if (cand && ((double)std::max<int64_t>(ntiles, nblk) * 4 * np * 8 +
-                 (std::max(nsplit, nsplit_g) > 1 ? (double)std::max(nsplit, nsplit_g) * 4 * nc * 8 : 0.0)) >
-                    64.0 * (1ULL << 30))
+    int64_t counted = 1;
+    if (cand) bidir_grid_bytes(c, mode, nblk, np, &counted);
+    counted = std::max<int64_t>(counted, nsplit);
+    if (cand && (double)std::max<int64_t>(ntiles, nblk) * 4 * np * 8 +
+                        (counted > 1 ? (double)counted * 4 * nc * 8 : 0.0) > kFusedLimit)
       cand = false;
-    const int64_t prows = std::max<int64_t>(ntiles, cand ? nblk : 0);
+    const bool both = cand && known_cols < 0, generic = !cand || both;
+    const int64_t prows = std::max<int64_t>(generic ? ntiles : 0, cand ? bidir_groups(nblk) : 0);
     if ((rc = c->bppart.ensure((size_t)prows * 4 * np * sizeof(double)))) return rc;
-    const int nsp = std::max(nsplit, cand ? nsplit_g : 1);
+    const int nsp = std::max(generic ? nsplit : 1, cand ? nsplit_g : 1);
     if (nsp > 1 && (rc = c->part.ensure((size_t)nsp * 4 * nc * sizeof(double)))) return rc;
     tg::Out CG = CO, PG = PO, CX = CO, PX = PO;   // column pipeline (G), generic pipeline (X)
-    const bool both = cand && known_cols < 0, generic = !cand || both;
     if (both) {
       if ((rc = c->colflag.ensure(sizeof(int)))) return rc;
       int* fl = c->colflag.as<int>();
@@ -1894,7 +1913,7 @@ int tgrav_bidirectional(tgrav_ctx* c, int64_t nc, const double* cx, const double
     if (rc) return rc;
     if (cand) {
       if (nsplit_g > 1 && (rc = reduce_chunks(c, c->part.as<double>(), nc, nsplit_g, nc, CG))) return rc;
-      if ((rc = reduce_particle_partials(c, (nblk + TG_BIGRID_BLOCKS - 1) / TG_BIGRID_BLOCKS, np, PG))) return rc;
+      if ((rc = reduce_particle_partials(c, bidir_groups(nblk), np, PG))) return rc;
     }
     if (generic) {
       if (nsplit > 1 && (rc = reduce_chunks(c, c->part.as<double>(), nc, nsplit, nc, CX))) return rc;
