@@ -397,3 +397,52 @@ def test_pair_keys_of_near_and_far_sets(quirks, far):
     # sum of the terms' sizes: images of density 1 / (Lx Ly Lz) out to R = nrep min(L) add 4 pi R / V per mass
     sa = W.G_PC_MSUN_KMS * m.sum() * 4 * np.pi * 6 * L.min() / L.prod()
     check(outs["known"], outs["walk"], sa, np.abs(outs["walk"][3]).max())
+
+
+@pytest.mark.parametrize("quirks", [False, True])
+@pytest.mark.parametrize("span", [0.5, 1.0 - 1e-12, 1.0, 1.5, 3.0])     # in units of 2 boxes
+def test_pair_keys_on_the_device(quirks, span):
+    """Sets on the device, whose checks tell the sort how far apart they are: just below two boxes, at two
+    boxes (pairs of that very separation among them) and beyond, the bits of unchecked calls (which always
+    take the long key) and the sums of the per-target walk."""
+    import torch
+    rng = W.rng_for(101)
+    L = np.array([2.0, 2.5, 3.0])
+    reach = span * L.min()                            # largest |coordinate| of each set
+    S = [np.concatenate([[reach, -reach, 0.3], rng.uniform(-1, 1, 67) * min(reach, 0.5 * L[q])]) for q in range(3)]
+    T = [np.concatenate([[-reach, reach, -0.2], rng.uniform(-1, 1, 62) * reach]) for q in range(3)]
+    m = rng.uniform(0.5, 2.0, 70)
+    d = lambda a: torch.as_tensor(np.ascontiguousarray(a), device="cuda")  # noqa: E731
+    outs = {}
+    for name, validate, walk in (("known", True, False), ("unknown", False, False), ("walk", True, True)):
+        with GasGravityField("fp64", validate=validate) as f:
+            f.set_sources(*[d(a) for a in S], d(m), d(np.zeros(70)))
+            f.set_softening("spline", 0.05, quirks=quirks)
+            f.set_periodic(tuple(L), nrep=6, per_target=walk)
+            outs[name] = [a.cpu().numpy() for a in f.evaluate(None, *[d(a) for a in T])]
+    for a, b in zip(outs["known"], outs["unknown"]):
+        np.testing.assert_array_equal(a, b)
+    sa = W.G_PC_MSUN_KMS * m.sum() * 4 * np.pi * 6 * L.min() / L.prod()
+    check(outs["known"], outs["walk"], sa, np.abs(outs["walk"][3]).max())
+
+
+@pytest.mark.parametrize("nb", [8, 16])
+def test_pair_keys_of_block_targets(nb):
+    """Target blocks of 8 and of 16 cells an edge, the larger ones reaching past two boxes: the bits of
+    unchecked calls."""
+    import torch
+    rng = W.rng_for(nb)
+    L = np.array([2.0, 2.5, 3.0])
+    S = [rng.uniform(-0.5, 0.5, 70) * L[q] for q in range(3)]
+    m = rng.uniform(0.5, 2.0, 70)
+    d = lambda a: torch.as_tensor(np.ascontiguousarray(a), device="cuda")  # noqa: E731
+    o, dx = np.array([[0.0, -0.4, 0.1], [-1.0, -1.0, -1.0]]), np.array([0.3, 0.2])
+    outs = []
+    for validate in (True, False):
+        with GasGravityField("fp64", validate=validate) as f:
+            f.set_sources(*[d(a) for a in S], d(m), d(np.zeros(70)))
+            f.set_softening("spline", 0.05, quirks=True)
+            f.set_periodic(tuple(L), nrep=6)
+            outs.append(f.evaluate_blocks(d(o), d(dx), nb=nb))
+    for a, b in zip(*outs):
+        assert torch.equal(a, b)

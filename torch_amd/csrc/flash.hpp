@@ -350,7 +350,7 @@ __global__ __launch_bounds__(NT) void k_eval_flash(Tgt T, const double4* __restr
 #ifndef TG_PAIR_BITS
 #define TG_PAIR_BITS 10      // separation key: bits per axis (bins of L / 64, 8 boxes either way)
 #endif
-// Bits per axis where no separation exceeds 2 boxes (the same bins, and the same order of the pairs): the
+// Bits per axis where every separation is below 2 boxes (the same bins, and the same order of the pairs): the
 // radix sort takes 3 passes over 24 bits instead of 4 over 30.
 #define TG_PAIR_BITS_NEAR 8
 #define TG_PAIR_SLACK 1e-4   // image spacings; the square roots (v_rsq_f64, ~2^-24) are off by < 1e-5

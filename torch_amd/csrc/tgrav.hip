@@ -515,7 +515,8 @@ static int mixed_range_ok(const double* S, const double* T, const char* what) {
 // waited for), the kernels are then gated on the device.
 struct Known {
   bool valid = false, cols = false, srcb = false;
-  double span = 0.0;    // largest |coordinate| of the sources plus that of the targets
+  double span = INFINITY;   // bound on a separation along an axis: largest |coordinate| of the sources plus
+                            //   that of the targets
 };
 
 // One pass over the (device) targets of an evaluation and one wait: NaN/Inf, column structure and, mixed,
@@ -538,7 +539,8 @@ static int check_targets(tgrav_ctx* c, const tg::Tgt& T, int64_t nin, int mode, 
   k->valid = true;
   k->cols = !T.blocks && c->host_flag[HW_EVAL + tg::ST_WORDS] == 0ULL;
   k->srcb = c->ns > 0 && c->host_flag[HW_EVAL + 8 + tg::ST_WORDS] == 1ULL;
-  k->span = host_stats(c, HW_EVAL)[tg::ST_RMAX] + (c->ns > 0 ? host_stats(c, HW_EVAL + 8)[tg::ST_RMAX] : 0.0);
+  if (!(T.blocks && T.nb > 8))   // the check takes blocks to end 8 cells from their corners
+    k->span = host_stats(c, HW_EVAL)[tg::ST_RMAX] + (c->ns > 0 ? host_stats(c, HW_EVAL + 8)[tg::ST_RMAX] : 0.0);
   return 0;
 }
 
@@ -826,8 +828,9 @@ static int flash_gridsrc_kernel(tgrav_ctx* c, const tg::Tgt& T, const tg::Out& o
 static const int64_t kMaxPairs = 1LL << 25;
 static int launch_flash_pairs(tgrav_ctx* c, const tg::Tgt& T, const tg::Out& O, const tg::Flash& P,
                               const Known& known) {
-  const int bits = known.valid && known.span <= 2.0 * std::min(P.lx, std::min(P.ly, P.lz)) ? TG_PAIR_BITS_NEAR
-                                                                                          : TG_PAIR_BITS;
+  // the short key's 256 bins of L / 64 hold separations below 2 L on every axis (1e-9: roundings on the way)
+  const bool near = known.valid && known.span <= 2.0 * (1.0 - 1e-9) * std::min(P.lx, std::min(P.ly, P.lz));
+  const int bits = near ? TG_PAIR_BITS_NEAR : TG_PAIR_BITS;
   const int64_t nt = T.n, ns = c->ns;
   const int64_t tb = std::max<int64_t>(1, std::min<int64_t>(nt, kMaxPairs / ns)), nmax = tb * ns;
   size_t tmp = 0;
