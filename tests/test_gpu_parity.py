@@ -706,3 +706,32 @@ def test_fp64_slices_and_zero_pairs(ns, variant):
                 err = np.abs(got[q] - ref[q])
                 scale = np.abs(ref[q]) if q == 3 else np.sqrt(ref[0] ** 2 + ref[1] ** 2 + ref[2] ** 2)
                 assert np.all(err <= 1e-12 * (scale + np.abs(size))), (q, nsplit, err.max())
+
+
+@pytest.mark.parametrize("mode", ["fp64", "mixed"])
+@pytest.mark.parametrize("nsplit", [2, 5, 15, 16, 17, 100])
+def test_chunk_sums_of_what_is_asked_for(mode, nsplit):
+    """All four components, the acceleration alone and the potential alone from 2 to 100 source chunks, few
+    and many targets, as a call and as a plan: the same bits."""
+    import torch
+    from torch_amd.batch import BatchPlan
+    rng = W.rng_for(nsplit)
+    ns = 256 * 100 + 3
+    d = lambda a: torch.as_tensor(np.ascontiguousarray(a), device="cuda")  # noqa: E731
+    S = [d(a) for a in rng.normal(size=(3, ns))] + [d(rng.uniform(0.5, 2.0, ns)), d(np.full(ns, 0.01))]
+    for nt in (3, 700):
+        T = [d(a) for a in rng.normal(size=(3, nt))]
+        with StellarGravityField(mode) as f:
+            f.set_config(nsplit=nsplit)
+            f.set_stars(*S)
+            both = f.evaluate(None, *T)
+            acc = f.get_gravity_at_point(None, *T)
+            pot = f.get_potential_at_point(None, *T)
+            for q in range(4):
+                assert torch.equal(both[q], pot if q == 3 else acc[q]), (nt, q)
+            prob = [dict(sources=dict(zip(("x", "y", "z", "m", "eps"), S)), targets=dict(zip("xyz", T)))]
+            res = [[a.clone() if a is not None else None for a in BatchPlan(f, prob, potential=p).run()[0]]
+                   for p in (True, False)]
+            for q in range(3):
+                assert torch.equal(res[0][q], res[1][q])
+            assert res[1][3] is None and torch.isfinite(res[0][3]).all()

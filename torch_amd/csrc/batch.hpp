@@ -329,17 +329,11 @@ __global__ void k_batch_reduce(int nred, const int* __restrict__ ids,
   const int64_t t = i - prefix[q];
   const int64_t n = P.T.n;
   const double* base = part + P.part_off;
-  double s0 = 0, s1 = 0, s2 = 0, s3 = 0;
-  for (int c = 0; c < P.nchunk; ++c) {
-    const double* pc = base + (int64_t)c * 4 * n;
-    s0 += pc[t];
-    s1 += pc[n + t];
-    s2 += pc[2 * n + t];
-    if (!P.O.nopot) s3 += pc[3 * n + t];
-  }
+  double s[4] = {0.0, 0.0, 0.0, 0.0};
+  sum_chunks(base, n, t, 0, P.nchunk, false, P.O.nopot, s);
   Out o = P.O;
   o.part = nullptr;
-  store_result(o, t, s0, s1, s2, s3);
+  store_result(o, t, s[0], s[1], s[2], s[3]);
 }
 
 }  // namespace tg

@@ -594,6 +594,27 @@ __global__ __launch_bounds__(NT) void k_eval_mixed(Tgt T, const double4* __restr
   process_mixed<K, NT>(L, T, tile0, src4, srce2, sb, se, sst, o);
 }
 
+// s += the partials of target t from chunks [c0, c1), in chunk order: the components that somebody wants
+// (the others are not written).  The choice is made once, around the loop: tests inside it kept the loads of
+// successive chunks from being in flight together (10 targets, 1,000,001 sources in FP64, 485 us per call
+// against 398; 512 cells, 300,000 sources 201 against 156).
+template <int Q0, int Q1>
+__device__ __forceinline__ void sum_chunks_of(const double* __restrict__ part, int64_t pstride, int64_t t, int c0,
+                                              int c1, double (&s)[4]) {
+#pragma unroll 4
+  for (int c = c0; c < c1; ++c) {
+    const double* p = part + (int64_t)c * 4 * pstride + t;
+#pragma unroll
+    for (int q = Q0; q < Q1; ++q) s[q] += p[q * pstride];
+  }
+}
+__device__ __forceinline__ void sum_chunks(const double* __restrict__ part, int64_t pstride, int64_t t, int c0,
+                                           int c1, bool noacc, bool nopot, double (&s)[4]) {
+  if (noacc) sum_chunks_of<3, 4>(part, pstride, t, c0, c1, s);
+  else if (nopot) sum_chunks_of<0, 3>(part, pstride, t, c0, c1, s);
+  else sum_chunks_of<0, 4>(part, pstride, t, c0, c1, s);
+}
+
 // Sum of the nsplit chunk partials of each target in chunk order, then the G scaling,
 // the stores and the fused kick.
 __global__ void k_reduce_chunks(const double* __restrict__ part, int64_t pstride, int nsplit,
@@ -601,19 +622,11 @@ __global__ void k_reduce_chunks(const double* __restrict__ part, int64_t pstride
   if (gated_off(O)) return;
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= n) return;
-  double s0 = 0, s1 = 0, s2 = 0, s3 = 0;
-  for (int c = 0; c < nsplit; ++c) {
-    const double* p = part + (int64_t)c * 4 * pstride;
-    if (!O.noacc) {
-      s0 += p[t];
-      s1 += p[pstride + t];
-      s2 += p[2 * pstride + t];
-    }
-    if (!O.nopot) s3 += p[3 * pstride + t];
-  }
+  double s[4] = {0.0, 0.0, 0.0, 0.0};
+  sum_chunks(part, pstride, t, 0, nsplit, O.noacc, O.nopot, s);
   Out o = O;
   o.part = nullptr;
-  store_result(o, t, s0, s1, s2, s3);
+  store_result(o, t, s[0], s[1], s[2], s[3]);
 }
 
 // The same reduction for few targets and many chunks (k_reduce_chunks would run a handful of
@@ -629,22 +642,10 @@ __global__ __launch_bounds__(1024) void k_reduce_chunks_wide(const double* __res
   const int64_t t = (int64_t)blockIdx.x * 64 + lane;
   const int per = (nsplit + 15) / 16;
   const int c0 = w * per, c1 = min(nsplit, c0 + per);
-  double s0 = 0, s1 = 0, s2 = 0, s3 = 0;
-  if (t < n) {
-    for (int c = c0; c < c1; ++c) {
-      const double* p = part + (int64_t)c * 4 * pstride;
-      if (!O.noacc) {
-        s0 += p[t];
-        s1 += p[pstride + t];
-        s2 += p[2 * pstride + t];
-      }
-      if (!O.nopot) s3 += p[3 * pstride + t];
-    }
-  }
-  red[w][0][lane] = s0;
-  red[w][1][lane] = s1;
-  red[w][2][lane] = s2;
-  red[w][3][lane] = s3;
+  double s[4] = {0.0, 0.0, 0.0, 0.0};
+  if (t < n) sum_chunks(part, pstride, t, c0, c1, O.noacc, O.nopot, s);
+#pragma unroll
+  for (int q = 0; q < 4; ++q) red[w][q][lane] = s[q];
   __syncthreads();
   if (w == 0 && t < n) {
     double a0 = red[0][0][lane], a1 = red[0][1][lane], a2 = red[0][2][lane], a3 = red[0][3][lane];
