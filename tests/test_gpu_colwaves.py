@@ -269,3 +269,30 @@ def test_block_source_chunks_match_oracle(mode, nblk, nt):
                 s = _util.summary(f.evaluate(None, *T), ref)
                 print(mode, nblk, nt, waves, nsplit, s, flush=True)
                 check_bar(mode, s)
+
+
+@pytest.mark.parametrize("mode", ["fp64", "mixed"])
+@pytest.mark.parametrize("nblk", [59, 60, 61, 64, 65, 95, 96, 97])
+def test_line_between_thin_and_column_launches(mode, nblk):
+    """4 chunks of 4 waves per block, on either side of 3.75, 4 and 6 column waves per CU: blocks, explicit
+    centres and a plan (which keeps the column code) give the same bits."""
+    import torch
+    from torch_amd.blocks import block_centres
+    d = lambda a: torch.as_tensor(np.ascontiguousarray(a), device="cuda")  # noqa: E731
+    rng = W.rng_for(nblk)
+    o, w = rng.uniform(-1, 1, (nblk, 3)), rng.uniform(0.01, 0.1, nblk)
+    cx, cy, cz, _ = block_centres(o, w)
+    s = [d(a) for a in rng.uniform(-1, 1, (3, 1100))] + [d(rng.uniform(0.1, 1, 1100)), d(np.full(1100, 0.01))]
+    with StellarGravityField(mode) as f:
+        f.set_config(nsplit=4)
+        f.set_stars(*s)
+        a = f.evaluate_blocks(d(o), d(w))
+        b = f.evaluate(None, d(cx), d(cy), d(cz))
+        f.set_config(nsplit=1)
+        one = f.evaluate_blocks(d(o), d(w))
+        src = dict(x=s[0], y=s[1], z=s[2], m=s[3], eps=s[4])
+        c = BatchPlan(f, [dict(sources=src, targets=dict(block_origin=d(o), block_dx=d(w)))]).run()[0]
+        for q in range(4):
+            assert torch.equal(a[q], b[q])
+            assert torch.allclose(one[q], c[q], rtol=1e-5 if mode == "mixed" else 1e-12, atol=1e-12 * float(c[q].abs().max()))
+            assert torch.allclose(one[q], a[q], rtol=1e-5 if mode == "mixed" else 1e-12, atol=(1e-6 if mode == "mixed" else 1e-12) * float(c[q].abs().max()))

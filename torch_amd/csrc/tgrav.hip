@@ -619,18 +619,27 @@ static void grid_shape(const tgrav_ctx* c, int mode, int64_t ns, int64_t nblk, i
   *nsplit = (int)((ns + ch - 1) / ch);
 }
 
-// Launches of at most this many column waves per CU (2 per SIMD) take k_eval_thin, whose waves are 8
-// times as many and an eighth as long: a column wave's pass over 64 sources alone takes 15 us in FP64.
-// Per call, thin / column: 1 block x 1,024 stars 66 / 81 us (FP64), 66 / 73 (mixed); 7 x 4,000 75 / 106;
-// 28 x 3,000 94 / 107, mixed 82 / 89; 56 x 4,000 146 / 187, mixed 104 / 128; 200 x 1,000 156 / 167.  Past
-// the line the column's shared dx, dy, dz win: 700 x 300 with the line at 16 or 32 163 against 161.
-#define TG_THIN_WAVES 8
+// Launches too small for the column kernels take k_eval_thin, whose waves are 8 times as many and an eighth
+// as long.  A column wave's pass takes the same time for up to one wave per SIMD (4 per CU) and 1.7 times that
+// for two; the thin kernel's time grows with the waves, and past 6 column waves per CU (in FP64 also just
+// below 4) the column's shared dx, dy, dz win.  Thin against column at w column waves per CU, per call: FP64
+// w = 1.6 (100 blocks x 1,024 sources) 51 / 89 us, 3.1 (200 x 1,024) 84 / 90, 4.0 (64 x 4,096) 100 / 94,
+// 4.7 (300 x 1,024) 117 / 149, 6.0 (32 x 100,000) 1,107 / 1,186, 6.3 (100 x 4,096) 154 / 154, 7.8 (500 x
+// 1,024) 184 / 151; mixed 29 / 56, 42 / 57, 52 / 62, 57 / 68, 494 / 512, 75 / 74, 86 / 70.
+// Waves that their chunk leaves without sources do not count (500 blocks x 100 sources, 2 of 4 waves: 56 / 64).
+static bool thin_columns(const tgrav_ctx* c, bool mixed, int64_t wgs, int W, int64_t chunk) {
+  const int busy = (int)std::min<int64_t>(W, (chunk + 63) / 64);
+  const double w = (double)(wgs * busy) / c->num_cu;
+  if (w > 6.0 || (double)(wgs * W) / c->num_cu > 8.0) return false;
+  return mixed || busy < W || w <= 3.7 || w > 4.0;
+}
+
 // The column kernels for the context's waves per workgroup: k_eval_grid (block targets) or
 // k_eval_cols (explicit targets in the blocks' C order), grid (groups, source chunks).
 template <bool MIXED, int W>
 static void column_kernel_w(tgrav_ctx* c, bool blocks, dim3 g, const tg::Tgt& T, int64_t ns,
                             int64_t chunk, const tg::Out& o) {
-  if ((int64_t)g.x * g.y * W <= TG_THIN_WAVES * (int64_t)c->num_cu)
+  if (thin_columns(c, MIXED, (int64_t)g.x * g.y, W, chunk))
     tg::k_eval_thin<MIXED, W><<<dim3(8 * g.x, g.y), 64 * W, 0, c->stream>>>(
         T, c->s4.as<double4>(), c->se2.as<double>(), ns, chunk, c->stat.as<const double>(), o);
   else if (blocks)
