@@ -162,6 +162,32 @@ __device__ __forceinline__ void fp64_tile(const double4* __restrict__ s4,
                                           const double (&tz)[K], const double (&te2)[K],
                                           double (&ax)[K], double (&ay)[K], double (&az)[K],
                                           double (&ap)[K]) {
+  // K = 8 fills a group by itself and has no registers left for one: pair by pair (10^6 points x 8,193
+  // unsoftened sources 6,040 us per call against 6,360, 8,193 x 10^6 softened 5,795 against 6,305).
+  if constexpr (K >= 8) {
+#pragma unroll 2
+    for (int j = 0; j < cnt; ++j) {
+      const double4 s = s4[j];
+      const double e2 = se2[j];
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+        const double dx = s.x - tx[k], dy = s.y - ty[k], dz = s.z - tz[k];
+        const double r2 = fma(dx, dx, fma(dy, dy, fma(dz, dz, (FL & F_UNIF) ? e2 : e2 + te2[k])));
+        const double y = rsqrt_f64<FL>(r2);
+        if constexpr (FL & F_NOACC) {
+          ap[k] = fma(s.w, y, ap[k]);
+          continue;
+        }
+        const double mr = s.w * y;
+        if (!(FL & F_NOPOT)) ap[k] += mr;
+        const double w = mr * (y * y);
+        ax[k] = fma(w, dx, ax[k]);
+        ay[k] = fma(w, dy, ay[k]);
+        az[k] = fma(w, dz, az[k]);
+      }
+    }
+    return;
+  }
   constexpr int J = K >= TG_FP64_GROUP ? 1 : TG_FP64_GROUP / K;   // sources per group
 #pragma unroll 1
   for (int j = 0; j < cnt; j += J) {
