@@ -735,3 +735,27 @@ def test_chunk_sums_of_what_is_asked_for(mode, nsplit):
             for q in range(3):
                 assert torch.equal(res[0][q], res[1][q])
             assert res[1][3] is None and torch.isfinite(res[0][3]).all()
+
+
+@pytest.mark.parametrize("mode", ["fp64", "mixed"])
+@pytest.mark.parametrize("ns,nt", [(262143, 3), (300001, 64), (300001, 65), (40000, 16384), (40000, 16385)])
+def test_many_sources_for_few_targets(mode, ns, nt):
+    """The automatic split where the number of chunks is limited for the reduction, and on either side of it,
+    against sums in 64 bits."""
+    import torch
+    gen = torch.Generator(device="cuda").manual_seed(ns + nt)
+    r = lambda *s: torch.rand(*s, dtype=torch.float64, device="cuda", generator=gen)  # noqa: E731
+    S = [2 * r(ns) - 1 for _ in range(3)] + [0.5 + r(ns), 0.02 + 0.01 * r(ns)]
+    T = [2 * r(nt) - 1 for _ in range(3)]
+    with StellarGravityField(mode, G=1.0) as f:
+        f.set_stars(*S)
+        got = f.evaluate(None, *T)
+    at = torch.arange(0, nt, max(1, nt // 60), device="cuda")
+    d = [S[q][None, :] - T[q][at, None] for q in range(3)]
+    y = 1.0 / torch.sqrt(d[0] ** 2 + d[1] ** 2 + d[2] ** 2 + S[4][None, :] ** 2)
+    mr = S[3][None, :] * y
+    ref = [(mr * y * y * d[q]).sum(1) for q in range(3)] + [-mr.sum(1)]
+    tol = 1e-12 if mode == "fp64" else 1e-4
+    size = (mr * y).sum(1)                              # sum of the acceleration terms' sizes
+    for q in range(4):
+        assert bool(((got[q][at] - ref[q]).abs() <= tol * (size if q < 3 else ref[3].abs())).all())
