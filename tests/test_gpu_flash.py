@@ -446,3 +446,24 @@ def test_pair_keys_of_block_targets(nb):
             outs.append(f.evaluate_blocks(d(o), d(dx), nb=nb))
     for a, b in zip(*outs):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("nt,nblk", [(70000, 4), (130816, 4), (131073, 4), (10000, 30), (1000, 128)])
+def test_block_sources_of_many_points(nt, nblk):
+    """Many points on few blocks, on either side of the line to one block per chunk: a sample of the points
+    has the sums of the same cells given one by one (block kernel off)."""
+    import torch
+    rng = W.rng_for(nt + nblk)
+    o, size = rng.uniform(-1.0, 0.5, (nblk, 3)), rng.choice([0.125, 0.25, 0.5], nblk)
+    m = rng.uniform(0.5, 2.0, nblk * 512)
+    d = lambda a: torch.as_tensor(np.ascontiguousarray(a), device="cuda")  # noqa: E731
+    T = [d(a) for a in rng.uniform(-1, 1, (3, nt))]
+    at = torch.arange(0, nt, nt // 200, device="cuda")
+    with GasGravityField("fp64") as f:
+        f.set_softening("spline", 0.3)
+        f.set_blocks(d(o), d(size / 8), d(m))
+        got = f.evaluate(None, *T)
+        f.set_block_kernel(False)
+        ref = f.evaluate(None, *[t[at].contiguous() for t in T])
+    scale = W.G_PC_MSUN_KMS * m.sum()
+    check([g[at].cpu().numpy() for g in got], [r.cpu().numpy() for r in ref], scale / 0.3 ** 2, scale / 0.3)
