@@ -296,3 +296,27 @@ def test_line_between_thin_and_column_launches(mode, nblk):
             assert torch.equal(a[q], b[q])
             assert torch.allclose(one[q], c[q], rtol=1e-5 if mode == "mixed" else 1e-12, atol=1e-12 * float(c[q].abs().max()))
             assert torch.allclose(one[q], a[q], rtol=1e-5 if mode == "mixed" else 1e-12, atol=(1e-6 if mode == "mixed" else 1e-12) * float(c[q].abs().max()))
+
+
+@pytest.mark.parametrize("mode", ["fp64", "mixed"])
+@pytest.mark.parametrize("nblk,nt", [(7, 33000), (31, 5000), (32, 5000), (33, 5000), (61, 1500), (300, 3000), (29, 129)])
+@pytest.mark.parametrize("waves", [1, 2, 4])
+def test_block_source_chunks_by_xcd(mode, nblk, nt, waves):
+    """The automatic source split at few chunks (shared by all places), at 8 and more (a chunk's tiles on one
+    XCD) and with a part chunk at the end: the unsplit sums, to rounding."""
+    import torch
+    rng = W.rng_for(nblk * 7 + nt)
+    d = lambda a: torch.as_tensor(np.ascontiguousarray(a), device="cuda")  # noqa: E731
+    o, w = d(rng.uniform(-2.0, 1.5, (nblk, 3))), d(rng.choice([0.125, 0.25, 0.5], nblk) / 8)
+    m = d(rng.uniform(0.5, 1.0, nblk * 512))
+    T = [d(a) for a in rng.uniform(-2, 2, (3, nt))]
+    with GravityField(mode, tune_cache=None) as f:
+        f.set_column_waves(waves)
+        f.set_source_blocks(o, w, m)
+        got = f.evaluate(None, *T)
+        f.set_config(nsplit=1)
+        one = f.evaluate(None, *T)
+    size = m.sum() * W.G_PC_MSUN_KMS
+    for q in range(4):
+        tol = (1e-12 if mode == "fp64" else 1e-5) * (one[3].abs().max() if q == 3 else size / 0.01)
+        assert bool(((got[q] - one[q]).abs() <= tol).all())

@@ -717,6 +717,43 @@ static int launch_grid(tgrav_ctx* c, int mode, const tg::Tgt& T, const tg::Out& 
 template <bool MIXED>
 static constexpr int gs_plan_k() { return MIXED ? TG_GS_K : 4; }
 
+// Rounds (a block per wave) of a chunk, of `rounds` in all, for ntiles tiles on workgroups of W waves.  A CU has
+// 4 / W workgroup places (one wave per SIMD), and with 8 or more chunks a chunk's tiles are on one XCD
+// (k_eval_gridsrc), so the XCD with one chunk more than others sets the time: its turns of a chunk's rounds.
+// With fewer, places share all the work evenly up to about half a chunk at the end.  One turn alone is a tenth
+// slower (one wave per SIMD), two a fortieth.  Partial sums are written and read at 5 TB/s, and a chunk costs
+// the reduction 0.02 us; a round takes 32 us in FP64 and 12.7 mixed.  Fitted to 19 sizes of 30 to 100,000
+// points and 50 to 20,000 blocks in each mode, with every chunk length: the choice is within 3% of the fastest
+// (chunks of turns_split's, which knows no XCDs: up to 35% above it).
+static int64_t gridsrc_rounds(const tgrav_ctx* c, int mode, int64_t nt, int64_t ntiles, int64_t rounds, int W,
+                              int64_t most) {
+  const double places = c->num_cu * 4.0 / W, unit = mode == TGRAV_MIXED ? 12.7 : 32.0;
+  int64_t best_t = rounds;
+  double best = INFINITY;
+  auto look = [&](int64_t t) {
+    const int64_t n = (rounds + t - 1) / t;
+    if (n > most) return;
+    double turns, cost;
+    if (n >= 8) {
+      turns = ceil((double)(ntiles * ((n + 7) / 8)) / (places / 8));
+      cost = (turns + 0.3) * (double)t;
+    } else {
+      turns = std::max(1.0, ceil((double)(ntiles * n) / places));
+      cost = turns == 1.0 ? (double)t : (double)ntiles * (double)rounds / places + 0.6 * (double)t;
+    }
+    cost = cost * (1.0 + 0.1 / (turns * turns)) + ((double)n * (double)nt * 64.0 / 5e6 + 0.02 * (double)n) / unit;
+    if (cost < best) {
+      best = cost;
+      best_t = t;
+    }
+  };
+  look(rounds);
+  for (int64_t t = 1; t <= 16 && t < rounds; ++t) look(t);
+  for (int64_t i = 2; i < 8; ++i) look((rounds + i - 1) / i);
+  for (int64_t i = 8; i <= 128; i += 8) look((rounds + i - 1) / i);
+  return best_t;
+}
+
 static void gridsrc_shape(const tgrav_ctx* c, int mode, int64_t nt, int64_t nblk, int64_t* ntiles,
                           int* nsplit, int64_t* chunk) {
   const int K = TG_GS_K, W = c->col_waves;
@@ -725,12 +762,9 @@ static void gridsrc_shape(const tgrav_ctx* c, int mode, int64_t nt, int64_t nblk
   const int tuned = tuned_block_split(c, mode, "blocksrc", nt, nblk, W);
   if (tuned > 0) want = tuned;
   if (want <= 0) {
-    // Whole rounds of a block per wave, by turns.  Per call at the chunks this picks, against ~16 rounds of
-    // waves of at least 4 blocks each: 5,000 stars x 500 blocks 714 / 802 us, x 1,000 1,309 / 1,434 (FP64),
-    // 3,000 x 300 212 / 288 (mixed), 10,000 x 2,000 1,954 / 1,956 (mixed).
-    const int64_t rounds = (nblk + W - 1) / W;
-    const int n = turns_split(*ntiles, rounds, c->num_cu * 4.0 / W, 0.1, 0.8, 65535);
-    *chunk = (rounds + n - 1) / n * W;
+    // at most 12 x 2^20 target-chunks of partial sums (32 B each)
+    const int64_t most = std::max<int64_t>(1, std::min<int64_t>(65528, (12LL << 20) / std::max<int64_t>(nt, 1)));
+    *chunk = gridsrc_rounds(c, mode, nt, *ntiles, (nblk + W - 1) / W, W, most) * W;
     *nsplit = (int)((nblk + *chunk - 1) / *chunk);
     return;
   }
