@@ -717,31 +717,48 @@ static int launch_grid(tgrav_ctx* c, int mode, const tg::Tgt& T, const tg::Out& 
 template <bool MIXED>
 static constexpr int gs_plan_k() { return MIXED ? TG_GS_K : 4; }
 
+// Time until `full` jobs of length t and, after them, `part` jobs of length `last` <= t are done on `places`
+// places that each take the next job when free.
+static double list_time(int64_t full, int64_t t, int64_t part, int64_t last, int64_t places) {
+  const int64_t q = full / places, rem = full % places;
+  double time = (double)q * (double)t;
+  if (rem) {                     // places without a job in the last turn take short ones meanwhile
+    time += (double)t;
+    part = std::max<int64_t>(0, part - (places - rem) * (t / last));
+  }
+  return time + (double)((part + places - 1) / places) * (double)last;
+}
+
 // Rounds (a block per wave) of a chunk, of `rounds` in all, for ntiles tiles on workgroups of W waves.  A CU has
 // 4 / W workgroup places (one wave per SIMD), and with 8 or more chunks a chunk's tiles are on one XCD
-// (k_eval_gridsrc), so the XCD with one chunk more than others sets the time: its turns of a chunk's rounds.
-// With fewer, places share all the work evenly up to about half a chunk at the end.  One turn alone is a tenth
-// slower (one wave per SIMD), two a fortieth.  Partial sums are written and read at 5 TB/s, and a chunk costs
-// the reduction 0.02 us; a round takes 32 us in FP64 and 12.7 mixed.  Fitted to 19 sizes of 30 to 100,000
-// points and 50 to 20,000 blocks in each mode, with every chunk length: the choice is within 3% of the fastest
-// (chunks of turns_split's, which knows no XCDs: up to 35% above it).
+// (k_eval_gridsrc), so the XCD with one chunk more than others sets the time; the last chunk may be shorter.
+// 0.4 chunks are added for the end, where places are idle; a single turn is 15% slower in FP64 and half as
+// slow again in mixed mode (one wave per SIMD: no FP32 pairs).  Partial sums are written and read at 2 TB/s,
+// and a chunk costs the reduction 0.02 us; a round takes 32 us in FP64 and 12.7 mixed.  Fitted to 19 sizes of
+// 30 to 100,000 points and 50 to 20,000 blocks in each mode, with every chunk length: the choice is within
+// 3.5% of the fastest (chunks of turns_split, which knows no XCDs: up to 35% above it).
 static int64_t gridsrc_rounds(const tgrav_ctx* c, int mode, int64_t nt, int64_t ntiles, int64_t rounds, int W,
                               int64_t most) {
-  const double places = c->num_cu * 4.0 / W, unit = mode == TGRAV_MIXED ? 12.7 : 32.0;
+  const int64_t places = std::max<int64_t>(8, c->num_cu * 4 / W);
+  const bool mixed = mode == TGRAV_MIXED;
   int64_t best_t = rounds;
   double best = INFINITY;
   auto look = [&](int64_t t) {
-    const int64_t n = (rounds + t - 1) / t;
+    const int64_t n = (rounds + t - 1) / t, last = rounds - (n - 1) * t;
     if (n > most) return;
-    double turns, cost;
+    double cost;
+    bool single;
     if (n >= 8) {
-      turns = ceil((double)(ntiles * ((n + 7) / 8)) / (places / 8));
-      cost = (turns + 0.3) * (double)t;
+      const int64_t cx = (n + 7) / 8, part = n % 8 == 1 ? 1 : 0;   // XCD 0's chunks
+      cost = list_time(ntiles * (cx - part), t, ntiles * part, last, places / 8);
+      single = ntiles * cx <= places / 8;
     } else {
-      turns = std::max(1.0, ceil((double)(ntiles * n) / places));
-      cost = turns == 1.0 ? (double)t : (double)ntiles * (double)rounds / places + 0.6 * (double)t;
+      cost = list_time(ntiles * (n - 1), t, ntiles, last, places);
+      single = ntiles * n <= places;
     }
-    cost = cost * (1.0 + 0.1 / (turns * turns)) + ((double)n * (double)nt * 64.0 / 5e6 + 0.02 * (double)n) / unit;
+    cost += 0.4 * (double)t;
+    if (single) cost *= mixed ? 1.5 : 1.15;
+    cost += ((double)n * (double)nt * 64.0 / 2e6 + 0.02 * (double)n) / (mixed ? 12.7 : 32.0);
     if (cost < best) {
       best = cost;
       best_t = t;
