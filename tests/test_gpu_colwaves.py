@@ -320,3 +320,27 @@ def test_block_source_chunks_by_xcd(mode, nblk, nt, waves):
     for q in range(4):
         tol = (1e-12 if mode == "fp64" else 1e-5) * (one[3].abs().max() if q == 3 else size / 0.01)
         assert bool(((got[q] - one[q]).abs() <= tol).all())
+
+
+@pytest.mark.parametrize("mode", ["fp64", "mixed"])
+@pytest.mark.parametrize("ns", [1, 64, 65, 128, 129])
+@pytest.mark.parametrize("nblk", [200, 800, 1600])
+def test_few_sources_on_many_blocks(mode, ns, nblk):
+    """Chunks of one, two and more waves' sources, thin and column launches: blocks, explicit centres and a plan
+    (whose workgroups keep their 4 waves) give the same bits."""
+    import torch
+    from torch_amd.blocks import block_centres
+    d = lambda a: torch.as_tensor(np.ascontiguousarray(a), device="cuda")  # noqa: E731
+    rng = W.rng_for(nblk + ns)
+    o, w = rng.uniform(-1, 1, (nblk, 3)), rng.uniform(0.01, 0.1, nblk)
+    cx, cy, cz, _ = block_centres(o, w)
+    s = [d(a) for a in rng.uniform(-1, 1, (3, ns))] + [d(rng.uniform(0.1, 1, ns)), d(np.full(ns, 0.01))]
+    with StellarGravityField(mode) as f:
+        f.set_config(nsplit=1)
+        f.set_stars(*s)
+        a = f.evaluate_blocks(d(o), d(w))
+        b = f.evaluate(None, d(cx), d(cy), d(cz))
+        src = dict(x=s[0], y=s[1], z=s[2], m=s[3], eps=s[4])
+        c = BatchPlan(f, [dict(sources=src, targets=dict(block_origin=d(o), block_dx=d(w)))]).run()[0]
+        for q in range(4):
+            assert torch.equal(a[q], b[q]) and torch.equal(a[q], c[q])

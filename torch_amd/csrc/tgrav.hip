@@ -625,17 +625,17 @@ static void grid_shape(const tgrav_ctx* c, int mode, int64_t ns, int64_t nblk, i
 
 // Launches too small for the column kernels take k_eval_thin, whose waves are 8 times as many and an eighth
 // as long.  A column wave's pass takes the same time for up to one wave per SIMD (4 per CU) and 1.7 times that
-// for two; the thin kernel's time grows with the waves, and past 6 column waves per CU (in FP64 also just
+// for two; the thin kernel's time grows with the waves, and past 6.5 column waves per CU (in FP64 also just
 // below 4) the column's shared dx, dy, dz win.  Thin against column at w column waves per CU, per call: FP64
 // w = 1.6 (100 blocks x 1,024 sources) 51 / 89 us, 3.1 (200 x 1,024) 84 / 90, 4.0 (64 x 4,096) 100 / 94,
-// 4.7 (300 x 1,024) 117 / 149, 6.0 (32 x 100,000) 1,107 / 1,186, 6.3 (100 x 4,096) 154 / 154, 7.8 (500 x
-// 1,024) 184 / 151; mixed 29 / 56, 42 / 57, 52 / 62, 57 / 68, 494 / 512, 75 / 74, 86 / 70.
-// Waves that their chunk leaves without sources do not count (500 blocks x 100 sources, 2 of 4 waves: 56 / 64).
+// 4.7 (300 x 1,024) 117 / 149, 6.0 (32 x 100,000) 1,107 / 1,186, 6.3 (100 x 4,096) 154 / 154, (400 x 300)
+// 55 / 64, 7.8 (500 x 1,024) 184 / 151; mixed 29 / 56, 42 / 57, 52 / 62, 57 / 68, 494 / 512, 75 / 74, 30 / 36,
+// 86 / 70.  Waves without sources (a chunk of at most 64 W - 64) do not count: 500 blocks x 100 sources 38 / 50,
+// x 129 44 / 47.
 static bool thin_columns(const tgrav_ctx* c, bool mixed, int64_t wgs, int W, int64_t chunk) {
   const int busy = (int)std::min<int64_t>(W, (chunk + 63) / 64);
   const double w = (double)(wgs * busy) / c->num_cu;
-  if (w > 6.0 || (double)(wgs * W) / c->num_cu > 8.0) return false;
-  return mixed || busy < W || w <= 3.7 || w > 4.0;
+  return w <= 6.5 && (mixed || busy < 4 || w <= 3.7 || w > 4.0);
 }
 
 // The column kernels for the context's waves per workgroup: k_eval_grid (block targets) or
@@ -658,7 +658,10 @@ static int column_kernel(tgrav_ctx* c, int mode, bool blocks, int64_t ngrp, int 
                          const tg::Tgt& T, int64_t ns, int64_t chunk, const tg::Out& o) {
   const dim3 g((unsigned)ngrp, (unsigned)nsplit);
   const bool mixed = mode == TGRAV_MIXED;
-  switch (c->col_waves) {
+  // Waves that their chunk leaves without sources are not launched (the same sums).  12,000 blocks, per call
+  // with 1 wave / 4: 8 sources FP64 228 / 422 us, mixed 172 / 305; with
+  // 2 / 4, 100 sources: FP64 417 / 533, mixed 196 / 340.
+  switch (std::min(c->col_waves, chunk <= 64 ? 1 : chunk <= 128 ? 2 : 4)) {
     case 4:
       if (mixed) column_kernel_w<true, 4>(c, blocks, g, T, ns, chunk, o);
       else column_kernel_w<false, 4>(c, blocks, g, T, ns, chunk, o);
