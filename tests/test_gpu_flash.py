@@ -467,3 +467,30 @@ def test_block_sources_of_many_points(nt, nblk):
         ref = f.evaluate(None, *[t[at].contiguous() for t in T])
     scale = W.G_PC_MSUN_KMS * m.sum()
     check([g[at].cpu().numpy() for g in got], [r.cpu().numpy() for r in ref], scale / 0.3 ** 2, scale / 0.3)
+
+
+@pytest.mark.parametrize("quirks", [False, True])
+@pytest.mark.parametrize("where", ["target", "source", "mass"])
+def test_periodic_nan_without_validation(quirks, where):
+    """Unchecked NaN inputs: wherever a pair's NaN reaches the acceleration it reaches the potential too, with
+    and without quirks; a NaN target always has both, and the other targets neither."""
+    rng = W.rng_for(8)
+    S = [rng.uniform(-1, 1, 70) for _ in range(3)]
+    T = [rng.uniform(-1, 1, 9) for _ in range(3)]
+    m = rng.uniform(0.5, 2.0, 70)
+    if where == "target":
+        T[1][4] = np.nan
+    elif where == "source":
+        S[1][4] = np.nan
+    else:
+        m[4] = np.nan
+    with GasGravityField("fp64", validate=False) as f:
+        f.set_sources(*S, m, np.zeros(70))
+        f.set_softening("spline", 0.05, quirks=quirks)
+        f.set_periodic((2.0, 2.5, 3.0), nrep=2)
+        got = np.isnan(np.array(f.evaluate(None, *T)))
+    np.testing.assert_array_equal(got[3], got[0])
+    if where == "target":
+        np.testing.assert_array_equal(got, np.tile(np.arange(9) == 4, (4, 1)))
+    if where == "mass":
+        assert got.all()

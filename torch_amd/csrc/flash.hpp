@@ -631,7 +631,7 @@ __global__ __launch_bounds__(64) void k_eval_flash_pairs(Tgt T, int64_t t0, cons
       py = fma(skv, dy, py);
     }
   }
-  if (QUIRKS && r2l > 0.0) pp = rsqrt_f64<0>(r2l);
+  if (QUIRKS && !(r2l == 0.0)) pp = rsqrt_f64<0>(r2l);   // NaN positions of unchecked calls stay NaN
   if (valid) pairbuf[pr] = make_double4(px, py, pz, pp);
 }
 
