@@ -149,7 +149,7 @@ __global__ __launch_bounds__(256) void k_batch_pack(int nprob, const BSrc* __res
   if (p0 >= 0) {
     for (int q = p0; q <= p1; ++q) {
       const bool mine = p == q;
-      fold_source_stats(mine ? e2min : 0x7ff0000000000000ULL, 0, mine ? rmax : 0ULL, mine ? e2max : 0ULL,
+      fold_source_stats(mine ? e2min : 0x7ff0000000000000ULL, mine ? rmax : 0ULL, mine ? e2max : 0ULL,
                         mine ? mmax : 0ULL, stats + (int64_t)ST_WORDS * q);
     }
   }

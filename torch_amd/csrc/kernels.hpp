@@ -141,7 +141,7 @@ __device__ __forceinline__ double rsqrt_f64(double r2) {
 // F_GUARD for a group of pairs: y[q] = 0 where r2[q] == 0.  Zero pairs are rare (a point on an unsoftened
 // source), so the group is tested at once -- the smallest of its r2's high words, which no r2 >= 2^-1042
 // has zero -- and the selects are in a branch the wave takes only then: 5 instructions for 8 pairs instead
-// of 24.  20,011 points, 5,003 unsoftened sources: @GUARD@
+// of 24.
 template <int N>
 __device__ __forceinline__ void guard_zero(const double (&r2)[N], double (&y)[N]) {
   unsigned h = (unsigned)__double2hiint(r2[0]);
@@ -699,18 +699,16 @@ __device__ __forceinline__ unsigned long long shfl_xor_u64(unsigned long long v,
 // Folds one lane's source statistics (ST_* words) into `stat`: reduced within each wave by
 // shuffles, across the workgroup's (at most 4) waves through LDS, then at most one atomic per
 // word.  Every lane of the workgroup (<= 256 lanes) must call it.
-__device__ __forceinline__ void fold_source_stats(unsigned long long e2min, int bad, unsigned long long rmax,
+__device__ __forceinline__ void fold_source_stats(unsigned long long e2min, unsigned long long rmax,
                                                   unsigned long long e2max, unsigned long long mmax,
                                                   unsigned long long* stat) {
   __shared__ unsigned long long sm[4][4];
-  __shared__ int sbad[4];
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) {
     e2min = min(e2min, shfl_xor_u64(e2min, off));
     rmax = max(rmax, shfl_xor_u64(rmax, off));
     e2max = max(e2max, shfl_xor_u64(e2max, off));
     mmax = max(mmax, shfl_xor_u64(mmax, off));
-    bad |= __shfl_xor(bad, off);
   }
   const int t = threadIdx.x, w = t >> 6, nw = (blockDim.x + 63) >> 6;
   if ((t & 63) == 0) {
@@ -718,7 +716,6 @@ __device__ __forceinline__ void fold_source_stats(unsigned long long e2min, int 
     sm[1][w] = rmax;
     sm[2][w] = e2max;
     sm[3][w] = mmax;
-    sbad[w] = bad;
   }
   __syncthreads();
   if (t == 0) {
@@ -727,14 +724,13 @@ __device__ __forceinline__ void fold_source_stats(unsigned long long e2min, int 
       sm[1][0] = max(sm[1][0], sm[1][q]);
       sm[2][0] = max(sm[2][0], sm[2][q]);
       sm[3][0] = max(sm[3][0], sm[3][q]);
-      sbad[0] |= sbad[q];
     }
   }
   __syncthreads();
   // One lane per word; the atomic only where the workgroup's value improves on what the word
   // already holds (a plain read, possibly stale, which only costs an atomic): with thousands of
   // workgroups on the same five words, most then skip their atomics instead of queueing on them.
-  if (t < 5) {
+  if (t < ST_WORDS) {
     volatile unsigned long long* w = stat + t;
     if (t == ST_E2MIN) {
       if (sm[0][0] < *w) atomicMin(&stat[ST_E2MIN], sm[0][0]);
@@ -744,8 +740,6 @@ __device__ __forceinline__ void fold_source_stats(unsigned long long e2min, int 
       if (sm[2][0] > *w) atomicMax(&stat[ST_E2MAX], sm[2][0]);
     } else if (t == ST_MMAX) {
       if (sm[3][0] > *w) atomicMax(&stat[ST_MMAX], sm[3][0]);
-    } else if (sbad[0]) {
-      atomicOr(&stat[ST_BAD], 1ULL);
     }
   }
 }
@@ -946,11 +940,6 @@ __global__ void k_kick(int64_t n, double dt, const double* __restrict__ ax,
     vy[i] = vy[i] + dt * ay[i];
     vz[i] = vz[i] + dt * az[i];
   }
-}
-
-// flag[0] = v (one lane; a kernel rather than a memset, so a captured graph replays it).
-__global__ void k_set_flag(int* flag, int v) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) flag[0] = v;
 }
 
 // Gate value of an explicit-target evaluation whose structure the host does not know: 2 if the sources
